@@ -1,7 +1,7 @@
 // Shared pieces of the gfx950 absorbed-MLA decode kernels (mla_coop.hip: up
-// to 16 query rows per CTA; mla_decode.hip: 32; mla_wide.hip: 128): the fused
-// fp8 row format, launch parameters, exact fp8 -> bf16 widening, and the
-// device-side split plan the kernels deal their units from.
+// to 16 query rows per CTA; mla_rows64.hip: 64): the fused fp8 row format,
+// launch parameters, exact fp8 -> bf16 widening, and the device-side split
+// plans the kernels deal their units from.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -16,33 +16,17 @@ namespace mla {
 constexpr int kLat = 512;
 constexpr int kRope = 64;
 constexpr int kQK = kLat + kRope;              // 576 bytes per fp8 row
-constexpr int kTileTok = 32;                   // tokens per tile
-constexpr int kTileBytes = kTileTok * kQK;     // 18432 fp8 bytes per tile
-constexpr int kDmaPerTile = kTileBytes / 1024; // 18 wave-DMA instructions (64 x 16 B)
-constexpr int kKPairs = kQK / 32;              // 18 pairs of 16-dim k-steps (16 latent + 2 rope)
-constexpr int kDTiles = kLat / 32;             // 16 output d-tiles of 32
+constexpr int kTileTok = 32;                   // parts are whole multiples of it (equal parts)
 constexpr int kMaxQLen = 8;
 constexpr int kMaxHeads = 128;
 // A row's running max is fixed at its first non-empty tile; later tiles may
 // exceed it by up to 2^64 (p <= 2^64, no fp32 overflow of O or l). Beyond that
 // the CTA falls back to an exact-max second pass.
 constexpr float kGrowLimit = 64.f;
-// Q dims [448, 576) (the last four k-step pairs) stay in LDS, the rest in
-// VGPRs: 256 B per query row in LDS, 16-byte chunk c of row r at chunk c ^ (r & 15).
-constexpr int kQRegPairs = 14;                 // k-step pairs whose Q lives in VGPRs
-constexpr int kQLdsDim0 = kQRegPairs * 32;     // 448
-constexpr int kQLdsRowBytes = (kQK - kQLdsDim0) * 2;  // 256
-// Order of the k-step pairs in the QK loops: position s handles pair
-// qk_pair_at(s). The four LDS-resident pairs run at positions 6..9, not last,
-// so their one-step-ahead Q reads overlap the K reads already in flight (and,
-// in the 128-row kernel, steps that also carry PV MFMAs): -2% for the 32-row
-// kernel at H=128 q_len 2. The scores are fp32 sums in a different order,
-// equally close to the exact sum.
-__device__ __forceinline__ constexpr int qk_pair_at(int s) { return s < 6 ? s : (s < 10 ? s + 8 : s - 4); }
-static_assert(kQRegPairs == 14 && kKPairs == 18, "qk_pair_at permutes 18 pairs with the LDS ones at 6..9");
-
+constexpr float kGrowSum = 18446744073709551616.f;  // 2^kGrowLimit, for tests on sums of p
+constexpr int kRows64 = 64;  // query rows per CTA of the 64-row kernel
 // Split partial records. Workspace: the O records (one per (b, part): rec_rows
-// rows of 512 fp32, row-major, or in the 128-row kernel's fragment order), then
+// rows of 512 fp32, row-major), then
 // the (m, l) pair of every (b, part, query row), then an 8-byte (parts, first
 // record) entry per request. kMaxRecords caps the O rows of a workspace.
 constexpr size_t kMaxRecords = 65536;
@@ -59,9 +43,10 @@ struct Params {
   const int* kv_indptr;   // [B+1] (paged)
   int B, H, q_len, S_fixed, parts, ngroups, paged;
   int unit_cap;           // units one round of CTAs over the CUs holds
+  int workers;            // > 0: balanced split over this many units (see plan_work), 0: equal parts
   int qrows;              // H * q_len
-  int rec_rows;           // O rows per split record: qrows, or a multiple of 32 for the fragment order
-  int rec_frag;           // 1: O records in the 128-row kernel's fragment order
+  int rec_rows;           // O rows per split record (>= qrows)
+  int seg_cost;           // places one more part costs a unit (balanced split)
   float score_c;          // scale * kv_scale * log2(e), fp32
   float kv_scale;
 };
@@ -74,8 +59,6 @@ __device__ __forceinline__ int* ws_tbl(const Params& p) {
 }
 
 typedef int i32x2 __attribute__((ext_vector_type(2)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 // Two fp8 of a dword (lo or hi half) -> two bf16, exact (scale 1).
 template <bool HI>
@@ -85,15 +68,6 @@ __device__ __forceinline__ uint32_t fp8x2_bf16(uint32_t w) {
 __device__ __forceinline__ bf16x8 fp8x8_bf16(uint32_t lo, uint32_t hi) {
   u32x4 o = {fp8x2_bf16<false>(lo), fp8x2_bf16<true>(lo), fp8x2_bf16<false>(hi), fp8x2_bf16<true>(hi)};
   return __builtin_bit_cast(bf16x8, o);
-}
-
-// O^T += V^T P^T into an AGPR accumulator. The s_nop covers the VALU-write ->
-// MFMA-read distance for operands converted just before (the compiler cannot
-// see through the asm); consecutive calls always target different
-// accumulators, and every VALU read of an accumulator is preceded by
-// mfma_result_fence().
-__device__ __forceinline__ void pv_mfma(f32x16& acc, bf16x8 a, bf16x8 b) {
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
 // Field `k` (16 bits) of a packed pair, extracted where it is used (volatile:
@@ -338,6 +312,112 @@ __device__ __forceinline__ Unit plan_unit_contig(int S, int B, int P, int cap, i
   return Unit{u / np, u % np, np, (u / np) * np, part_tokens(S, np), B * np, S, 0};
 }
 
+// ---- balanced split --------------------------------------------------------------------
+// With records for it (W + B - 1 <= B * P) a round of W units shares the
+// batch's tiles evenly, whatever its lengths: the requests' 64-token tiles are
+// laid end to end, p.seg_cost places before each request standing for what
+// starting one costs a unit (4 with 64-row CTAs, 6 with 16-row ones, whose
+// tiles are shorter: 2..8 measured), and unit u walks places [u * tw, (u + 1) * tw), one
+// segment per request it meets there. Equal parts per request leave the longest
+// part 14% (256 units) to 80% (64 units) above the mean on lengths of
+// U[1024, 8192]. A request's segments are consecutive units, so its records
+// are consecutive too: segment (u, b) takes record u + b.
+constexpr int kWorkTile = 64;  // tokens per tile
+constexpr int kMinWork = 4;    // places per unit at least
+
+// A part of a request: what a CTA works on at a time.
+struct Seg {
+  int b;               // request, -1: none
+  int part, nparts;    // part within the request
+  int rec0;            // record index of the request's part 0
+  int kv_lo, kv_hi;    // tokens of the part
+  int len;             // context length of the request
+  int slot0;           // its first flat slot index (paged)
+  int pos;             // place of the request's first tile (balanced split)
+  int tw;              // places per unit (0: equal parts, one segment per unit)
+};
+__device__ __forceinline__ int work_tiles(int len) { return len > kWorkTile ? (len - 1) / kWorkTile + 1 : 1; }
+
+// Unit u's segment of a request whose first tile is at `pos`.
+__device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, int slot0) {
+  const int nt = work_tiles(len);
+  const int u0 = pos / tw;
+  const int lo = u * tw > pos ? u * tw - pos : 0;
+  const int hi = (u + 1) * tw - pos < nt ? (u + 1) * tw - pos : nt;
+  const int end = len > 0 ? len : 0;
+  Seg r{b, u - u0, (pos + nt - 1) / tw - u0 + 1, u0 + b, lo * kWorkTile, end, len, slot0, pos, tw};
+  if (hi < nt) r.kv_hi = hi * kWorkTile;
+  if (hi <= 0) r.b = -1;  // the unit's places end before the tiles begin
+  return r;
+}
+
+// The first segment of unit u, by one wave (`scratch`: as plan_unit_paged).
+template <bool PAGED>
+__device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
+  if (p.workers == 0) {
+    const Unit un = PAGED ? plan_unit_paged(p.seq_lens, p.kv_indptr, p.B, p.parts, p.unit_cap, u, lane, scratch)
+                          : plan_unit_contig(p.S_fixed, p.B, p.parts, p.unit_cap, u);
+    const long long lo = (long long)un.part * un.ptok;
+    const int kv_lo = lo < un.len ? (int)lo : un.len;
+    const int kv_hi = lo + un.ptok < un.len ? (int)(lo + un.ptok) : un.len;
+    return Seg{u < un.units ? un.b : -1, un.part, un.nparts, un.rec0, kv_lo, kv_hi, un.len, un.slot0, 0, 0};
+  }
+  const Seg none{-1, 0, 1, 0, 0, 0, 0, 0, 0, 1};
+  if (u >= p.workers) return none;
+  auto share = [&](int total) {
+    const int tw = ceil_div_u(total, p.workers);
+    return tw > kMinWork ? tw : kMinWork;
+  };
+  if constexpr (!PAGED) {
+    const int per = work_tiles(p.S_fixed) + p.seg_cost;
+    const int tw = share(p.B * per);
+    const int b = u * tw / per;
+    return b < p.B ? work_seg(u, tw, b, b * per + p.seg_cost, p.S_fixed, 0) : none;
+  }
+  const int l0 = lane < p.B ? p.seq_lens[lane] : 0;  // the first 64 requests cost one round trip
+  const int s0 = lane < p.B ? p.kv_indptr[lane] : 0;
+  auto len_at = [&](int c0) { return c0 == 0 ? l0 : (c0 + lane < p.B ? p.seq_lens[c0 + lane] : 0); };
+  auto places = [&](int c0, int l) { return c0 + lane < p.B ? work_tiles(l) + p.seg_cost : 0; };
+  int total = 0;
+  for (int c0 = 0; c0 < p.B; c0 += 64) total += wave_sum_i(places(c0, len_at(c0)));
+  const int tw = share(total);
+  int run = 0;
+  for (int c0 = 0; c0 < p.B; c0 += 64) {
+    const int l = len_at(c0);
+    const int inc = run + wave_incl_scan(places(c0, l));  // end of the request's places
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(c0 + lane < p.B && inc > u * tw);
+    if (hit) {
+      const int h = (int)__builtin_ctzll(hit);
+      const int len = __builtin_amdgcn_readlane(l, h);
+      const int pos = __builtin_amdgcn_readlane(inc, h) - work_tiles(len);
+      const int slot0 = c0 == 0 ? __builtin_amdgcn_readlane(s0, h) : p.kv_indptr[c0 + h];
+      return work_seg(u, tw, c0 + h, pos, len, slot0);
+    }
+    run = __builtin_amdgcn_readlane(inc, 63);
+  }
+  return none;
+}
+
+// Unit u's segment after `sg`, or b = -1. `len`, `slot0`: of request sg.b + 1.
+__device__ __forceinline__ Seg next_work(const Params& p, const Seg& sg, int u, int len, int slot0) {
+  Seg r = sg;
+  r.b = -1;
+  if (sg.tw == 0 || sg.b + 1 >= p.B) return r;
+  const int pos = sg.pos + work_tiles(sg.len) + p.seg_cost;
+  return pos < (u + 1) * sg.tw ? work_seg(u, sg.tw, sg.b + 1, pos, len, slot0) : r;
+}
+
+// One wave's segment to all: posted in `misc` (10 ints), read after a barrier.
+__device__ __forceinline__ void post_seg(int* misc, const Seg& s) {
+  const int v[10] = {s.b, s.part, s.nparts, s.rec0, s.kv_lo, s.kv_hi, s.len, s.slot0, s.pos, s.tw};
+#pragma unroll
+  for (int i = 0; i < 10; ++i) misc[i] = v[i];
+}
+__device__ __forceinline__ Seg read_seg(const int* misc) {
+  auto at = [&](int i) { return __builtin_amdgcn_readfirstlane(misc[i]); };
+  return Seg{at(0), at(1), at(2), at(3), at(4), at(5), at(6), at(7), at(8), at(9)};
+}
+
 // 4-byte global -> LDS DMA (lane l's dword lands at lds_dst + 4*l), counted by
 // the kernel itself like dma16_opaque.
 __device__ __forceinline__ void dma4_opaque(const void* gsrc, const char* lds_dst) {
@@ -351,10 +431,10 @@ __device__ __forceinline__ void dma4_opaque(const void* gsrc, const char* lds_ds
 // V^T transpose read hit distinct LDS banks.
 __device__ __forceinline__ int swz(int t) { return (t >> 2) & 3; }
 
-// Host launchers of the 128-row kernel (mla_wide.hip) and of the 16-row kernel
-// (mla_coop.hip); grid = CTAs.
-int launch_wide_kernel(const Params& p, long long grid, hipStream_t st);
+// Host launchers of the 16-row kernel (mla_coop.hip) and the 64-row kernel
+// (mla_rows64.hip); grid = CTAs.
 int launch_coop_kernel(const Params& p, long long grid, hipStream_t st);
+int launch_rows64_kernel(const Params& p, long long grid, hipStream_t st);
 
 }  // namespace mla
 }  // namespace mm

@@ -1,0 +1,112 @@
+"""The work split of the MLA decode: the balanced split (a full round of CTAs
+shares the batch's 64-token tiles, several requests to a CTA and several CTAs
+to a request) at its edges, against the CPU oracle, and its arithmetic on the
+CPU. Tolerance: the oracle's 1-ULP rule of test_mla_gpu."""
+import numpy as np
+import pytest
+import torch
+
+import moonmath_attention as ma
+from mla_inputs import KV_SCALE, QK, SCALE_576, fp8_bits, paged_pool, ragged_lens, rand_kv_rows, rand_q
+from test_mla_gpu import DEV, _check, _d
+
+
+def _tiles(n):
+    return max(1, -(-n // 64))
+
+
+def _segments(lens, units, cost):
+    """csrc/mla_common.hpp plan_work: (unit, request, first tile, end tile, part, parts, record) of
+    every segment."""
+    total = sum(_tiles(n) + cost for n in lens)
+    tw = max(-(-total // units), 4)
+    out, pos = [], 0
+    for b, n in enumerate(lens):
+        pos += cost
+        nt = _tiles(n)
+        u0, u1 = pos // tw, (pos + nt - 1) // tw
+        for u in range(u0, u1 + 1):
+            out.append((u, b, max(u * tw - pos, 0), min((u + 1) * tw - pos, nt), u - u0, u1 - u0 + 1, u + b))
+        pos += nt
+    return out
+
+
+@pytest.mark.parametrize("units", [256, 128, 85, 64, 16])
+def test_balanced_split_covers_every_tile_once(units):
+    """Each request's tiles are cut into consecutive, non-empty parts on
+    consecutive units, every unit is below the round's size, and the records
+    (unit + request) are distinct, consecutive per request and fit the B * P
+    of the workspace whenever units <= B * (P - 1) + 1."""
+    rng = np.random.default_rng(units)
+    cases = [rng.integers(0, 9000, size=int(rng.integers(1, 400))).tolist() for _ in range(60)]
+    cases += [[0] * 300, [1] * 70, [100000] + [0] * 90, [64] * 256, [8192] * 64, [5]]
+    for lens in cases:
+        for cost in (4, 6):
+            segs = _segments(lens, units, cost)
+            B = len(lens)
+            P = 1 + -(-(units - 1) // B)  # the fewest parts the host lets the split run with
+            recs = [s[6] for s in segs]
+            assert recs == sorted(set(recs)) and recs[-1] < B * P, (lens, units)
+            at = [0] * B
+            for u, b, lo, hi, part, parts, rec in segs:
+                assert 0 <= u < units and lo == at[b] < hi
+                at[b] = hi
+                assert 0 <= part < parts
+            assert at == [_tiles(n) for n in lens]
+
+
+LENS = [0, 1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513, 700, 1500, 2100, 9000]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,q_len,page", [(16, 1, 64), (16, 1, 1), (5, 3, 5), (17, 1, 64), (33, 1, 1), (64, 1, 64),
+                                          (65, 1, 5), (128, 1, 64), (16, 4, 3), (128, 2, 64), (96, 8, 64)])
+def test_balanced_split_matches_oracle(H, q_len, page):
+    """Enough parts for the balanced split on 16 requests: an empty request and
+    lengths at the edges of tiles, of a CTA's share and of its index batches;
+    row groups of 64 with 1 to 64 rows; pages of consecutive slots, single
+    scattered slots, and runs that straddle a wave's 8 or 16 tokens."""
+    B = len(LENS)
+    # The oracle has no empty requests: their rows are zero.
+    pool, idx, indptr = paged_pool(LENS, 91, page=page)
+    q_lat, q_pe = rand_q(B, q_len, H, 91)
+    o = torch.full((B, q_len, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+    op = ma.mla_decode_a16w8_paged_dev
+    op(_d(q_lat), _d(q_pe), _d(pool), o, _d(torch.tensor(LENS, dtype=torch.int32)), None, _d(idx), _d(indptr), 20,
+       SCALE_576, KV_SCALE)
+    torch.cuda.synchronize()
+    assert torch.all(o[0] == 0)
+    o[0] = 0
+    _check(o, q_lat, q_pe, fp8_bits(pool), LENS, SCALE_576, kv_indices=idx.numpy(), kv_indptr=indptr.numpy(),
+           batches=list(range(1, B)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,q_len,B,S", [(16, 1, 5, 3001), (64, 1, 130, 100), (128, 1, 3, 1025), (32, 4, 2, 4097)])
+def test_balanced_split_contiguous(H, q_len, B, S):
+    kv = rand_kv_rows(B * S, 93).view(B, S, QK)
+    q_lat, q_pe = rand_q(B, q_len, H, 93)
+    if q_len == 1:
+        q_lat, q_pe = q_lat[:, 0].contiguous(), q_pe[:, 0].contiguous()
+    o = torch.full(q_lat.shape, float("nan"), dtype=torch.bfloat16, device=DEV)
+    (ma.mla_decode_a16w8 if q_len == 1 else ma.mla_decode_a16w8_multiq)(_d(q_lat), _d(q_pe), _d(kv), o, SCALE_576,
+                                                                        KV_SCALE)
+    torch.cuda.synchronize()
+    _check(o, q_lat, q_pe, fp8_bits(kv), [S] * B, SCALE_576)
+
+
+@pytest.mark.gpu
+def test_balanced_split_many_requests():
+    """More requests than a round of CTAs: several whole requests to a CTA."""
+    B, H = 700, 8
+    lens = ragged_lens(B, 0, 300, 95)
+    pool, idx, indptr = paged_pool(lens, 95)
+    q_lat, q_pe = rand_q(B, 1, H, 95)
+    o = torch.full((B, 1, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ma.mla_decode_a16w8_paged_dev(_d(q_lat), _d(q_pe), _d(pool), o, _d(torch.tensor(lens, dtype=torch.int32)), None,
+                                  _d(idx), _d(indptr), 2, SCALE_576, KV_SCALE)
+    torch.cuda.synchronize()
+    pick = [b for b in range(0, B, 13) if lens[b] > 0] + [b for b in range(B - 3, B) if lens[b] > 0]
+    _check(o, q_lat, q_pe, fp8_bits(pool), lens, SCALE_576, kv_indices=idx.numpy(), kv_indptr=indptr.numpy(),
+           batches=pick)
+    assert not torch.isnan(o.float()).any()
