@@ -16,7 +16,8 @@ namespace mla {
 constexpr int kLat = 512;
 constexpr int kRope = 64;
 constexpr int kQK = kLat + kRope;              // 576 bytes per fp8 row
-constexpr int kTileTok = 32;                   // parts are whole multiples of it (equal parts)
+constexpr int kPage = 64;                      // tokens per page of a block table
+constexpr int kTileTok = 64;                   // tokens per tile; parts are whole tiles
 constexpr int kMaxQLen = 8;
 constexpr int kMaxHeads = 128;
 // A row's running max is fixed at its first non-empty tile; later tiles may
@@ -41,15 +42,32 @@ struct Params {
   const int* rows;        // [B] q/out row per request, or null
   const int* kv_indices;  // flat per-token slots (paged)
   const int* kv_indptr;   // [B+1] (paged)
+  const int* table;       // [B, max_blocks] 64-token pages (paged, instead of kv_indices / kv_indptr), or null
+  int max_blocks, num_blocks;
   int B, H, q_len, S_fixed, parts, ngroups, paged;
   int unit_cap;           // units one round of CTAs over the CUs holds
   int workers;            // > 0: balanced split over this many units (see plan_work), 0: equal parts
   int qrows;              // H * q_len
   int rec_rows;           // O rows per split record (>= qrows)
-  int seg_cost;           // places one more part costs a unit (balanced split)
   float score_c;          // scale * kv_scale * log2(e), fp32
   float kv_scale;
 };
+
+// Request b's context length and its place in the index array: its first flat
+// slot, or its row of the block table. With a table no length reaches past the
+// row and no page id (page_slot: the slot of its first token) past the pool.
+__device__ __forceinline__ int req_len(const Params& p, int b) {
+  const int len = p.seq_lens[b];
+  if (!p.table) return len;
+  const long long most = (long long)p.max_blocks * kPage;
+  return len < 0 ? 0 : (len < most ? len : (int)most);
+}
+__device__ __forceinline__ int req_slot0(const Params& p, int b) {
+  return p.table ? b * p.max_blocks : p.kv_indptr[b];
+}
+__device__ __forceinline__ int page_slot(const Params& p, int page) {
+  return (page < 0 ? 0 : (page < p.num_blocks ? page : p.num_blocks - 1)) * kPage;
+}
 
 // Split workspace regions (see kMaxRecords).
 __device__ __forceinline__ float* ws_rec_o(const Params& p, size_t rec) { return p.ws + rec * p.rec_rows * kLat; }
@@ -84,8 +102,8 @@ __device__ __forceinline__ uint32_t u16_field(uint32_t w, int k) {
 //   U = max(B, min(B * P, cap))
 // units (request parts). Every request is cut into chunks of C tokens, request
 // b getting nparts_b = max(1, ceil(L_b / C)) parts of equal size (rounded up to
-// 32 tokens; the last part takes the remainder), with C the smallest multiple
-// of 32, at least 512, for which sum_b nparts_b <= U -- found by bisection,
+// a tile; the last part takes the remainder), with C the smallest multiple of
+// the tile, at least 512, for which sum_b nparts_b <= U -- found by bisection,
 // since the count only falls as C grows and C = max_b L_b gives B units. So the
 // partial records always fit the B * P * qrows workspace, one round of CTAs
 // covers the batch, and the longest part (the CTA that ends last) is as short
@@ -170,17 +188,17 @@ struct Unit {
 // in `scratch` (12 * B bytes of LDS that no other wave touches meanwhile). The
 // first 64 lengths and kv_indptr entries are loaded in one round of latency, so
 // the unit's length and slot offset cost no further round trip for b < 64.
-__device__ Unit plan_unit_paged(const int* seq_lens, const int* kv_indptr, int B, int P, int cap, int u, int lane,
-                                int* scratch) {
+__device__ Unit plan_unit_paged(const Params& p, int u, int lane, int* scratch) {
+  const int B = p.B, P = p.parts, cap = p.unit_cap;
   int* lens = scratch;            // [B] lengths
   int* req_at = scratch + B;      // [B] request at each position
   int* np_at = scratch + 2 * B;   // [B] parts of the request at each position
-  const int ip0 = lane < B ? kv_indptr[lane] : 0;
-  const int l0 = lane < B ? seq_lens[lane] : 0;  // the first 64 lengths stay in a register
+  const int ip0 = lane < B ? req_slot0(p, lane) : 0;
+  const int l0 = lane < B ? req_len(p, lane) : 0;  // the first 64 lengths stay in a register
   long long suml = 0;
   int maxl = 0;
   for (int c0 = 0; c0 < B; c0 += 64) {
-    const int l = c0 == 0 ? l0 : ((c0 + lane < B) ? seq_lens[c0 + lane] : 0);
+    const int l = c0 == 0 ? l0 : ((c0 + lane < B) ? req_len(p, c0 + lane) : 0);
     if (c0 + lane < B) lens[c0 + lane] = l;
     suml += wave_sum_i(l);  // per-chunk sums stay below 2^31 for lengths < 2^25
     maxl = max(maxl, wave_max_i(l));
@@ -219,7 +237,7 @@ __device__ Unit plan_unit_paged(const int* seq_lens, const int* kv_indptr, int B
     }
     r.units = run;
     r.ptok = part_tokens(r.len, r.nparts);
-    r.slot0 = r.b < 64 ? __builtin_amdgcn_readlane(ip0, r.b) : kv_indptr[r.b];
+    r.slot0 = r.b < 64 ? __builtin_amdgcn_readlane(ip0, r.b) : req_slot0(p, r.b);
     return r;
   }
   // More requests than the cap (several rounds of CTAs): longest parts first.
@@ -292,7 +310,7 @@ __device__ Unit plan_unit_paged(const int* seq_lens, const int* kv_indptr, int B
   r.units = run;
   r.len = lens[r.b];
   r.ptok = part_tokens(r.len, r.nparts);
-  r.slot0 = r.b < 64 ? __builtin_amdgcn_readlane(ip0, r.b) : kv_indptr[r.b];
+  r.slot0 = r.b < 64 ? __builtin_amdgcn_readlane(ip0, r.b) : req_slot0(p, r.b);
   // Record offset: parts of the requests before b, in request-index order.
   int rec0 = 0;
   for (int c0 = 0; c0 < B; c0 += 64) {
@@ -315,14 +333,15 @@ __device__ __forceinline__ Unit plan_unit_contig(int S, int B, int P, int cap, i
 // ---- balanced split --------------------------------------------------------------------
 // With records for it (W + B - 1 <= B * P) a round of W units shares the
 // batch's tiles evenly, whatever its lengths: the requests' 64-token tiles are
-// laid end to end, p.seg_cost places before each request standing for what
-// starting one costs a unit (4 with 64-row CTAs, 6 with 16-row ones, whose
-// tiles are shorter: 2..8 measured), and unit u walks places [u * tw, (u + 1) * tw), one
+// laid end to end, kSegCost places before each request standing for what
+// starting one costs a unit (2 .. 8 measured: 64 requests of 1024 .. 8192
+// tokens, 16 heads 39.2 us with 3, 38.3 with 4 and 5; 128 heads 103.3 us with 2,
+// 101.0 with 4, 101.6 with 8), and unit u walks places [u * tw, (u + 1) * tw), one
 // segment per request it meets there. Equal parts per request leave the longest
 // part 14% (256 units) to 80% (64 units) above the mean on lengths of
 // U[1024, 8192]. A request's segments are consecutive units, so its records
 // are consecutive too: segment (u, b) takes record u + b.
-constexpr int kWorkTile = 64;  // tokens per tile
+constexpr int kSegCost = 4;
 constexpr int kMinWork = 4;    // places per unit at least
 
 // A part of a request: what a CTA works on at a time.
@@ -336,7 +355,7 @@ struct Seg {
   int pos;             // place of the request's first tile (balanced split)
   int tw;              // places per unit (0: equal parts, one segment per unit)
 };
-__device__ __forceinline__ int work_tiles(int len) { return len > kWorkTile ? (len - 1) / kWorkTile + 1 : 1; }
+__device__ __forceinline__ int work_tiles(int len) { return len > kTileTok ? (len - 1) / kTileTok + 1 : 1; }
 
 // Unit u's segment of a request whose first tile is at `pos`.
 __device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, int slot0) {
@@ -345,8 +364,8 @@ __device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, 
   const int lo = u * tw > pos ? u * tw - pos : 0;
   const int hi = (u + 1) * tw - pos < nt ? (u + 1) * tw - pos : nt;
   const int end = len > 0 ? len : 0;
-  Seg r{b, u - u0, (pos + nt - 1) / tw - u0 + 1, u0 + b, lo * kWorkTile, end, len, slot0, pos, tw};
-  if (hi < nt) r.kv_hi = hi * kWorkTile;
+  Seg r{b, u - u0, (pos + nt - 1) / tw - u0 + 1, u0 + b, lo * kTileTok, end, len, slot0, pos, tw};
+  if (hi < nt) r.kv_hi = hi * kTileTok;
   if (hi <= 0) r.b = -1;  // the unit's places end before the tiles begin
   return r;
 }
@@ -355,7 +374,7 @@ __device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, 
 template <bool PAGED>
 __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
   if (p.workers == 0) {
-    const Unit un = PAGED ? plan_unit_paged(p.seq_lens, p.kv_indptr, p.B, p.parts, p.unit_cap, u, lane, scratch)
+    const Unit un = PAGED ? plan_unit_paged(p, u, lane, scratch)
                           : plan_unit_contig(p.S_fixed, p.B, p.parts, p.unit_cap, u);
     const long long lo = (long long)un.part * un.ptok;
     const int kv_lo = lo < un.len ? (int)lo : un.len;
@@ -369,15 +388,15 @@ __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
     return tw > kMinWork ? tw : kMinWork;
   };
   if constexpr (!PAGED) {
-    const int per = work_tiles(p.S_fixed) + p.seg_cost;
+    const int per = work_tiles(p.S_fixed) + kSegCost;
     const int tw = share(p.B * per);
     const int b = u * tw / per;
-    return b < p.B ? work_seg(u, tw, b, b * per + p.seg_cost, p.S_fixed, 0) : none;
+    return b < p.B ? work_seg(u, tw, b, b * per + kSegCost, p.S_fixed, 0) : none;
   }
-  const int l0 = lane < p.B ? p.seq_lens[lane] : 0;  // the first 64 requests cost one round trip
-  const int s0 = lane < p.B ? p.kv_indptr[lane] : 0;
-  auto len_at = [&](int c0) { return c0 == 0 ? l0 : (c0 + lane < p.B ? p.seq_lens[c0 + lane] : 0); };
-  auto places = [&](int c0, int l) { return c0 + lane < p.B ? work_tiles(l) + p.seg_cost : 0; };
+  const int l0 = lane < p.B ? req_len(p, lane) : 0;  // the first 64 requests cost one round trip
+  const int s0 = lane < p.B ? req_slot0(p, lane) : 0;
+  auto len_at = [&](int c0) { return c0 == 0 ? l0 : (c0 + lane < p.B ? req_len(p, c0 + lane) : 0); };
+  auto places = [&](int c0, int l) { return c0 + lane < p.B ? work_tiles(l) + kSegCost : 0; };
   int total = 0;
   for (int c0 = 0; c0 < p.B; c0 += 64) total += wave_sum_i(places(c0, len_at(c0)));
   const int tw = share(total);
@@ -390,7 +409,7 @@ __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
       const int h = (int)__builtin_ctzll(hit);
       const int len = __builtin_amdgcn_readlane(l, h);
       const int pos = __builtin_amdgcn_readlane(inc, h) - work_tiles(len);
-      const int slot0 = c0 == 0 ? __builtin_amdgcn_readlane(s0, h) : p.kv_indptr[c0 + h];
+      const int slot0 = c0 == 0 ? __builtin_amdgcn_readlane(s0, h) : req_slot0(p, c0 + h);
       return work_seg(u, tw, c0 + h, pos, len, slot0);
     }
     run = __builtin_amdgcn_readlane(inc, 63);
@@ -403,7 +422,7 @@ __device__ __forceinline__ Seg next_work(const Params& p, const Seg& sg, int u, 
   Seg r = sg;
   r.b = -1;
   if (sg.tw == 0 || sg.b + 1 >= p.B) return r;
-  const int pos = sg.pos + work_tiles(sg.len) + p.seg_cost;
+  const int pos = sg.pos + work_tiles(sg.len) + kSegCost;
   return pos < (u + 1) * sg.tw ? work_seg(u, sg.tw, sg.b + 1, pos, len, slot0) : r;
 }
 

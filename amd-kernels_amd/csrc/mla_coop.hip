@@ -23,9 +23,13 @@
 //    l sums cross waves at the end.
 //  * One CTA barrier per tile publishes P^T (double-buffered by tile parity) and
 //    frees the ring slot that the tile three ahead is gathered into.
-//  * The split plan also returns the request's length and slot offset, and the
-//    first slot-index batch and Q are loaded in one round of memory latency, so
-//    the first tile is requested after three dependent round trips.
+//  * A part starts with three dependent round trips: the lengths (plan), the
+//    first slot indices, then tile 0 with Q and tile 1 behind it. Later indices
+//    follow by batches of four tiles into a small ring (with a block table they
+//    are the tiles' pages), and whether a wave's 16 slots are consecutive is seen
+//    when its tile is gathered: no table is built first. Against staging all
+//    indices with Q and building a tile table: 64 requests of 1024..8192 tokens
+//    39.9 -> 38.3 us, one of 4097 19.5 -> 17.8 us.
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -50,19 +54,18 @@ constexpr int kCSlots = 4;                              // tile ring depth
 constexpr int kCQPairs = kQK / 64;                      // 9 pairs of 32-dim k-steps
 
 // LDS map (bytes). Ring slot 3 receives its first tile only after the first
-// tile barrier; before that it holds the plan scratch (wave 0), then each
-// wave's staged slot indices (9 KB per wave: 144 tiles, which bounds a segment).
+// tile barrier; before that it holds the plan scratch (wave 0), then the query
+// rows.
 constexpr int kCRingBytes = kCSlots * kCTileBytes;              // 147456
 constexpr int kCScratchOff = 3 * kCTileBytes;                   // slot 3
-constexpr int kCStageBytes = kCTileBytes / kCWaves;             // 9216 per wave
-constexpr int kCTabTiles = kCStageBytes / (kCSubTok * 4);       // 144 tiles per segment (9216 tokens)
 constexpr int kCPOff = kCRingBytes;                             // P^T of a tile: [16 rows][64 tokens] bf16
 constexpr int kCPBytes = kCRows * kCTileTok * 2;                // 2048
-constexpr int kCTabOff = kCPOff + 2 * kCPBytes;                 // 151552: [wave][kCTabTiles] first slots
-constexpr int kCMaxOff = kCTabOff + kCWaves * kCTabTiles * 4;   // 153856: [wave][16 rows] row max
-constexpr int kCLOff = kCMaxOff + kCWaves * kCRows * 4;         // 154112: [wave][16 rows] row l
-constexpr int kCMiscOff = kCLOff + kCWaves * kCRows * 4;        // 154368: unit broadcast, fallback flags
-constexpr int kCLdsBytes = kCMiscOff + 64;                      // 154432
+constexpr int kCIdxOff = kCPOff + 2 * kCPBytes;                 // slot indices [wave][2 batches of 4 tiles][16 tokens]
+constexpr int kCIdxBytes = 2 * 64 * 4;                          // per wave
+constexpr int kCMaxOff = kCIdxOff + kCWaves * kCIdxBytes;       // [wave][16 rows] row max
+constexpr int kCLOff = kCMaxOff + kCWaves * kCRows * 4;         // [wave][16 rows] row l
+constexpr int kCMiscOff = kCLOff + kCWaves * kCRows * 4;        // unit broadcast, fallback flags
+constexpr int kCLdsBytes = kCMiscOff + 64;
 static_assert(12 * kMaxPagedB <= kCTileBytes, "plan scratch fits ring slot 3");
 static_assert(kCLdsBytes <= 160 * 1024, "LDS budget");
 static_assert(kCSubBytes % 1024 == 0, "a wave's share of a tile is whole DMA instructions");
@@ -101,8 +104,7 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     asm volatile("" : "+v"(lane), "+s"(wave));
     const int i = lane & 15;  // MFMA column (query row); row of A (token for QK, dim for PV)
     const int G = lane >> 4;  // 16-lane group: k-slice of the operands, 4-row slice of the result
-    char* stg = lds + kCScratchOff + wave * kCStageBytes;  // this wave's staged slot indices
-    int* tab = reinterpret_cast<int*>(lds + kCTabOff) + wave * kCTabTiles;
+    char* idx = lds + kCIdxOff + wave * kCIdxBytes;  // this wave's slot indices
     float* red_m = reinterpret_cast<float*>(lds + kCMaxOff);
     float* red_l = reinterpret_cast<float*>(lds + kCLOff);
 
@@ -110,8 +112,8 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     const int part = sg.part;
     // The next request's length and first slot, loaded early.
     const int bn = b + 1 < p.B ? b + 1 : b;
-    const int next_len = PAGED ? p.seq_lens[bn] : p.S_fixed;
-    const int next_slot0 = PAGED ? p.kv_indptr[bn] : 0;
+    const int next_len = PAGED ? req_len(p, bn) : p.S_fixed;
+    const int next_slot0 = PAGED ? req_slot0(p, bn) : 0;
     int qb = b;
     if (p.rows) {
       qb = p.rows[b];
@@ -127,45 +129,7 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     const int qr = row_ok ? i : p.qrows - 1;  // padding columns repeat the last row
     const int t_pos = qr / p.H;
     const int lim = S - (p.q_len - 1 - t_pos);  // tokens >= lim are masked for this row
-    const long long qoff = (long long)qb * p.qrows + qr;
-
-    auto seg_end = [&](int seg_lo) {
-      const long long e = (long long)seg_lo + kCTabTiles * kCTileTok;
-      return e < kv_hi ? (int)e : kv_hi;
-    };
-    auto ntiles_of = [&](int seg_lo, int seg_hi) { return (seg_hi - seg_lo + kCTileTok - 1) / kCTileTok; };
-    // Slot indices of this wave's 16 tokens of every tile of a segment, into its
-    // staging area: one 4-byte DMA per 4 tiles (lane (G, i): tile 4q + G, token
-    // i), 256 B per DMA. Tokens past the segment re-read its last index.
-    auto stage = [&](int seg_lo, int seg_hi, int ntiles) {
-      for (int q = 0; q < (ntiles + 3) / 4; ++q) {
-        int tok = seg_lo + kCTileTok * (4 * q + G) + kCSubTok * wave + i;
-        tok = tok < seg_hi ? tok : seg_hi - 1;
-        dma4_opaque(p.kv_indices + slot0 + tok, stg + 256 * q);
-      }
-    };
-    bool prestaged = false;
-    if constexpr (PAGED) {
-      if (kv_lo < kv_hi) {
-        const int seg_hi = seg_end(kv_lo);
-        stage(kv_lo, seg_hi, ntiles_of(kv_lo, seg_hi));
-        prestaged = true;
-      }
-    }
-    // Q, as the B operand of S^T = K Q^T: k-step pair s covers dims 64s .. 64s+63;
-    // lane group G holds dims 64s + 16G .. +16 of its row, the first 8 for k-step
-    // 2s and the next 8 for k-step 2s+1 (the K fragment holds the same dims).
-    // Pair 8 is the rope part (q_pe).
-    bf16x8 qf[2 * kCQPairs];
-#pragma unroll
-    for (int s = 0; s < kCQPairs; ++s) {
-      const uint16_t* src = (s < kCQPairs - 1) ? p.q_lat + qoff * kLat + 64 * s + 16 * G : p.q_pe + qoff * kRope + 16 * G;
-      qf[2 * s] = *reinterpret_cast<const bf16x8*>(src);
-      qf[2 * s + 1] = *reinterpret_cast<const bf16x8*>(src + 8);
-    }
-    // Staged indices and Q in one round of latency; visible to the compiler, so
-    // it adds no wait of its own for Q later (when tile gathers are in flight).
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt and lgkmcnt untouched
+    const int ntiles = (kv_hi - kv_lo + kCTileTok - 1) / kCTileTok;
 
     // ---- per-lane constant offsets inside a staged tile --------------------------------
     // Staging layout: token t's 576-byte row at t*576, its
@@ -204,8 +168,138 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
       const uint32_t off = tg * kQK + 16 * (cs ^ swz(tg));
       dma_pk[k / 2] = (k & 1) ? (dma_pk[k / 2] | (off << 16)) : off;
     }
-    auto dma_off = [&](int k) -> int { return (int)((dma_pk[k / 2] >> (16 * (k & 1))) & 0xFFFFu); };
+    // The same for the slow paths, worked out again from a lane id the compiler
+    // cannot hoist, so that nothing of it stays live through the tile loop.
+    auto dma_place = [&](int k, int& tg, int& off) {
+      int l = lane;
+      asm volatile("" : "+v"(l));
+      const int pc = 64 * k + l;
+      tg = pc / 36;
+      off = 16 * ((pc - 36 * tg) ^ swz(tg));
+    };
     auto dma_offv = [&](int k) { return u16_field(dma_pk[k / 2], k & 1); };
+
+    // Slot indices of this wave's 16 tokens of tiles 4q .. 4q + 3 (lane (G, i): tile
+    // 4q + G, token i), into half q & 1 of its index ring: per-token slots, or with
+    // a block table the tile's page. Tokens past the part re-read its last index.
+    auto load_idx = [&](int q) {
+      int tok = kv_lo + kCTileTok * (4 * q + G) + kCSubTok * wave + i;
+      tok = tok < kv_hi ? tok : kv_hi - 1;
+      dma4_opaque(p.table ? p.table + slot0 + tok / kPage : p.kv_indices + slot0 + tok, idx + 256 * (q & 1));
+    };
+    // Slot of token i of this wave's share of tile j.
+    auto idx_at = [&](int j) -> int {
+      if constexpr (PAGED) {
+        const int v = *reinterpret_cast<const int*>(idx + 64 * (j & 7) + 4 * i);
+        return p.table ? page_slot(p, v) + kCSubTok * wave + i : v;
+      } else {
+        return 0;
+      }
+    };
+
+    // This wave's share of the gather of tile j (slots `v`: idx_at(j)) into ring
+    // slot j % 4. Fast path: the 16 rows are consecutive slots (one SGPR base +
+    // lane offsets); with `defer` its 9 DMAs are left pending (pend_base, pend_dst)
+    // and go out one per step of the next body. Partial: rows past the valid ones
+    // re-read the last valid row. Slow: row by row from the slots. The indices of
+    // the batch after next take the half that tile j's batch has just followed.
+    const uint8_t* pend_base = nullptr;
+    const char* pend_dst = nullptr;
+    auto issue_tile = [&](int j, int v, bool defer) -> bool {
+      const char* dst = lds + (j & (kCSlots - 1)) * kCTileBytes + wave * kCSubBytes;
+      const int tok0 = kv_lo + j * kCTileTok + kCSubTok * wave;
+      const int nvalid = kv_hi - tok0;  // <= 0: every row re-reads the part's last token
+      const uint8_t* base;
+      bool fast = true;
+      if constexpr (PAGED) {
+        if ((j & 3) == 0 && j > 0 && j + 4 < ntiles) load_idx(j / 4 + 1);
+        const int s0 = __builtin_amdgcn_readfirstlane(v);
+        base = p.kv + (long long)s0 * kQK;
+        fast = __builtin_amdgcn_ballot_w64(tok0 + i < kv_hi && v != s0 + i) == 0;
+      } else {
+        base = p.kv + ((long long)b * p.S_fixed + (nvalid > 0 ? tok0 : kv_hi - 1)) * kQK;
+      }
+      if (fast && nvalid >= kCSubTok) {
+        if (defer) {
+          pend_base = base;
+          pend_dst = dst;
+          return true;
+        }
+#pragma unroll
+        for (int k = 0; k < kCDmaPerSub; ++k) dma16_sbase_nt(base, dma_offv(k), dst + 1024 * k);
+      } else if (fast) {
+        const int nv = nvalid > 0 ? nvalid : 1;
+#pragma unroll 1
+        for (int k = 0; k < kCDmaPerSub; ++k) {
+          int tg, off;
+          dma_place(k, tg, off);
+          const int t = tg < nv ? tg : nv - 1;
+          dma16_opaque_nt(base + t * kQK + off, dst + 1024 * k);
+        }
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < kCDmaPerSub; ++k) {
+          int tg, off;
+          dma_place(k, tg, off);
+          const int row = __shfl(v, tg);
+          dma16_opaque_nt(p.kv + (long long)row * kQK + off, dst + 1024 * k);
+        }
+      }
+      return false;
+    };
+    // DMA k of a deferred gather, skipped inside the asm when nothing is
+    // pending (no branch for the compiler to split the step sequence at).
+    auto dma_if = [&](int pending, int k) {
+      const uint32_t m0v = (uint32_t)(uintptr_t)(MM_LDS const char*)(pend_dst + 1024 * k);
+      const int pu = __builtin_amdgcn_readfirstlane(pending);
+      asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 1f\n\tglobal_load_lds_dwordx4 %0, %1 nt\n1:" ::"v"(dma_offv(k)),
+                   "s"(pend_base), "{m0}"(m0v), "s"(pu)
+                   : "memory", "scc");
+    };
+    bool primed = false;  // tile 0 is on its way
+    auto prime = [&]() {
+      if constexpr (PAGED) {
+        load_idx(0);
+        if (ntiles > 4) load_idx(1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      issue_tile(0, idx_at(0), false);
+      primed = true;
+    };
+    if (ntiles > 0) prime();
+    // The query rows, 1152 bytes each (512 latent dims, 64 rope dims), into ring
+    // slot 3 by whole-row DMAs behind tile 0, row rr's 16-byte chunk c at rr *
+    // 1152 + 16 * (c ^ ((rr / 2) & 7)) (conflict-free fragment reads). Wave w
+    // fetches rows 4w .. 4w+3; padding rows repeat the last row.
+    const char* qstage = lds + kCScratchOff;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const int pc = 64 * k + lane;
+      const int rl = pc / 72, cs = pc - 72 * rl;
+      const int rr = 4 * wave + rl;
+      const int ch = cs ^ ((rr >> 1) & 7);
+      const long long qoff = (long long)qb * p.qrows + (rr < p.qrows ? rr : p.qrows - 1);
+      const uint16_t* src = ch < 64 ? p.q_lat + qoff * kLat + 8 * ch : p.q_pe + qoff * kRope + 8 * (ch - 64);
+      if (k < 4 || lane < 32) dma16_opaque(src, qstage + 4608 * wave + 1024 * k);
+    }
+    // Tile 1 goes out behind them (tile 2 in body(0)) and stays in flight.
+    if (ntiles > 1) {
+      issue_tile(1, idx_at(1), false);
+      asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    // Q, as the B operand of S^T = K Q^T: k-step pair s covers dims 64s .. 64s+63;
+    // lane group G holds dims 64s + 16G .. +16 of its row, the first 8 for k-step
+    // 2s and the next 8 for k-step 2s+1 (the K fragment holds the same dims).
+    // Pair 8 is the rope part. (Slot 3 takes its first tile after the first tile
+    // barrier.)
+    bf16x8 qf[2 * kCQPairs];
+#pragma unroll
+    for (int s = 0; s < 2 * kCQPairs; ++s) {
+      const int ch = 8 * (s >> 1) + 2 * G + (s & 1);
+      qf[s] = *reinterpret_cast<const bf16x8*>(qstage + i * 1152 + 16 * (ch ^ ((i >> 1) & 7)));
+    }
 
     f32x4 oacc[8];  // O^T, d-block j: lane (G, i) element e = dim 128w + 16j + 4G + e of row i
 #pragma unroll
@@ -214,7 +308,6 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     float row_l = 0.f;                // this lane's share of row i's sum
     bool m_fixed = false;
     bool grew = false;                // a later tile exceeded row_m by more than kGrowLimit
-    bool ring_used = false;           // a segment has run (the next one starts with a barrier)
     const float c = p.score_c;
 
     // One pass over the part. Accumulate mode: softmax + PV with each row's max
@@ -222,122 +315,16 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     // this lane's largest masked score (row_m).
     auto sweep = [&](auto max_only_tag) {
       constexpr bool kMaxOnly = decltype(max_only_tag)::value;
-      for (int seg_lo = kv_lo; seg_lo < kv_hi; seg_lo += kCTabTiles * kCTileTok) {
-        const int seg_hi = seg_end(seg_lo);
-        const int ntiles = ntiles_of(seg_lo, seg_hi);
-        // A later segment or pass: every wave is done with the ring and its
-        // staging area. (The first segment of the first pass needs no barrier:
-        // each wave gathers only its own sub-tiles, from its own table, into ring
-        // slots 0..2, and slot 3 -- plan scratch, staging -- takes its first tile
-        // only after the first tile barrier.)
-        if (ring_used) lds_reads_done_barrier();
-        ring_used = true;
-        if constexpr (PAGED) {
-          if (!prestaged) {
-            stage(seg_lo, seg_hi, ntiles);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          }
-          prestaged = false;
+      if (ntiles > 0) {
+        // A second pass: every wave is done with the ring. (In the first one tiles
+        // 0 and 1 were gathered around Q; each wave scores its own share of them.)
+        if (!primed) {
+          lds_reads_done_barrier();
+          prime();
+          if (ntiles > 1) issue_tile(1, idx_at(1), false);
         }
-        // Tile table of this wave: tab[j] = slot of the first of its 16 tokens of
-        // tile j when its valid tokens occupy consecutive slots, else -1. Built in
-        // batches of up to 8 staged dwords (4 tiles each), read before any table
-        // write so their LDS latencies overlap; the first batch covers the first
-        // gathers, the rest is built while they are in flight.
-        const int nq = (ntiles + 3) / 4;
-        auto build_tab = [&](int qa, int qb_end, auto batch_tag) {
-          constexpr int kB = decltype(batch_tag)::value;
-          for (int q0 = qa; q0 < qb_end; q0 += kB) {
-            int vv[kB];
-#pragma unroll
-            for (int k = 0; k < kB; ++k)
-              vv[k] = (q0 + k < qb_end) ? *reinterpret_cast<const int*>(stg + 256 * (q0 + k) + 4 * lane) : 0;
-#pragma unroll
-            for (int k = 0; k < kB; ++k) {
-              if (q0 + k < qb_end) {
-                const int v = vv[k];
-                const int j = 4 * (q0 + k) + G;
-                const int f0 = __builtin_amdgcn_readlane(v, 0), f1 = __builtin_amdgcn_readlane(v, 16);
-                const int f2 = __builtin_amdgcn_readlane(v, 32), f3 = __builtin_amdgcn_readlane(v, 48);
-                const int first = G == 0 ? f0 : (G == 1 ? f1 : (G == 2 ? f2 : f3));
-                const int tok = seg_lo + kCTileTok * j + kCSubTok * wave + i;
-                const unsigned long long bal = __builtin_amdgcn_ballot_w64(tok >= seg_hi || v == first + i);
-                const bool contiguous = ((bal >> (16 * G)) & 0xFFFFull) == 0xFFFFull;
-                if (i == 0 && j < ntiles) tab[j] = contiguous ? first : -1;
-              }
-            }
-          }
-        };
-        if constexpr (PAGED) build_tab(0, 1, std::integral_constant<int, 1>{});  // tiles 0..3
-        const int eff = lim < seg_hi ? lim : seg_hi;  // this row's token limit in the segment
-
-        // This wave's share of the gather of tile j into ring slot j % 4. Fast
-        // path: the 16 rows are consecutive slots (one SGPR base + lane offsets);
-        // with `defer` its 9 DMAs are left pending (pend_base, pend_dst) and go out
-        // one per step of the next body. Partial: rows past the valid ones re-read
-        // the last valid row. Slow path: every lane looks its row up.
-        const uint8_t* pend_base = nullptr;
-        const char* pend_dst = nullptr;
-        auto issue_tile = [&](int j, int tabv, bool defer) -> bool {
-          const char* dst = lds + (j & (kCSlots - 1)) * kCTileBytes + wave * kCSubBytes;
-          const int tok0 = seg_lo + j * kCTileTok + kCSubTok * wave;
-          const int nvalid = seg_hi - tok0;  // <= 0: every row re-reads the segment's last token
-          const uint8_t* base;
-          bool fast = true;
-          if constexpr (PAGED) {
-            const int s0 = __builtin_amdgcn_readfirstlane(tabv);
-            base = p.kv + (long long)s0 * kQK;
-            fast = s0 >= 0;
-          } else {
-            base = p.kv + ((long long)b * p.S_fixed + (nvalid > 0 ? tok0 : seg_hi - 1)) * kQK;
-          }
-          if (fast && nvalid >= kCSubTok) {
-            if (defer) {
-              pend_base = base;
-              pend_dst = dst;
-              return true;
-            }
-#pragma unroll
-            for (int k = 0; k < kCDmaPerSub; ++k) dma16_sbase_nt(base, dma_offv(k), dst + 1024 * k);
-          } else if (fast) {
-            const int nv = nvalid > 0 ? nvalid : 1;
-#pragma unroll 1
-            for (int k = 0; k < kCDmaPerSub; ++k) {
-              const int o = dma_off(k);
-              const int tg = (o * 7282) >> 22;  // o / 576 for o < 9216
-              const int t = tg < nv ? tg : nv - 1;
-              dma16_opaque_nt(base + t * kQK + (o - tg * kQK), dst + 1024 * k);
-            }
-          } else {
-            int tk = tok0 + i;
-            tk = tk < seg_hi ? tk : seg_hi - 1;
-            const int myrow = p.kv_indices[slot0 + tk];  // lanes (G, i): slot of token tok0 + i
-#pragma unroll 1
-            for (int k = 0; k < kCDmaPerSub; ++k) {
-              const int o = dma_off(k);
-              const int tg = (o * 7282) >> 22;
-              const int row = __shfl(myrow, tg);
-              dma16_opaque_nt(p.kv + (long long)row * kQK + (o - tg * kQK), dst + 1024 * k);
-            }
-          }
-          return false;
-        };
-        // DMA k of a deferred gather, skipped inside the asm when nothing is
-        // pending (no branch for the compiler to split the step sequence at).
-        auto dma_if = [&](int pending, int k) {
-          const uint32_t m0v = (uint32_t)(uintptr_t)(MM_LDS const char*)(pend_dst + 1024 * k);
-          const int pu = __builtin_amdgcn_readfirstlane(pending);
-          asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 1f\n\tglobal_load_lds_dwordx4 %0, %1 nt\n1:" ::"v"(dma_offv(k)),
-                       "s"(pend_base), "{m0}"(m0v), "s"(pu)
-                       : "memory", "scc");
-        };
-        auto tab_at = [&](int j) -> int {
-          if constexpr (PAGED) {
-            return tab[j];
-          } else {
-            return 0;
-          }
-        };
+        primed = false;
+        const int eff = lim < kv_hi ? lim : kv_hi;  // this row's token limit in the part
 
         // Software pipeline over the tiles. body(t) waits for this wave's share
         // of tile t and computes its S^T; interleaved with those 18 MFMAs run the
@@ -414,9 +401,9 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
         };
 
         bool pend = false;  // a deferred gather waits for the next body
-        auto finish = [&](int t, const f32x4 sacc, int tab_next) {
-          // Lane (G, i), element e: token seg_lo + 64t + 16w + 4G + e of row i.
-          const int rel = eff - (seg_lo + t * kCTileTok + kCSubTok * wave + 4 * G);  // e valid iff e < rel
+        auto finish = [&](int t, const f32x4 sacc, int idx_next) {
+          // Lane (G, i), element e: token kv_lo + 64t + 16w + 4G + e of row i.
+          const int rel = eff - (kv_lo + t * kCTileTok + kCSubTok * wave + 4 * G);  // e valid iff e < rel
           float sv[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) sv[e] = (e < rel) ? sacc[e] : -__builtin_inff();
@@ -448,25 +435,22 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
           // ---- tile barrier: P^T(t) published, every wave's share of tile t landed,
           // every wave done with tile t-1 (its slot takes tile t+3) ----
           lds_reads_done_barrier();
-          pend = (t + 3 < ntiles) ? issue_tile(t + 3, tab_next, true) : false;
+          pend = (t + 3 < ntiles) ? issue_tile(t + 3, idx_next, true) : false;
         };
 
-        // Tiles 0 and 1 now; a fast-path tile 2 goes out one DMA per step of
-        // body(0) (108 back-to-back DMAs per CU stall the issuing waves for ~1 us).
-        issue_tile(0, tab_at(0), false);
-        if (ntiles > 1) issue_tile(1, tab_at(1), false);
-        const bool pend0 = (ntiles > 2) ? issue_tile(2, tab_at(2), true) : false;
-        if constexpr (PAGED) build_tab(1, nq, std::integral_constant<int, 8>{});
+        // A fast-path tile 2 goes out one DMA per step of body(0) (108 back-to-back
+        // DMAs per CU stall the issuing waves for ~1 us).
+        const bool pend0 = (ntiles > 2) ? issue_tile(2, idx_at(2), true) : false;
         // Tile 0 has no PV before it (peeled, so the accumulators stay put in the loop).
-        finish(0, body(0, pend0, ntiles > 1 ? 9 : 0, std::false_type{}), ntiles > 3 ? tab_at(3) : 0);
+        finish(0, body(0, pend0, ntiles > 1 ? 9 : 0, std::false_type{}), ntiles > 3 ? idx_at(3) : 0);
         for (int t = 1; t < ntiles; ++t) {
-          const int tab_next = (t + 3 < ntiles) ? tab_at(t + 3) : 0;
+          const int idx_next = (t + 3 < ntiles) ? idx_at(t + 3) : 0;
           const int pd = pend;
           const int vm_left = t + 1 < ntiles ? 9 : 0;
           if constexpr (kMaxOnly) {
-            finish(t, body(t, pd, vm_left, std::false_type{}), tab_next);
+            finish(t, body(t, pd, vm_left, std::false_type{}), idx_next);
           } else {
-            finish(t, body(t, pd, vm_left, std::true_type{}), tab_next);
+            finish(t, body(t, pd, vm_left, std::true_type{}), idx_next);
           }
         }
         if constexpr (!kMaxOnly) pv_last(ntiles - 1);

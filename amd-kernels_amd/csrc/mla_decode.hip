@@ -13,7 +13,7 @@
 // format, the work split, the split records and the numerics (mla_common.hpp):
 // mla_coop.hip for up to 16 query rows, mla_rows64.hip for more (64 rows per
 // CTA). This file holds what surrounds them: the merge of split requests, the
-// block-table expansion, the planners and the C ABI.
+// planners and the C ABI.
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -146,38 +146,6 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(Params p) {
   __builtin_nontemporal_store(o, reinterpret_cast<u32x2*>(p.o_lat + ((long long)qb * p.qrows + qrow) * kLat + d));
 }
 
-// ---------------------------------------------------------------------------
-// 64-token block tables -> the flat per-token slots the decode reads. Request
-// b's slots go at stride max_blocks * 64: idx[b * stride + t] = page(b, t / 64)
-// * 64 + t % 64 for t < len_b, with page ids clamped to the pool and
-// len_b = seq_lens[b] clamped to [0, max_blocks * 64], so no table content
-// makes the decode read outside the pool. Index workspace (int32):
-// [B * stride slots][B lengths][B + 1 offsets]. One thread per token slot of
-// the table (4 pages per 256-thread CTA).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void expand_block_table_kernel(const int* __restrict__ seq_lens,
-                                                                 const int* __restrict__ table, int max_blocks,
-                                                                 int num_blocks, int B, int* __restrict__ ws) {
-  const long long page = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (page >= (long long)B * max_blocks) return;
-  const int b = (int)(page / max_blocks), j = (int)(page % max_blocks);
-  const long long stride = (long long)max_blocks * 64;
-  int len = seq_lens[b];
-  len = len < 0 ? 0 : (len > stride ? (int)stride : len);
-  const int t = j * 64 + lane;
-  if (t < len) {
-    int blk = table[page];
-    blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
-    ws[b * stride + t] = blk * 64 + lane;
-  }
-  if (j == 0 && lane == 0) {
-    ws[B * stride + b] = len;
-    ws[B * stride + B + b] = (int)(b * stride);
-    if (b == B - 1) ws[B * stride + 2 * B] = (int)(B * stride);
-  }
-}
-
 // Test hook: decode fp8 bytes with the same hardware convert the kernel uses.
 __global__ void fp8_to_bf16_kernel(const uint8_t* in, uint16_t* out, int n) {
   const int i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
@@ -291,7 +259,7 @@ int check_launch_args(const void* q_lat, const void* q_pe, const void* kv, const
 int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, const void* seq_lens,
            const void* rows, const void* kv_indices, const void* kv_indptr, int B, int H, int S_fixed, int parts,
            int q_len, int lat_dim, int rope_dim, float scale, float kv_scale, void* workspace, void* stream,
-           bool paged) {
+           bool paged, const void* table = nullptr, int max_blocks = 0, int num_blocks = 0) {
   const int arg_rc = check_launch_args(q_lat, q_pe, kv, o_lat, seq_lens, kv_indices, kv_indptr, B, H, S_fixed, q_len,
                                        lat_dim, rope_dim, paged);
   if (arg_rc != 0) return arg_rc;
@@ -305,6 +273,9 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   p.rows = static_cast<const int*>(rows);
   p.kv_indices = static_cast<const int*>(kv_indices);
   p.kv_indptr = static_cast<const int*>(kv_indptr);
+  p.table = static_cast<const int*>(table);
+  p.max_blocks = max_blocks;
+  p.num_blocks = num_blocks;
   p.B = B;
   p.H = H;
   p.q_len = q_len;
@@ -316,7 +287,6 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   p.paged = paged ? 1 : 0;
   p.qrows = H * q_len;
   p.rec_rows = rec_rows_for(H, q_len);
-  p.seg_cost = use_coop(H, q_len) ? 6 : 4;
   p.score_c = (float)((double)scale * (double)kv_scale * 1.4426950408889634);
   p.kv_scale = kv_scale;
   // Unit slots per XCD for the snake deal of units 0..U-1, U <= B * parts (the
@@ -443,15 +413,10 @@ int launch_mla_decode_a16w8_paged_blocks_dev(const void* q_lat, const void* q_pe
   if (max_blocks < 1 || num_blocks < 1) return -11;
   const long long words = (long long)B * max_blocks * 64 + 2LL * B + 1;
   if (words > 0x7FFFFFFFLL || (long long)num_blocks * 64 > 0x7FFFFFFFLL) return -11;
-  int* ws = static_cast<int*>(index_workspace);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const long long pages = (long long)B * max_blocks;
-  hipLaunchKernelGGL(expand_block_table_kernel, dim3((unsigned)((pages + 3) / 4)), dim3(256), 0, st,
-                     static_cast<const int*>(seq_lens), static_cast<const int*>(block_table), max_blocks, num_blocks,
-                     B, ws);
-  const long long stride_all = (long long)B * max_blocks * 64;
-  return launch(q_lat, q_pe, kv_pool, o_lat, ws + stride_all, rows, ws, ws + stride_all + B, B, H, 0, parts, q_len,
-                lat_dim, rope_dim, scale, kv_scale, workspace, stream, true);
+  // The kernels read the table themselves (a page is a tile): no per-token slots
+  // are written, and the index workspace, sized for them, stays untouched.
+  return launch(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, block_table, block_table, B, H, 0, parts, q_len, lat_dim,
+                rope_dim, scale, kv_scale, workspace, stream, true, block_table, max_blocks, num_blocks);
 }
 
 int launch_mla_decode_a16w8_multiq(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, int B, int H,

@@ -134,8 +134,8 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
     const int part = sg.part;
     // The next request's length and first slot, loaded early.
     const int bn = b + 1 < p.B ? b + 1 : b;
-    const int next_len = PAGED ? p.seq_lens[bn] : p.S_fixed;
-    const int next_slot0 = PAGED ? p.kv_indptr[bn] : 0;
+    const int next_len = PAGED ? req_len(p, bn) : p.S_fixed;
+    const int next_slot0 = PAGED ? req_slot0(p, bn) : 0;
     int qb = b;
     if (p.rows) {
       qb = p.rows[b];
@@ -203,17 +203,18 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
     };
 
     // Slot indices of this wave's 8 tokens of tiles 8q .. 8q + 7 (lane 8j + i: tile
-    // 8q + j, token i), into half q & 1 of its index ring. Tokens past the part
-    // re-read its last index.
+    // 8q + j, token i), into half q & 1 of its index ring: per-token slots, or with
+    // a block table the tile's page. Tokens past the part re-read its last index.
     auto load_idx = [&](int q) {
       int tok = kv_lo + kRTileTok * (8 * q + (lane >> 3)) + kRSubTok * wave + (lane & 7);
       tok = tok < kv_hi ? tok : kv_hi - 1;
-      dma4_opaque(p.kv_indices + slot0 + tok, idx + 256 * (q & 1));
+      dma4_opaque(p.table ? p.table + slot0 + tok / kPage : p.kv_indices + slot0 + tok, idx + 256 * (q & 1));
     };
     // Slot of token lane % 8 of this wave's share of tile j.
     auto idx_at = [&](int j) -> int {
       if constexpr (PAGED) {
-        return *reinterpret_cast<const int*>(idx + 32 * (j & 15) + 4 * (lane & 7));
+        const int v = *reinterpret_cast<const int*>(idx + 32 * (j & 15) + 4 * (lane & 7));
+        return p.table ? page_slot(p, v) + kRSubTok * wave + (lane & 7) : v;
       } else {
         return 0;
       }

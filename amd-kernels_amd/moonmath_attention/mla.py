@@ -196,9 +196,8 @@ def mla_decode_a16w8_paged_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_t
     [B, max_blocks], request b's token t is row t % 64 of page
     block_table[b, t // 64]; q_lat [B,H,512] (q_len 1) or [B,q_len,H,512]
     (q_len <= 8), draft window end-aligned; rows as in the paged ops. Device
-    driven and graph capturable with ``parts`` fixed: the table is expanded to
-    per-token slots on the GPU (page ids clamped to the pool, lengths to the
-    table) and the flat-slot decode runs on the same stream.
+    driven and graph capturable with ``parts`` fixed: the decode reads the table
+    on the GPU (page ids clamped to the pool, lengths to the table).
     """
     who = "mla_decode_a16w8_paged_blocks"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
@@ -227,14 +226,12 @@ def mla_decode_a16w8_paged_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_t
     num_blocks = kv_pool.numel() // (_PAGE * _QK)
     max_blocks = block_table.shape[1]
     dev = q_lat.device
-    lib = _lib.lib
     with torch.cuda.device(dev):
         ws = _workspace(B, H, parts, q_len, dev)
-        idx_ws = torch.empty(lib.mla_decode_a16w8_blocks_index_bytes(B, max_blocks), dtype=torch.uint8, device=dev)
         _run("launch_mla_decode_a16w8_paged_blocks_dev", _lib.ptr(q_lat), _lib.ptr(q_pe), _lib.ptr(kv_pool),
              _lib.ptr(o_lat), _lib.ptr(seq_lens), _lib.ptr(rows), _lib.ptr(block_table), max_blocks, num_blocks,
              B, H, int(parts), q_len, _LAT, _ROPE, float(scale), float(kv_scale), float(scale_p), _lib.ptr(ws),
-             _lib.ptr(idx_ws), _lib.stream_ptr(dev))
+             _lib.ptr(block_table), _lib.stream_ptr(dev))  # the index workspace is not touched
 
 
 def mla_decode_a16w8_plan_parts(B: int, H: int, max_seq_len: int, lat_dim: int = 512) -> int:

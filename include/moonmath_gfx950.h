@@ -165,10 +165,10 @@ int launch_mla_decode_a16w8_paged_dev_noalloc(const void* q_lat, const void* q_p
  * 64 fused 576-byte rows; request b's token t lives in page
  * block_table[b * max_blocks + t / 64], row t % 64; q_len 1..8 as in
  * launch_mla_decode_a16w8_paged_dev (rows, parts, workspace likewise).
- * index_workspace: mla_decode_a16w8_blocks_index_bytes(B, max_blocks) bytes
- * into which the table is expanded to per-token slots (page ids clamped to
- * [0, num_blocks), lengths to [0, max_blocks * 64]) before the decode, on the
- * same stream. Codes: as the paged launcher, plus -11 (max_blocks or
+ * Page ids are clamped to [0, num_blocks), lengths to [0, max_blocks * 64]. The
+ * kernels read the table themselves: index_workspace, once the place of the
+ * expanded slots (mla_decode_a16w8_blocks_index_bytes), must be given but is
+ * not touched. Codes: as the paged launcher, plus -11 (max_blocks or
  * num_blocks < 1, or tables beyond int32 indexing). No counterpart in the
  * reference, whose decode takes flat per-token slots only: this is the
  * block-table form a serving stack's paged KV cache keeps. */

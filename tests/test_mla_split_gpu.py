@@ -15,7 +15,7 @@ def _tiles(n):
     return max(1, -(-n // 64))
 
 
-def _segments(lens, units, cost):
+def _segments(lens, units, cost=4):
     """csrc/mla_common.hpp plan_work: (unit, request, first tile, end tile, part, parts, record) of
     every segment."""
     total = sum(_tiles(n) + cost for n in lens)
@@ -41,18 +41,17 @@ def test_balanced_split_covers_every_tile_once(units):
     cases = [rng.integers(0, 9000, size=int(rng.integers(1, 400))).tolist() for _ in range(60)]
     cases += [[0] * 300, [1] * 70, [100000] + [0] * 90, [64] * 256, [8192] * 64, [5]]
     for lens in cases:
-        for cost in (4, 6):
-            segs = _segments(lens, units, cost)
-            B = len(lens)
-            P = 1 + -(-(units - 1) // B)  # the fewest parts the host lets the split run with
-            recs = [s[6] for s in segs]
-            assert recs == sorted(set(recs)) and recs[-1] < B * P, (lens, units)
-            at = [0] * B
-            for u, b, lo, hi, part, parts, rec in segs:
-                assert 0 <= u < units and lo == at[b] < hi
-                at[b] = hi
-                assert 0 <= part < parts
-            assert at == [_tiles(n) for n in lens]
+        segs = _segments(lens, units)
+        B = len(lens)
+        P = 1 + -(-(units - 1) // B)  # the fewest parts the host lets the split run with
+        recs = [s[6] for s in segs]
+        assert recs == sorted(set(recs)) and recs[-1] < B * P, (lens, units)
+        at = [0] * B
+        for u, b, lo, hi, part, parts, rec in segs:
+            assert 0 <= u < units and lo == at[b] < hi
+            at[b] = hi
+            assert 0 <= part < parts
+        assert at == [_tiles(n) for n in lens]
 
 
 LENS = [0, 1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513, 700, 1500, 2100, 9000]
@@ -110,3 +109,25 @@ def test_balanced_split_many_requests():
     _check(o, q_lat, q_pe, fp8_bits(pool), lens, SCALE_576, kv_indices=idx.numpy(), kv_indptr=indptr.numpy(),
            batches=pick)
     assert not torch.isnan(o.float()).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,parts", [(16, 1), (16, 70), (64, 1), (64, 70)])
+def test_block_table_clamps_pages_and_lengths(H, parts):
+    """The table is read by the decode itself: page ids outside the pool and
+    lengths outside the table give what the clamped table and lengths give, bit
+    for bit, in both kernels and both splits."""
+    B, max_blocks, num_blocks = 4, 9, 20
+    g = torch.Generator().manual_seed(97)
+    pool = rand_kv_rows(num_blocks * 64, 97).view(num_blocks, 64, QK)
+    table = torch.randint(-5, num_blocks + 5, (B, max_blocks), generator=g, dtype=torch.int32)
+    lens = torch.tensor([-3, 577, 130, 100000], dtype=torch.int32)
+    q_lat, q_pe = (t[:, 0].contiguous() for t in rand_q(B, 1, H, 97))
+    outs = []
+    for t, n in ((table, lens), (table.clamp(0, num_blocks - 1), lens.clamp(0, max_blocks * 64))):
+        o = torch.full((B, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ma.mla_decode_a16w8_paged_blocks(_d(q_lat), _d(q_pe), _d(pool), o, _d(n), _d(t), parts, SCALE_576, KV_SCALE)
+        torch.cuda.synchronize()
+        outs.append(o)
+    assert not torch.isnan(outs[0].float()).any()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
