@@ -3,13 +3,15 @@
 Every ``csrc/*.hip`` file is compiled to an object for gfx950 only, then all
 objects are linked into one shared library next to this file. No torch
 extension machinery is involved: the library exports plain ``extern "C"``
-symbols that ``_lib.py`` binds with ctypes.
+symbols that ``_lib.py`` binds with ctypes. ``csrc/calls.cpp`` (host code
+against libtorch and the CPython C API) becomes the ``_calls`` module.
 """
 import os
 import pathlib
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 ROOT = pathlib.Path(__file__).resolve().parent
 PKG_DIR = ROOT / "moonmath_attention"
@@ -17,6 +19,7 @@ SRC_DIR = ROOT / "csrc"
 BUILD_DIR = ROOT / "_build"
 LIB_NAME = "libmoonmath_gfx950.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+CALLS_PATH = PKG_DIR / "_calls.so"
 
 ARCH = "gfx950"
 # -packed-fp32-ops: keep hipcc from emitting v_pk_{add,mul,fma}_f32 (ordinary
@@ -44,8 +47,21 @@ def sources():
     return sorted(SRC_DIR.glob("*.hip"))
 
 
+def _calls_command(out):
+    """Compile and link ``csrc/calls.cpp`` with the host compiler."""
+    from importlib.util import find_spec
+
+    torch_dir = pathlib.Path(find_spec("torch").origin).parent
+    inc = torch_dir / "include"
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}",
+            f"-I{sysconfig.get_paths()['include']}", f"-I{pathlib.Path(_hipcc()).parents[1] / 'include'}",
+            str(SRC_DIR / "calls.cpp"), "-o", str(out), f"-L{torch_dir / 'lib'}",
+            "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
+
+
 def build(verbose=False):
-    """Compile all sources (in parallel) and link the shared library."""
+    """Compile all sources (in parallel), link the shared library and the _calls module."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     procs = []
@@ -57,6 +73,11 @@ def build(verbose=False):
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
+    calls_tmp = CALLS_PATH.with_suffix(".so.tmp")
+    cmd = _calls_command(calls_tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    procs.append((SRC_DIR / "calls.cpp", subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
     failed = []
     for src, p in procs:
         out, _ = p.communicate()
@@ -76,6 +97,7 @@ def build(verbose=False):
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout.decode(errors="replace"))
     os.replace(tmp, LIB_PATH)
+    os.replace(calls_tmp, CALLS_PATH)
     return LIB_PATH
 
 

@@ -39,6 +39,9 @@ def forward(
     Returns:
         torch.bfloat16 tensor of q's shape on q's device.
     """
+    res = _lib.calls.forward(q, k, v, out, round_mode, layout)
+    if res is not None:
+        return res
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be torch.Tensor; got {type(t).__name__}")
@@ -191,6 +194,10 @@ def forward_lite(
     pins processed blocks as kept in the next list.
     MOONMATH_LITE_PLAIN=1 disables the LPT (heaviest-first) CTA order.
     """
+    if must_do_list is None:
+        res = _lib.calls.forward_lite(q, k, v, read_list, write_list, threshold, phase, out, round_mode, layout)
+        if res is not None:
+            return res
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be torch.Tensor; got {type(t).__name__}")

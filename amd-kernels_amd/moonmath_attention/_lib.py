@@ -9,6 +9,8 @@ at import time -- there is no fallback path.
 import ctypes
 import os
 
+import torch  # noqa: F401  (loads the libtorch that _calls is linked to)
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("MOONMATH_LIB") or os.path.join(_HERE, "libmoonmath_gfx950.so")
 
@@ -83,11 +85,19 @@ class _Lib:
 
 lib = _Lib(LIB_PATH)
 
+try:
+    from . import _calls as calls
+except ImportError as e:
+    raise ImportError(
+        f"moonmath_attention: the _calls module is not usable ({e}). "
+        "Build it with `python amd-kernels_amd/build_lib.py`."
+    ) from e
+# The plain GPU calls go through native code to the same launchers (csrc/calls.cpp).
+calls.bind({name: ctypes.cast(getattr(lib.dll, name), _p).value for name in calls.bound_names()})
+
 
 def stream_ptr(device):
     """Raw hipStream_t of torch's current stream on ``device``."""
-    import torch
-
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 

@@ -144,6 +144,8 @@ def mla_decode_a16w8(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0) -> No
     o_lat [B,H,512] bf16 (written in place). scale = softmax scale,
     kv_scale = per-tensor fp8 KV descale. (Reference mla.py:41-61.)
     """
+    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, False):
+        return
     who = "mla_decode_a16w8"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
     if q_len != 1:
@@ -170,6 +172,9 @@ def mla_decode_a16w8_paged_dev(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_i
     int32 maps request -> q/out batch row (None = identity); parts is fixed by
     the caller (plan_parts*). (Reference mla.py:64-95.)
     """
+    if _lib.calls.mla_paged(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, parts, scale, kv_scale,
+                            False):
+        return
     who = "mla_decode_a16w8_paged_dev"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
     _check_paged(kv_pool, seq_lens, rows, kv_indices, kv_indptr, parts, B, who)
@@ -199,6 +204,8 @@ def mla_decode_a16w8_paged_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_t
     driven and graph capturable with ``parts`` fixed: the decode reads the table
     on the GPU (page ids clamped to the pool, lengths to the table).
     """
+    if _lib.calls.mla_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_table, parts, scale, kv_scale, rows):
+        return
     who = "mla_decode_a16w8_paged_blocks"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
     if not isinstance(kv_pool, torch.Tensor) or kv_pool.dtype != _FP8:
@@ -256,6 +263,8 @@ def mla_decode_a16w8_multiq(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0
     float8_e4m3fn; o_lat like q_lat. Position t attends kv[:, : S - q_len + t + 1].
     (Reference mla.py:122-145.)
     """
+    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, True):
+        return
     who = "mla_decode_a16w8_multiq"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=True)
     _check_slab(kv, B, who)
@@ -272,6 +281,9 @@ def mla_decode_a16w8_multiq_paged_dev(q_lat, q_pe, kv_pool, o_lat, seq_lens, row
                                       scale, kv_scale, scale_p=1.0) -> None:
     """Multi-query decode over a paged pool, device-driven (graph capturable).
     (Reference mla.py:148-176.)"""
+    if _lib.calls.mla_paged(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, parts, scale, kv_scale,
+                            True):
+        return
     who = "mla_decode_a16w8_multiq_paged_dev"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=True)
     _check_paged(kv_pool, seq_lens, rows, kv_indices, kv_indptr, parts, B, who)
@@ -303,6 +315,8 @@ def mla_kv_quantize(c_kv, k_pe, kv_pool, slots, kv_scale, saturate=False) -> Non
     (moonmath_attention/mla.py:17-20) filled the way its tests fill it
     (tests/test_mla_decode.py:34-38).
     """
+    if _lib.calls.kv_quantize(c_kv, k_pe, kv_pool, slots, kv_scale, saturate):
+        return
     who = "mla_kv_quantize"
     for name, t, w in (("c_kv", c_kv, _LAT), ("k_pe", k_pe, _ROPE)):
         if not isinstance(t, torch.Tensor) or t.dtype != torch.bfloat16:

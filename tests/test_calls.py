@@ -1,0 +1,165 @@
+"""The native call path (csrc/calls.cpp): it takes plain GPU calls and nothing
+else, and gives what the Python path gives."""
+import threading
+
+import pytest
+import torch
+
+import moonmath_attention as ma
+from moonmath_attention import _lib
+from mla_inputs import KV_SCALE, QK, SCALE_192, paged_pool, rand_kv_rows, rand_q
+
+DEV = "cuda:0"
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_leaves_everything_else_to_python():
+    """CPU tensors, other types, subclasses, wrong counts of arguments: None, with
+    nothing done, so that the wrapper's checks decide."""
+    q = torch.zeros(1, 2, 8, 128, dtype=torch.bfloat16)
+    c = _lib.calls
+    for args in ((q, q, q, None, "rtna", "bhsd"), (q.float(), q, q, None, "rtna", "bhsd"),
+                 (q.as_subclass(_Sub), q, q, None, "rtna", "bhsd"), (1, q, q, None, "rtna", "bhsd"),
+                 (q, q, q, None, "xyz", "bhsd"), (q, q, q, None, 3, "bhsd"), (q, q)):
+        assert c.forward(*args) is None
+    assert c.forward_lite(q, q, q, q, q, -6.0, 1, None, "rtna", "bhsd") is None
+    assert c.mla_slab(q, q, q, q, 1.0, 1.0, False) is None
+    assert c.mla_paged(q, q, q, q, q, None, q, q, 1, 1.0, 1.0, True) is None
+    assert c.mla_blocks(q, q, q, q, q, q, 1, 1.0, 1.0, None) is None
+    assert c.kv_quantize(q, q, q, q, 1.0, False) is None
+
+
+def test_binds_every_launcher_it_uses():
+    assert all(hasattr(_lib.lib, name) for name in _lib.calls.bound_names())
+
+
+def _python_path(monkeypatch):
+    """The wrappers without the native path."""
+
+    class Off:
+        def __getattr__(self, name):
+            return lambda *a: None
+
+    monkeypatch.setattr(_lib, "calls", Off())
+
+
+def _both(monkeypatch, fn):
+    got = fn()
+    torch.cuda.synchronize()
+    with monkeypatch.context() as m:
+        _python_path(m)
+        want = fn()
+        torch.cuda.synchronize()
+    for a, b in zip(got, want, strict=True):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.device == b.device
+        assert torch.equal(a.view(torch.int8), b.view(torch.int8))
+
+
+def _qkv(layout, Sq=300, Skv=200, B=2, H=3):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    shape = (lambda s: (B, H, s, 128)) if layout == "bhsd" else (lambda s: (B, s, H, 128))
+    return [torch.randn(shape(s), generator=g, device=DEV).bfloat16() for s in (Sq, Skv, Skv)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("mode", ["rtna", "rtne", "rtz"])
+def test_attention_equals_the_python_path(layout, mode, monkeypatch):
+    q, k, v = _qkv(layout)
+    _both(monkeypatch, lambda: [ma.forward(q, k, v, round_mode=mode, layout=layout)])
+    out = torch.empty_like(q)
+    assert ma.forward(q, k, v, out=out, round_mode=mode, layout=layout) is out
+    _both(monkeypatch, lambda: [ma.forward(q, k, v, out=out, round_mode=mode, layout=layout).clone()])
+
+    def lite():
+        la = ma.LiteAttention(threshold=-3.0, round_mode=mode, layout=layout)
+        outs = [la(q, k, v) for _ in range(3)]
+        return outs + [la.read_list.clone(), la.write_list.clone()]
+
+    _both(monkeypatch, lite)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_len", [1, 3])
+def test_mla_equals_the_python_path(q_len, monkeypatch):
+    B, H, lens = 3, 16, [700, 64, 1300]
+    pool, idx, indptr = paged_pool(lens, 5)
+    q_lat, q_pe = (t.to(DEV) for t in rand_q(B, q_len, H, 5))
+    if q_len == 1:
+        q_lat, q_pe = q_lat[:, 0].contiguous(), q_pe[:, 0].contiguous()
+    pool, idx, indptr = pool.to(DEV), idx.to(DEV), indptr.to(DEV)
+    n = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    rows = torch.tensor([2, 0, 1], dtype=torch.int32, device=DEV)
+    slab = rand_kv_rows(B * 500, 7).view(B, 500, QK).to(DEV)
+    table = torch.arange(3 * 5, dtype=torch.int32, device=DEV).view(3, 5)
+    multi = q_len > 1
+
+    def run():
+        outs = [torch.full_like(q_lat, 7.0) for _ in range(4)]
+        (ma.mla_decode_a16w8_multiq if multi else ma.mla_decode_a16w8)(q_lat, q_pe, slab, outs[0], SCALE_192, KV_SCALE)
+        op = ma.mla_decode_a16w8_multiq_paged_dev if multi else ma.mla_decode_a16w8_paged_dev
+        op(q_lat, q_pe, pool, outs[1], n, None, idx, indptr, 4, SCALE_192, KV_SCALE)
+        op(q_lat, q_pe, pool, outs[2], n, rows, idx, indptr, 1, SCALE_192, KV_SCALE)
+        ma.mla_decode_a16w8_paged_blocks(q_lat, q_pe, pool.view(-1, 64, QK), outs[3], n, table, 4, SCALE_192, KV_SCALE)
+        return outs
+
+    _both(monkeypatch, run)
+
+
+@pytest.mark.gpu
+def test_kv_quantize_equals_the_python_path(monkeypatch):
+    g = torch.Generator(device=DEV).manual_seed(9)
+    c, r = (torch.randn(50, w, generator=g, device=DEV).bfloat16() * 20 for w in (512, 64))
+    slots = torch.randperm(60, generator=g, device=DEV)[:50].int()
+
+    def run():
+        outs = []
+        for sat in (False, True):
+            pool = torch.zeros(60, QK, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn)
+            ma.mla_kv_quantize(c, r, pool, slots, 0.03125, sat)
+            outs.append(pool)
+        return outs
+
+    _both(monkeypatch, run)
+
+
+@pytest.mark.gpu
+def test_refusals_stay_refused_on_gpu():
+    q, k, v = _qkv("bhsd")
+    with pytest.raises(TypeError, match="must be torch.bfloat16"):
+        ma.forward(q.float(), k, v)
+    with pytest.raises(ValueError, match="must be contiguous"):
+        ma.forward(q.transpose(1, 2), k, v, layout="bshd")
+    with pytest.raises(ValueError, match="k shape mismatch"):
+        ma.forward(q, k[:1].contiguous(), v)
+    with pytest.raises(ValueError, match="out shape must match"):
+        ma.forward(q, k, v, out=k)
+    with pytest.raises(ValueError, match="round_mode must be"):
+        ma.forward(q, k, v, round_mode="up")
+    sub = ma.forward(q.as_subclass(_Sub), k, v)  # taken, by the Python path
+    assert torch.equal(sub.as_subclass(torch.Tensor), ma.forward(q, k, v))
+
+
+@pytest.mark.gpu
+def test_streams_and_threads():
+    """Calls from several threads, each on a stream of its own, on inputs of
+    their own: every result is that of the call alone."""
+    sets = [_qkv("bhsd", Sq=256 + 64 * i, Skv=1000) for i in range(4)]
+    want = [ma.forward(*s) for s in sets]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            outs = [ma.forward(*sets[i]) for _ in range(20)]
+        st.synchronize()
+        bad.extend(i for o in outs if not torch.equal(o, want[i]))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad
