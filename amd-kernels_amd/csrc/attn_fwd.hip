@@ -10,14 +10,14 @@
 //    S^T = K Q^T (A = K fragment, B = Q fragment), so each lane owns one query
 //    column and 16 kv rows per 32x32 tile; P^T then feeds O^T = V^T P^T as the
 //    B operand straight from registers (no shuffle).
-//  * K and the pre-transposed V_t are staged through LDS with 16-byte
-//    global->LDS DMA (global_load_lds_dwordx4) in 4-slot rings, two blocks of
-//    lead. Every DMA is inline asm, waited for by explicit vmcnt waits: with
+//  * K and V (up to 12288 query rows, see prefers_direct) or a pre-transposed
+//    V_t (more) are staged through LDS with 16-byte global->LDS DMA
+//    (global_load_lds_dwordx4) in 4-slot rings, two blocks of lead. Every DMA is inline asm, waited for by explicit vmcnt waits: with
 //    one the compiler can see in flight, its wait counting turns every LDS
 //    fragment wait into lgkmcnt(0) instead of the partial count the
 //    in-order reads allow. K slots are chunk-major in 16-row groups and V_t
 //    slots hold whole MFMA fragments in lane order, so every operand read is
-//    a conflict-free ds_read_b128.
+//    a conflict-free ds_read_b128; V slots hold rows, read by transposing reads.
 //  * Online softmax in base 2 with the running max kept on the integer grid:
 //    m = ceil(max(s) * log2(e)/sqrt(128)). Every rescale is an exact power of
 //    two, so the bf16 rounding of P (done with the output round mode, as in
@@ -110,7 +110,8 @@ struct ShortCtx {
 struct Params {
   const uint16_t* q;
   const uint16_t* k;
-  const uint16_t* vt;
+  const uint16_t* vt;  // V_t, or null: V itself is read (v)
+  const uint16_t* v;
   uint16_t* out;
   float* ws;         // split partials (null unless split)
   int B, H, Sq, Skv;
@@ -222,7 +223,12 @@ __device__ __forceinline__ void lite_emit(const Params& p, long long row, int n,
 // bf16(P) under the final max times an exact power of two (up to the last
 // fp32 bit of the exp2 argument): the output does not depend on where the
 // rebases happen, on the KV blocking or on the split.
-template <int MODE, bool LITE, bool SHORT = false>
+//
+// VROW: V is gathered in row order, as K is, and the V^T fragments come out of
+// two transposing reads (ds_read_b64_tr_b16) each instead of one ds_read_b128.
+// Those move half the bytes per clock, but no V_t pass precedes the launch (see
+// prefers_direct for both sides measured).
+template <int MODE, bool LITE, bool SHORT = false, bool VROW = false>
 __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb_begin, int kb_end, int part,
                                          char* lds, ShortCtx* sc = nullptr) {
   const int tid = threadIdx.x;
@@ -241,7 +247,8 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   const long long row_stride = p.bshd ? (long long)p.H * kD : kD;
   const uint16_t* qh = p.q + head_base(b, h, p.Sq, p.H, p.bshd);
   const char* kh = reinterpret_cast<const char*>(p.k + head_base(b, h, p.Skv, p.H, p.bshd));
-  const char* vth = reinterpret_cast<const char*>(p.vt + (long long)bh * p.nkb * kVtBlockElems);
+  const char* vth = VROW ? reinterpret_cast<const char*>(p.v + head_base(b, h, p.Skv, p.H, p.bshd))
+                         : reinterpret_cast<const char*>(p.vt + (long long)bh * p.nkb * kVtBlockElems);
   const float c = p.scale_log2e;
   const int kv_end = p.Skv < kb_end * kKvBlock ? p.Skv : kb_end * kKvBlock;
 
@@ -269,6 +276,14 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
 #pragma unroll
   for (int i = 0; i < 2; ++i) koff[i] = (uint32_t)(kdma_row(i) * row_stride * 2) + (uint32_t)(kdma_chunk(i) * 16);
   const long long kblk_bytes = (long long)kKvBlock * row_stride * 2;
+  // Instruction i of the last partial block: rows past Skv are clamped (they are
+  // masked in softmax).
+  auto issue_k_clamped = [&](int kb, int slot, int i) {
+    int kv = kb * kKvBlock + kdma_row(i);
+    kv = kv < p.Skv ? kv : p.Skv - 1;
+    dma16_opaque(kh + (long long)kv * row_stride * 2 + kdma_chunk(i) * 16,
+                 kring + slot * kKBytes + (wave * 2 + i) * kFragBytes);
+  };
   auto issue_k = [&](int kb, int slot) {
     char* st = kring + slot * kKBytes;
     if ((kb + 1) * kKvBlock <= p.Skv) {
@@ -276,22 +291,48 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
 #pragma unroll
       for (int i = 0; i < 2; ++i) dma16_sbase(base, koff[i], st + (wave * 2 + i) * kFragBytes);
     } else {
-      // Last partial block: clamp rows past Skv (they are masked in softmax).
+#pragma unroll
+      for (int i = 0; i < 2; ++i) issue_k_clamped(kb, slot, i);
+    }
+  };
+  // V_t: 1 KB fragments as they are. VROW: instruction j = 2 wave + i moves rows
+  // 4j .. 4j+3 (lane l: row 4j + l/16, 16-byte slot l % 16), row rr's chunk c at
+  // slot c ^ 4 (rr % 4): the four rows of a transposing read hit distinct banks.
+  auto vdma_row = [&](int i) { return 4 * (wave * 2 + i) + (lane >> 4); };
+  uint32_t voff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    voff[i] = VROW ? (uint32_t)(vdma_row(i) * row_stride * 2) + (uint32_t)(16 * ((lane & 15) ^ (4 * (vdma_row(i) & 3))))
+                   : (uint32_t)((wave * 2 + i) * kFragBytes + lane * 16);
+  const long long vblk_bytes = VROW ? kblk_bytes : (long long)kVBytes;
+  auto issue_v = [&](int kb, int slot) {
+    char* st = vring + slot * kVBytes;
+    const char* base = vth + kb * vblk_bytes;
+    if (!VROW || (kb + 1) * kKvBlock <= p.Skv) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dma16_sbase(base, voff[i], st + (wave * 2 + i) * kFragBytes);
+    } else {
+      // Last partial block: rows past Skv are zero (p = 0 there, and 0 x inf is
+      // not), written by the lanes that would have fetched them. The block waits
+      // count instructions, so an instruction without any valid row is replaced
+      // by a repeat of this wave's K one.
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        int kv = kb * kKvBlock + kdma_row(i);
-        kv = kv < p.Skv ? kv : p.Skv - 1;
-        dma16_opaque(kh + (long long)kv * row_stride * 2 + kdma_chunk(i) * 16, st + (wave * 2 + i) * kFragBytes);
+        char* dst = st + (wave * 2 + i) * kFragBytes;
+        const bool valid = kb * kKvBlock + vdma_row(i) < p.Skv;
+        if (__builtin_amdgcn_ballot_w64(valid) == 0) issue_k_clamped(kb, slot, i);
+        if (valid) {
+          dma16_opaque(base + voff[i], dst);
+        } else {
+          *reinterpret_cast<u32x4*>(dst + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+        }
       }
     }
   };
-  const uint32_t voff = (uint32_t)(wave * 2 * kFragBytes + lane * 16);
-  auto issue_v = [&](int kb, int slot) {
-    char* st = vring + slot * kVBytes;
-    const char* base = vth + (long long)kb * kVBytes;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_sbase(base, voff + i * kFragBytes, st + (wave * 2 + i) * kFragBytes);
-  };
+  // VROW fragment reads: this lane's 8 bytes of row 4g + m/4 (m = lane % 16) of a
+  // 16-row k-step, d-tile dt at vfrag_lane ^ 64 dt.
+  const int vm = lane & 15;
+  const int vfrag_lane = (4 * g + (vm >> 2)) * 256 + 64 * (vm >> 2) + 32 * ((lane >> 4) & 1) + 8 * (vm & 3);
 
   // ---- Q fragments (B operand of S^T = K Q^T), kept in registers --------------
   bf16x8 qf[8];
@@ -514,6 +555,7 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       const bool prefetch = sc->next_bh >= 0;
       if (prefetch) issue_q_stage(sc->next_bh, sc->next_qb);
       if (kv_new) {
+        if constexpr (VROW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // zeroed rows
         if (prefetch) {
           wait_vmem_barrier<8>();
         } else {
@@ -573,13 +615,13 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       if (dma3 && !dma3_full) issue_kv(kb3, (i + 3) % kRing);
       const int pd3 = __builtin_amdgcn_readfirstlane((int)dma3_full);
       const char* kbase3 = kh + (long long)kb3 * kblk_bytes;
-      const char* vbase3 = vth + (long long)kb3 * kVBytes;
+      const char* vbase3 = vth + (long long)kb3 * vblk_bytes;
       const char* kst3 = kring + ((i + 3) % kRing) * kKBytes;
       const char* vst3 = vring + ((i + 3) % kRing) * kVBytes;
       auto dma3_step = [&](int d) {  // d = 0, 1: K instructions; 2, 3: V instructions
         // Global address = SGPR base + 32-bit lane offset (no 64-bit VALU add).
         const char* base = d < 2 ? kbase3 : vbase3;
-        const uint32_t off = d < 2 ? koff[d] : voff + (uint32_t)((d - 2) * kFragBytes);
+        const uint32_t off = d < 2 ? koff[d] : voff[d - 2];
         const char* dst = d < 2 ? kst3 + (wave * 2 + d) * kFragBytes : vst3 + (wave * 2 + d - 2) * kFragBytes;
         const uint32_t m0v = (uint32_t)(uintptr_t)(MM_LDS const char*)dst;
         asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 1f\n\tglobal_load_lds_dwordx4 %0, %1\n1:" ::"v"(off),
@@ -654,7 +696,16 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       // V^T fragments in a 4-deep rolling buffer, 4 MFMAs ahead: PV MFMA n (0..15)
       // = row tile n/8, k-step (n/4)%2, d-tile n%4.
       auto vfrag_n = [&](int nn) {
-        return *reinterpret_cast<const bf16x8*>(vst + (((nn >> 2) & 3) * 4 + (nn & 3)) * kFragBytes + lane * 16);
+        if constexpr (VROW) {
+          const char* a = vst + (vfrag_lane ^ (64 * (nn & 3))) + ((nn >> 2) & 3) * 4096;
+          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MM_LDS i16x4*)a);
+          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((MM_LDS i16x4*)(a + 2048));
+          const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
+          const u32x4 w = {lo2[0], lo2[1], hi2[0], hi2[1]};
+          return __builtin_bit_cast(bf16x8, w);
+        } else {
+          return *reinterpret_cast<const bf16x8*>(vst + (((nn >> 2) & 3) * 4 + (nn & 3)) * kFragBytes + lane * 16);
+        }
       };
       // Raised wave priority over the QK + softmax phase: the wave in this phase
       // wins issue slots over its SIMD partner when both are ready (measured
@@ -896,13 +947,13 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   }
 }
 
-template <int MODE>
+template <int MODE, bool VROW>
 __global__ __launch_bounds__(kThreads, 1) void attn_fwd_kernel(Params p) {
   __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
   const int idx = blockIdx.x;
   if (idx < p.prefix_wgs) {
     const int w = xcd_remap(idx, p.prefix_wgs);
-    run_tile<MODE, false>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds);
+    run_tile<MODE, false, false, VROW>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds);
   } else {
     // Split part: tail q-block t, part j of G, contiguous kv-block range.
     const int part = idx - p.prefix_wgs;
@@ -910,7 +961,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_fwd_kernel(Params p) {
     const int w = p.prefix_wgs + t;
     const int kb0 = (int)((long long)p.nkb * j / p.split_ways);
     const int kb1 = (int)((long long)p.nkb * (j + 1) / p.split_ways);
-    run_tile<MODE, false>(p, w / p.nqb, w % p.nqb, kb0, kb1, part, lds);
+    run_tile<MODE, false, false, VROW>(p, w / p.nqb, w % p.nqb, kb0, kb1, part, lds);
   }
 }
 
@@ -920,7 +971,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_fwd_kernel(Params p) {
 // an item computes, the next item's Q is gathered into the LDS stage and the
 // previous item's output stores drain, so the q-blocks' HBM traffic overlaps
 // the MFMA work instead of alternating with it in lockstep rounds.
-template <int MODE>
+template <int MODE, bool VROW>
 __global__ __launch_bounds__(kThreads, 1) void attn_short_kernel(Params p, int per_cta) {
   __shared__ __attribute__((aligned(1024))) char lds[kLdsShortBytes];
   const int total = p.nqb * p.B * p.H;
@@ -931,7 +982,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_short_kernel(Params p, int p
     const int wn = w + 1 < w1 ? w + 1 : -1;
     sc.next_bh = wn >= 0 ? wn / p.nqb : -1;
     sc.next_qb = wn >= 0 ? wn % p.nqb : 0;
-    run_tile<MODE, false, true>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds, &sc);
+    run_tile<MODE, false, true, VROW>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds, &sc);
     sc.first = false;
     ++sc.item;
   }
@@ -1259,19 +1310,20 @@ TailPlan plan_tail(int nqb, int nbh, int nkb, int slots, bool enable, int force_
   return TailPlan{wgs - tail, tail, G, tail * G};
 }
 
-template <int MODE>
-int launch_fwd(const void* q, const void* k, const void* v_t, void* out, int batch, int heads, int seq_len,
+// VROW: v_or_vt is V itself (moonmath_attention_forward_direct), else V_t.
+template <int MODE, bool VROW>
+int launch_fwd(const void* q, const void* k, const void* v_or_vt, void* out, int batch, int heads, int seq_len,
                int seq_len_kv, int head_dim, int layout, void* workspace, int force_ways, void* stream) {
   if (batch <= 0 || heads <= 0) return 1;
   if (seq_len <= 0) return 2;
   if (head_dim != kD) return 3;
   if (seq_len_kv <= 0) return 5;
   if (layout != 0 && layout != 1) return 7;
-  if (!q || !k || !v_t || !out) return 8;
+  if (!q || !k || !v_or_vt || !out) return 8;
   Params p{};
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
-  p.vt = static_cast<const uint16_t*>(v_t);
+  (VROW ? p.v : p.vt) = static_cast<const uint16_t*>(v_or_vt);
   p.out = static_cast<uint16_t*>(out);
   p.ws = static_cast<float*>(workspace);
   p.B = batch;
@@ -1291,7 +1343,7 @@ int launch_fwd(const void* q, const void* k, const void* v_t, void* out, int bat
     // planner's minimum).
     const int per_cta = (int)((items + kSlots - 1) / kSlots);
     const int grid = (int)((items + per_cta - 1) / per_cta);
-    hipLaunchKernelGGL((attn_short_kernel<MODE>), dim3(grid), dim3(kThreads), 0, st, p, per_cta);
+    hipLaunchKernelGGL((attn_short_kernel<MODE, VROW>), dim3(grid), dim3(kThreads), 0, st, p, per_cta);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
   }
@@ -1299,7 +1351,7 @@ int launch_fwd(const void* q, const void* k, const void* v_t, void* out, int bat
   p.prefix_wgs = tp.prefix_wgs;
   p.split_ways = tp.split_ways;
   const int grid = tp.prefix_wgs + tp.parts;
-  hipLaunchKernelGGL((attn_fwd_kernel<MODE>), dim3(grid), dim3(kThreads), 0, st, p);
+  hipLaunchKernelGGL((attn_fwd_kernel<MODE, VROW>), dim3(grid), dim3(kThreads), 0, st, p);
   if (tp.parts > 0) {
     const int per_qb = kRowsPerCta * kD / 4 / kMergeThreads;
     hipLaunchKernelGGL((attn_merge_kernel<MODE>), dim3(tp.tail * per_qb), dim3(kMergeThreads), 0, st, p,
@@ -1308,6 +1360,35 @@ int launch_fwd(const void* q, const void* k, const void* v_t, void* out, int bat
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
+
+template <bool VROW>
+int launch_mode(const void* q, const void* k, const void* v, void* out, int batch, int heads, int seq_len,
+                int seq_len_kv, int head_dim, int layout, int round_mode, void* workspace, int force_ways,
+                void* stream) {
+  switch (round_mode) {
+    case 0:
+      return launch_fwd<mm::kRTNE, VROW>(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
+                                         force_ways, stream);
+    case 1:
+      return launch_fwd<mm::kRTNA, VROW>(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
+                                         force_ways, stream);
+    case 2:
+      return launch_fwd<mm::kRTZ, VROW>(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
+                                        force_ways, stream);
+    default:
+      return 10;
+  }
+}
+
+// Whether a forward is faster on V itself than with a V_t pass before it. The
+// pass costs a launch and 4 bytes of traffic per element of V, the transposing
+// reads ~1.5% of a CTA's main loop, so the line depends on the q rows that share
+// a V. Measured (V_t pass + kernel -> direct, us): (1,2,256) 14.4 -> 12.0,
+// (1,24,1531) 47.3 -> 39.5, (2,24,8192) x 77 55.3 -> 49.8, (2,24,4097) x 512 71.2
+// -> 66.8, (2,24,4096) 349 -> 337, (2,24,8192) 1412 -> 1399; (1,32,16384) 3628 ->
+// 3636, (2,24,16384) x 2048 748 -> 756, (2,8,32768) x 4096 929 -> 941.
+constexpr int kDirectMaxSq = 12288;
+bool prefers_direct(int seq_len) { return seq_len <= kDirectMaxSq; }
 
 // LiteAttention launcher (reference launch_attention_forward_lite,
 // attention_kernel.hip:1599-1681). workspace: lite_workspace_bytes bytes for
@@ -1390,8 +1471,8 @@ extern "C" {
   int launch_attention_forward_##NAME(const void* q, const void* k, const void* v_t, void* out, int batch,   \
                                       int heads, int seq_len, int seq_len_kv, int head_dim, int layout,      \
                                       void* workspace, void* stream) {                                       \
-    return launch_fwd<MODE>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace, \
-                            0, stream);                                                                      \
+    return launch_fwd<MODE, false>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout,      \
+                                   workspace, 0, stream);                                                    \
   }                                                                                                          \
   size_t tail_workspace_bytes_##NAME(void) { return kWorkspaceBytes; }                                     \
   int launch_attention_forward_lite_##NAME(const void* q, const void* k, const void* v_t, void* out, int batch, \
@@ -1414,19 +1495,19 @@ MM_ATTN_MODE_SYMBOLS(rtz, mm::kRTZ)
 int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t, void* out, int batch, int heads,
                                   int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
                                   void* workspace, int force_split_ways, void* stream) {
-  switch (round_mode) {
-    case 0:
-      return launch_fwd<mm::kRTNE>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
-                                   force_split_ways, stream);
-    case 1:
-      return launch_fwd<mm::kRTNA>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
-                                   force_split_ways, stream);
-    case 2:
-      return launch_fwd<mm::kRTZ>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, workspace,
-                                  force_split_ways, stream);
-    default:
-      return 10;
-  }
+  return launch_mode<false>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, round_mode, workspace,
+                            force_split_ways, stream);
+}
+
+int moonmath_attention_forward_direct(const void* q, const void* k, const void* v, void* out, int batch, int heads,
+                                      int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
+                                      void* workspace, int force_split_ways, void* stream) {
+  return launch_mode<true>(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, round_mode, workspace,
+                           force_split_ways, stream);
+}
+
+int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv) {
+  return batch > 0 && heads > 0 && seq_len > 0 && seq_len_kv > 0 && prefers_direct(seq_len);
 }
 
 int moonmath_attention_plan_tail(int batch, int heads, int seq_len, int seq_len_kv, int enable, int force_split_ways,

@@ -36,6 +36,8 @@ struct Abi {
 #define MM_ABI(X)                                                                                          \
   X(launch_v_transpose_rtne)                                                                               \
   X(moonmath_attention_forward_ex)                                                                         \
+  X(moonmath_attention_forward_direct)                                                                     \
+  X(moonmath_attention_prefers_direct)                                                                     \
   X(moonmath_attention_plan_tail)                                                                          \
   X(moonmath_attention_vt_bytes)                                                                           \
   X(tail_workspace_bytes_rtne)                                                                             \
@@ -196,17 +198,20 @@ PyObject* forward(PyObject*, PyObject* const* x, Py_ssize_t n) {
       const c10::DeviceGuard guard(a.q.device());
       if (!a.own_out) a.out = at::empty_like(a.q);
       void* stream = stream_of(a.q);
-      const Tensor vt = bytes(abi.moonmath_attention_vt_bytes(a.B, a.H, a.Skv), a.q);
-      Tensor ws;
+      Tensor vt, ws;
       int plan[4];
       check_rc(abi.moonmath_attention_plan_tail(a.B, a.H, a.Sq, a.Skv, 1, 0, plan), "moonmath_attention_plan_tail");
       if (plan[3] > 0) ws = bytes(abi.tail_workspace_bytes_rtne(), a.q);
-      check_rc(abi.launch_v_transpose_rtne(a.v.data_ptr(), vt.data_ptr(), a.B * a.H * a.Skv, a.Skv, a.H, a.layout,
-                                           stream),
-               "launch_v_transpose");
-      check_rc(abi.moonmath_attention_forward_ex(a.q.data_ptr(), a.k.data_ptr(), vt.data_ptr(), a.out.data_ptr(), a.B,
-                                                 a.H, a.Sq, a.Skv, 128, a.layout, a.mode,
-                                                 ws.defined() ? ws.data_ptr() : nullptr, 0, stream),
+      const bool direct = abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
+      if (!direct) {
+        vt = bytes(abi.moonmath_attention_vt_bytes(a.B, a.H, a.Skv), a.q);
+        check_rc(abi.launch_v_transpose_rtne(a.v.data_ptr(), vt.data_ptr(), a.B * a.H * a.Skv, a.Skv, a.H, a.layout,
+                                             stream),
+                 "launch_v_transpose");
+      }
+      check_rc((direct ? abi.moonmath_attention_forward_direct : abi.moonmath_attention_forward_ex)(
+                   a.q.data_ptr(), a.k.data_ptr(), direct ? a.v.data_ptr() : vt.data_ptr(), a.out.data_ptr(), a.B, a.H,
+                   a.Sq, a.Skv, 128, a.layout, a.mode, ws.defined() ? ws.data_ptr() : nullptr, 0, stream),
                "launch_attention_forward");
     }
     return attn_result(a, x[3]);

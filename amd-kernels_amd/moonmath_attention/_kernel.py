@@ -124,7 +124,6 @@ def _forward_device(q, k, v, out, round_mode, layout):
     lib = _lib.lib
     with torch.cuda.device(dev):
         stream = _lib.stream_ptr(dev)
-        vt = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=dev)
         # Tail KV-split workspace, allocated only when the planner splits.
         # MOONMATH_NO_TAIL disables the split (reference csrc/attention_api.cpp:258-267);
         # MOONMATH_FORCE_SPLIT=G forces G parts on the last round (test hook).
@@ -135,13 +134,17 @@ def _forward_device(q, k, v, out, round_mode, layout):
             plan = _lib.plan_tail(B, H, Sq, Skv, True, force)
             if plan[3] > 0:
                 ws = torch.empty(lib.tail_workspace_bytes_rtne(), dtype=torch.uint8, device=dev)
-        rc = getattr(lib, f"launch_v_transpose_{round_mode}")(
-            _lib.ptr(v), _lib.ptr(vt), B * H * Skv, Skv, H, lay, stream
-        )
-        if rc != 0:
-            raise RuntimeError(f"launch_v_transpose returned error code {rc}")
-        rc = lib.moonmath_attention_forward_ex(
-            _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out), B, H, Sq, Skv, 128, lay,
+        src, fn = v, lib.moonmath_attention_forward_direct
+        if not lib.moonmath_attention_prefers_direct(B, H, Sq, Skv):
+            src = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=dev)
+            rc = getattr(lib, f"launch_v_transpose_{round_mode}")(
+                _lib.ptr(v), _lib.ptr(src), B * H * Skv, Skv, H, lay, stream
+            )
+            if rc != 0:
+                raise RuntimeError(f"launch_v_transpose returned error code {rc}")
+            fn = lib.moonmath_attention_forward_ex
+        rc = fn(
+            _lib.ptr(q), _lib.ptr(k), _lib.ptr(src), _lib.ptr(out), B, H, Sq, Skv, 128, lay,
             _MODES[round_mode], _lib.ptr(ws), force, stream,
         )
         if rc != 0:

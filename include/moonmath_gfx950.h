@@ -101,6 +101,14 @@ int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t,
                                   int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
                                   void* workspace, int force_split_ways, void* stream);
 
+/* The same forward on V itself ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit
+ * for bit. moonmath_attention_prefers_direct: 1 where that is the faster one
+ * (a V_t pass costs more than the transposing reads). */
+int moonmath_attention_forward_direct(const void* q, const void* k, const void* v, void* out, int batch, int heads,
+                                      int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
+                                      void* workspace, int force_split_ways, void* stream);
+int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv);
+
 /* Tail split plan -> out4 = {prefix CTAs, tail, split ways G, parts}. Pure host.
  * Replaces plan_tail_split, csrc/attention_kernel.hip:1349-1393. */
 int moonmath_attention_plan_tail(int batch, int heads, int seq_len, int seq_len_kv, int enable, int force_split_ways,

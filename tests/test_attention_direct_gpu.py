@@ -1,0 +1,52 @@
+"""The forward on V itself (transposing LDS reads) against the forward on V_t:
+the same operands in the same order, so bit-identical, at the edges of its key
+blocks and rows, with non-finite values in the last rows of V (rows past the
+end of the keys must add nothing)."""
+import ctypes
+
+import pytest
+import torch
+
+from moonmath_attention import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _run(name, q, k, v, B, H, Sq, Skv, layout, mode, force):
+    lib, p, st = _lib.lib, _lib.ptr, _lib.stream_ptr(DEV)
+    out = torch.full_like(q, float("nan"))
+    ws = torch.empty(lib.tail_workspace_bytes_rtne(), dtype=torch.uint8, device=DEV) if force else None
+    src = v
+    if name == "moonmath_attention_forward_ex":
+        src = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=DEV)
+        assert lib.launch_v_transpose_rtne(p(v), p(src), B * H * Skv, Skv, H, layout, st) == 0
+    assert getattr(lib, name)(p(q), p(k), p(src), p(out), B, H, Sq, Skv, 128, layout, mode, p(ws), force, st) == 0
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("B,H,Sq,Skv,force", [
+    (1, 2, 256, 256, 0), (2, 3, 300, 1, 0), (1, 2, 33, 61, 0), (1, 3, 200, 65, 0), (1, 2, 257, 125, 0),
+    (1, 2, 100, 193, 0), (2, 2, 520, 3000, 0), (1, 1, 64, 8191, 0),
+    (1, 3, 21800, 77, 0), (2, 24, 4097, 1, 0), (2, 24, 4097, 128, 0),   # persistent short-KV kernel
+    (1, 4, 1100, 1409, 3)])                                              # split parts
+def test_direct_equals_vt(B, H, Sq, Skv, force, layout):
+    g = torch.Generator(device=DEV).manual_seed(Sq + Skv)
+    shape = (lambda s: (B, s, H, 128)) if layout else (lambda s: (B, H, s, 128))
+    q, k, v = (torch.randn(shape(s), generator=g, device=DEV).bfloat16() for s in (Sq, Skv, Skv))
+    last = (v.transpose(1, 2) if layout else v)[0, 0, Skv - 1]
+    last[3], last[7], last[11] = float("inf"), float("nan"), float("-inf")
+    for mode in range(3):
+        a = _run("moonmath_attention_forward_ex", q, k, v, B, H, Sq, Skv, layout, mode, force)
+        b = _run("moonmath_attention_forward_direct", q, k, v, B, H, Sq, Skv, layout, mode, force)
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), mode
+
+
+def test_direct_argument_codes():
+    nul = ctypes.c_void_p(0)
+    f = _lib.lib.moonmath_attention_forward_direct
+    assert f(nul, nul, nul, nul, 0, 1, 1, 1, 128, 0, 0, nul, 0, nul) == 1
+    assert f(nul, nul, nul, nul, 1, 1, 1, 1, 128, 0, 0, nul, 0, nul) == 8
+    assert f(nul, nul, nul, nul, 1, 1, 1, 1, 128, 0, 9, nul, 0, nul) == 10
