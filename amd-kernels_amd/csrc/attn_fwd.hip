@@ -1011,13 +1011,13 @@ __device__ __forceinline__ int lpt_position(int s, int total) {
 // LiteAttention forward: one CTA per (b, h, q-block); grid slot s runs CTA
 // order[lpt_position(s)] (LPT order) or, without an order, the XCD-grouped
 // dense mapping.
-template <int MODE>
+template <int MODE, bool VROW>
 __global__ __launch_bounds__(kThreads, 1) void attn_lite_kernel(Params p) {
   __shared__ __attribute__((aligned(1024))) char lds[kLdsLiteBytes];
   const int total = p.nqb * p.B * p.H;
   const int w = p.order ? p.order[lpt_position(blockIdx.x, total)] : xcd_remap(blockIdx.x, total);
   if (w < 0 || w >= total) return;
-  run_tile<MODE, true>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds);
+  run_tile<MODE, true, false, VROW>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1397,8 +1397,8 @@ bool prefers_direct(int seq_len) { return seq_len <= kDirectMaxSq; }
 // reference).
 constexpr int kLiteMinKvBlocksForLpt = 48;
 
-template <int MODE>
-int launch_lite(const void* q, const void* k, const void* v_t, void* out, int batch, int heads, int seq_len,
+template <int MODE, bool VROW>
+int launch_lite(const void* q, const void* k, const void* v_or_vt, void* out, int batch, int heads, int seq_len,
                 int seq_len_kv, int head_dim, const void* read_list, void* write_list, const void* must_do,
                 float threshold, int phase, int layout, void* workspace, void* stream) {
   if (batch <= 0 || heads <= 0) return 1;
@@ -1407,11 +1407,11 @@ int launch_lite(const void* q, const void* k, const void* v_t, void* out, int ba
   if (!read_list || !write_list) return 4;
   if (seq_len_kv <= 0) return 5;
   if (layout != 0 && layout != 1) return 7;
-  if (!q || !k || !v_t || !out) return 8;
+  if (!q || !k || !v_or_vt || !out) return 8;
   Params p{};
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
-  p.vt = static_cast<const uint16_t*>(v_t);
+  (VROW ? p.v : p.vt) = static_cast<const uint16_t*>(v_or_vt);
   p.out = static_cast<uint16_t*>(out);
   p.B = batch;
   p.H = heads;
@@ -1438,7 +1438,7 @@ int launch_lite(const void* q, const void* k, const void* v_t, void* out, int ba
     hipLaunchKernelGGL(lite_order_kernel, dim3(1), dim3(kLptThreads), 0, st, bucket, static_cast<int*>(workspace),
                        (int)total);
   }
-  hipLaunchKernelGGL((attn_lite_kernel<MODE>), dim3((unsigned)total), dim3(kThreads), 0, st, p);
+  hipLaunchKernelGGL((attn_lite_kernel<MODE, VROW>), dim3((unsigned)total), dim3(kThreads), 0, st, p);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
@@ -1480,8 +1480,8 @@ extern "C" {
                                            const void* read_list, void* write_list, const void* must_do_list, \
                                            float threshold, int phase, int layout, void* workspace,           \
                                            void* stream) {                                                    \
-    return launch_lite<MODE>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, read_list,          \
-                             write_list, must_do_list, threshold, phase, layout, workspace, stream);          \
+    return launch_lite<MODE, false>(q, k, v_t, out, batch, heads, seq_len, seq_len_kv, head_dim, read_list,   \
+                                    write_list, must_do_list, threshold, phase, layout, workspace, stream);   \
   }                                                                                                          \
   size_t lite_workspace_bytes_##NAME(int batch, int heads, int seq_len) {                                    \
     if (batch <= 0 || heads <= 0 || seq_len <= 0) return 0;                                                  \
@@ -1504,6 +1504,20 @@ int moonmath_attention_forward_direct(const void* q, const void* k, const void* 
                                       void* workspace, int force_split_ways, void* stream) {
   return launch_mode<true>(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, layout, round_mode, workspace,
                            force_split_ways, stream);
+}
+
+int moonmath_attention_forward_lite_direct(const void* q, const void* k, const void* v, void* out, int batch,
+                                           int heads, int seq_len, int seq_len_kv, int head_dim,
+                                           const void* read_list, void* write_list, const void* must_do_list,
+                                           float threshold, int phase, int layout, int round_mode, void* workspace,
+                                           void* stream) {
+  const auto launch = round_mode == 0   ? launch_lite<mm::kRTNE, true>
+                      : round_mode == 1 ? launch_lite<mm::kRTNA, true>
+                      : round_mode == 2 ? launch_lite<mm::kRTZ, true>
+                                        : nullptr;
+  if (!launch) return 10;
+  return launch(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, read_list, write_list, must_do_list,
+                threshold, phase, layout, workspace, stream);
 }
 
 int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv) {

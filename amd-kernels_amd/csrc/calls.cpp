@@ -37,6 +37,7 @@ struct Abi {
   X(launch_v_transpose_rtne)                                                                               \
   X(moonmath_attention_forward_ex)                                                                         \
   X(moonmath_attention_forward_direct)                                                                     \
+  X(moonmath_attention_forward_lite_direct)                                                                \
   X(moonmath_attention_prefers_direct)                                                                     \
   X(moonmath_attention_plan_tail)                                                                          \
   X(moonmath_attention_vt_bytes)                                                                           \
@@ -236,17 +237,25 @@ PyObject* forward_lite(PyObject*, PyObject* const* x, Py_ssize_t n) {
       const c10::DeviceGuard guard(a.q.device());
       if (!a.own_out) a.out = at::empty_like(a.q);
       void* stream = stream_of(a.q);
-      const Tensor vt = bytes(abi.moonmath_attention_vt_bytes(a.B, a.H, a.Skv), a.q);
       const Tensor ws = bytes(abi.lite_workspace_bytes_rtne(a.B, a.H, a.Sq), a.q);
-      check_rc(abi.launch_v_transpose_rtne(a.v.data_ptr(), vt.data_ptr(), a.B * a.H * a.Skv, a.Skv, a.H, a.layout,
-                                           stream),
-               "launch_v_transpose");
-      const auto launch = a.mode == 0   ? abi.launch_attention_forward_lite_rtne
-                          : a.mode == 1 ? abi.launch_attention_forward_lite_rtna
-                                        : abi.launch_attention_forward_lite_rtz;
-      check_rc(launch(a.q.data_ptr(), a.k.data_ptr(), vt.data_ptr(), a.out.data_ptr(), a.B, a.H, a.Sq, a.Skv, 128,
-                      read.data_ptr(), write.data_ptr(), nullptr, threshold, phase, a.layout, ws.data_ptr(), stream),
-               "launch_attention_forward_lite");
+      if (abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv)) {
+        check_rc(abi.moonmath_attention_forward_lite_direct(
+                     a.q.data_ptr(), a.k.data_ptr(), a.v.data_ptr(), a.out.data_ptr(), a.B, a.H, a.Sq, a.Skv, 128,
+                     read.data_ptr(), write.data_ptr(), nullptr, threshold, phase, a.layout, a.mode, ws.data_ptr(),
+                     stream),
+                 "launch_attention_forward_lite");
+      } else {
+        const Tensor vt = bytes(abi.moonmath_attention_vt_bytes(a.B, a.H, a.Skv), a.q);
+        check_rc(abi.launch_v_transpose_rtne(a.v.data_ptr(), vt.data_ptr(), a.B * a.H * a.Skv, a.Skv, a.H, a.layout,
+                                             stream),
+                 "launch_v_transpose");
+        const auto launch = a.mode == 0   ? abi.launch_attention_forward_lite_rtne
+                            : a.mode == 1 ? abi.launch_attention_forward_lite_rtna
+                                          : abi.launch_attention_forward_lite_rtz;
+        check_rc(launch(a.q.data_ptr(), a.k.data_ptr(), vt.data_ptr(), a.out.data_ptr(), a.B, a.H, a.Sq, a.Skv, 128,
+                        read.data_ptr(), write.data_ptr(), nullptr, threshold, phase, a.layout, ws.data_ptr(), stream),
+                 "launch_attention_forward_lite");
+      }
     }
     return attn_result(a, x[7]);
   });

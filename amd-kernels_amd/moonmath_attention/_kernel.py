@@ -223,21 +223,26 @@ def forward_lite(
     lib = _lib.lib
     with torch.cuda.device(dev):
         stream = _lib.stream_ptr(dev)
-        vt = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=dev)
         ws = None
         if os.environ.get("MOONMATH_LITE_PLAIN") is None:
             ws = torch.empty(getattr(lib, f"lite_workspace_bytes_{round_mode}")(B, H, Sq), dtype=torch.uint8,
                              device=dev)
-        rc = getattr(lib, f"launch_v_transpose_{round_mode}")(
-            _lib.ptr(v), _lib.ptr(vt), B * H * Skv, Skv, H, lay, stream
-        )
-        if rc != 0:
-            raise RuntimeError(f"launch_v_transpose returned error code {rc}")
-        rc = getattr(lib, f"launch_attention_forward_lite_{round_mode}")(
-            _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out), B, H, Sq, Skv, 128,
-            _lib.ptr(read_list), _lib.ptr(write_list), _lib.ptr(must_do_list), float(threshold), int(phase), lay,
-            _lib.ptr(ws), stream,
-        )
+        lists = (_lib.ptr(read_list), _lib.ptr(write_list), _lib.ptr(must_do_list), float(threshold), int(phase), lay)
+        if lib.moonmath_attention_prefers_direct(B, H, Sq, Skv):
+            rc = lib.moonmath_attention_forward_lite_direct(
+                _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), B, H, Sq, Skv, 128, *lists, _MODES[round_mode],
+                _lib.ptr(ws), stream,
+            )
+        else:
+            vt = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=dev)
+            rc = getattr(lib, f"launch_v_transpose_{round_mode}")(
+                _lib.ptr(v), _lib.ptr(vt), B * H * Skv, Skv, H, lay, stream
+            )
+            if rc != 0:
+                raise RuntimeError(f"launch_v_transpose returned error code {rc}")
+            rc = getattr(lib, f"launch_attention_forward_lite_{round_mode}")(
+                _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out), B, H, Sq, Skv, 128, *lists, _lib.ptr(ws), stream,
+            )
         if rc != 0:
             raise RuntimeError(f"launch_attention_forward_lite returned error code {rc}")
     return out

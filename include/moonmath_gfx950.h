@@ -101,12 +101,18 @@ int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t,
                                   int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
                                   void* workspace, int force_split_ways, void* stream);
 
-/* The same forward on V itself ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit
- * for bit. moonmath_attention_prefers_direct: 1 where that is the faster one
- * (a V_t pass costs more than the transposing reads). */
+/* The same forward, and the same LiteAttention forward, on V itself
+ * ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit for bit.
+ * moonmath_attention_prefers_direct: 1 where that is the faster one (a V_t pass
+ * costs more than the transposing reads). */
 int moonmath_attention_forward_direct(const void* q, const void* k, const void* v, void* out, int batch, int heads,
                                       int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
                                       void* workspace, int force_split_ways, void* stream);
+int moonmath_attention_forward_lite_direct(const void* q, const void* k, const void* v, void* out, int batch,
+                                           int heads, int seq_len, int seq_len_kv, int head_dim,
+                                           const void* read_list, void* write_list, const void* must_do_list,
+                                           float threshold, int phase, int layout, int round_mode, void* workspace,
+                                           void* stream);
 int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv);
 
 /* Tail split plan -> out4 = {prefix CTAs, tail, split ways G, parts}. Pure host.

@@ -44,6 +44,40 @@ def test_direct_equals_vt(B, H, Sq, Skv, force, layout):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), mode
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("B,H,Sq,Skv", [(1, 2, 300, 1000), (2, 3, 700, 8190), (1, 2, 256, 64), (1, 1, 50, 3)])
+def test_lite_direct_equals_vt(B, H, Sq, Skv, layout):
+    """Three steps from the full list on keys of growing norm (blocks drop out):
+    outputs and written lists."""
+    lib, p, st = _lib.lib, _lib.ptr, _lib.stream_ptr(DEV)
+    g = torch.Generator(device=DEV).manual_seed(Sq + Skv)
+    shape = (lambda s: (B, s, H, 128)) if layout else (lambda s: (B, H, s, 128))
+    q, k, v = (torch.randn(shape(s), generator=g, device=DEV) for s in (Sq, Skv, Skv))
+    ramp = torch.linspace(0.2, 3.0, Skv, device=DEV)
+    k = k * (ramp.view(1, Skv, 1, 1) if layout else ramp.view(1, 1, Skv, 1))
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    nqb, nkb = -(-Sq // 256), -(-Skv // 64)
+    vt = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=DEV)
+    assert lib.launch_v_transpose_rtne(p(v), p(vt), B * H * Skv, Skv, H, layout, st) == 0
+    for mode, name in enumerate(("rtne", "rtna", "rtz")):
+        got = []
+        for direct in (False, True):
+            pair = torch.zeros(2, B, H, nqb, nkb + 2, dtype=torch.int16, device=DEV)
+            pair[0, ..., :3] = torch.tensor([2, nkb - 1, -1], dtype=torch.int16)
+            for step in range(3):
+                out = torch.full_like(q, float("nan"))
+                ws = torch.empty(lib.lite_workspace_bytes_rtne(B, H, Sq), dtype=torch.uint8, device=DEV)
+                head = (p(q), p(k), p(v if direct else vt), p(out), B, H, Sq, Skv, 128, p(pair[step & 1]),
+                        p(pair[1 - (step & 1)]), None, -3.0, 1 - (step & 1), layout)
+                rc = (lib.moonmath_attention_forward_lite_direct(*head, mode, p(ws), st) if direct else
+                      getattr(lib, f"launch_attention_forward_lite_{name}")(*head, p(ws), st))
+                assert rc == 0
+                torch.cuda.synchronize()
+                got.append((out.clone(), pair.clone()))
+        for (a, x), (b, y) in zip(got[:3], got[3:], strict=True):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and torch.equal(x, y)
+
+
 def test_direct_argument_codes():
     nul = ctypes.c_void_p(0)
     f = _lib.lib.moonmath_attention_forward_direct
