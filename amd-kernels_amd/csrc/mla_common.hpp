@@ -46,6 +46,7 @@ struct Params {
   int max_blocks, num_blocks;
   int B, H, q_len, S_fixed, parts, ngroups, paged;
   int unit_cap;           // units one round of CTAs over the CUs holds
+  int min_chunk;          // tokens of the shortest part (equal parts)
   int workers;            // > 0: balanced split over this many units (see plan_work), 0: equal parts
   int qrows;              // H * q_len
   int rec_rows;           // O rows per split record (>= qrows)
@@ -103,12 +104,11 @@ __device__ __forceinline__ uint32_t u16_field(uint32_t w, int k) {
 // units (request parts). Every request is cut into chunks of C tokens, request
 // b getting nparts_b = max(1, ceil(L_b / C)) parts of equal size (rounded up to
 // a tile; the last part takes the remainder), with C the smallest multiple of
-// the tile, at least 512, for which sum_b nparts_b <= U -- found by bisection,
+// the tile, at least min_chunk, for which sum_b nparts_b <= U -- found by bisection,
 // since the count only falls as C grows and C = max_b L_b gives B units. So the
 // partial records always fit the B * P * qrows workspace, one round of CTAs
 // covers the batch, and the longest part (the CTA that ends last) is as short
 // as the budget allows.
-constexpr int kMinChunk = 512;
 // The paged plan keeps three B-entry tables (12 * B bytes) in LDS scratch.
 constexpr int kMaxPagedB = 3072;  // 12 B per request: 36 KB of plan scratch
 
@@ -127,24 +127,24 @@ __device__ __forceinline__ int unit_budget(int B, int P, int cap) {
   const long long m = bp < cap ? bp : cap;
   return (int)(m > B ? m : B);
 }
-// Smallest chunk C (a multiple of 32, >= kMinChunk) with units(C) <= budget,
+// Smallest chunk C (a multiple of the tile, >= min_chunk) with units(C) <= budget,
 // for a units(C) that is non-increasing in C with units(max L) = B <= budget.
 // Wave-uniform.
 template <class UnitsFn>
-__device__ int search_chunk(long long sumL, int maxL, int B, int budget, UnitsFn units) {
-  int hi = maxL < kMinChunk ? kMinChunk : ((maxL + kTileTok - 1) & ~(kTileTok - 1));
+__device__ int search_chunk(long long sumL, int maxL, int B, int budget, int min_chunk, UnitsFn units) {
+  int hi = maxL < min_chunk ? min_chunk : ((maxL + kTileTok - 1) & ~(kTileTok - 1));
   if (budget <= B) return hi;  // one part per request
   // ceil(L / C) < L / C + 1, so C >= sumL / (budget - B) is feasible too.
   auto ceil_div_ll = [](long long a, int d) -> long long {  // 32-bit division whenever it suffices
     return a < 0x7FFFFFFF ? (long long)ceil_div_u((int)a, d) : (a + d - 1) / d;
   };
   const long long ok = ceil_div_ll(sumL, budget - B);
-  if (ok < hi) hi = ok < kMinChunk ? kMinChunk : (int)((ok + kTileTok - 1) & ~(long long)(kTileTok - 1));
+  if (ok < hi) hi = ok < min_chunk ? min_chunk : (int)((ok + kTileTok - 1) & ~(long long)(kTileTok - 1));
   // units(C) >= sumL / C, so C >= sumL / budget.
   const long long need = ceil_div_ll(sumL, budget);
   int lo = need > hi ? hi : (int)need;
   lo = (lo + kTileTok - 1) & ~(kTileTok - 1);
-  lo = lo < kMinChunk ? kMinChunk : (lo > hi ? hi : lo);
+  lo = lo < min_chunk ? min_chunk : (lo > hi ? hi : lo);
   while (lo < hi) {
     const int mid = lo + ((hi - lo) / (2 * kTileTok)) * kTileTok;
     if (units(mid) <= budget) {
@@ -205,7 +205,7 @@ __device__ Unit plan_unit_paged(const Params& p, int u, int lane, int* scratch) 
   }
   auto len_at = [&](int c0) { return c0 == 0 ? l0 : ((c0 + lane < B) ? lens[c0 + lane] : 0); };
   const int budget = unit_budget(B, P, cap);
-  const int C = search_chunk(suml, maxl, B, budget, [&](int c) {
+  const int C = search_chunk(suml, maxl, B, budget, p.min_chunk, [&](int c) {
     int n = 0;
     for (int c0 = 0; c0 < B; c0 += 64) n += wave_sum_i(c0 + lane < B ? nparts_of(len_at(c0), c) : 0);
     return n;
@@ -323,9 +323,9 @@ __device__ Unit plan_unit_paged(const Params& p, int u, int lane, int* scratch) 
 
 // Unit `u` of a contiguous batch (every request S tokens): the same chunking,
 // units in request order.
-__device__ __forceinline__ Unit plan_unit_contig(int S, int B, int P, int cap, int u) {
+__device__ __forceinline__ Unit plan_unit_contig(int S, int B, int P, int cap, int min_chunk, int u) {
   const int C =
-      search_chunk((long long)B * S, S, B, unit_budget(B, P, cap), [&](int c) { return B * nparts_of(S, c); });
+      search_chunk((long long)B * S, S, B, unit_budget(B, P, cap), min_chunk, [&](int c) { return B * nparts_of(S, c); });
   const int np = nparts_of(S, C);
   return Unit{u / np, u % np, np, (u / np) * np, part_tokens(S, np), B * np, S, 0};
 }
@@ -375,7 +375,7 @@ template <bool PAGED>
 __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
   if (p.workers == 0) {
     const Unit un = PAGED ? plan_unit_paged(p, u, lane, scratch)
-                          : plan_unit_contig(p.S_fixed, p.B, p.parts, p.unit_cap, u);
+                          : plan_unit_contig(p.S_fixed, p.B, p.parts, p.unit_cap, p.min_chunk, u);
     const long long lo = (long long)un.part * un.ptok;
     const int kv_lo = lo < un.len ? (int)lo : un.len;
     const int kv_hi = lo + un.ptok < un.len ? (int)(lo + un.ptok) : un.len;

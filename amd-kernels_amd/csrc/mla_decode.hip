@@ -27,90 +27,51 @@
 namespace mm {
 namespace mla {
 
-// Merge of NU 4-dim slices of one query row over its request's parts:
-// M = max_p m_p, w_p = 2^(m_p - M), out = sum w_p O_p * kv_scale / sum w_p l_p,
-// parts in order. o_at(j, u): part j's 16-byte O slice u; ml_at(j): part j's
-// (m, l) pair (shared by the slices: one row). The (m, l) pairs and O slices
-// of up to kBatch parts are loaded together, so a request of up to kBatch
-// parts costs one round of memory latency.
-template <int NU, class OAt, class MlAt>
-__device__ __forceinline__ void merge_slices(int nparts, float kv_scale, OAt o_at, MlAt ml_at, u32x2 (&out)[NU]) {
-  constexpr int kBatch = 8;
-  float M = -__builtin_inff();
-  f32x4 acc[NU];
-#pragma unroll
-  for (int u = 0; u < NU; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float L = 0.f;
-  float mb[kBatch], lb[kBatch];
-  f32x4 ob[kBatch][NU];
-  // Parts past the request's last are not loaded (uniform across the CTA: a
-  // CTA's cells belong to one request).
-  auto load_batch = [&](int j0) {
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      if (j0 + k < nparts) {
-        const float2 m_l = *reinterpret_cast<const float2*>(ml_at(j0 + k));
-        mb[k] = m_l.x;
-        lb[k] = m_l.y;
-#pragma unroll
-        for (int u = 0; u < NU; ++u) ob[k][u] = *reinterpret_cast<const f32x4*>(o_at(j0 + k, u));
-      } else {
-        mb[k] = -__builtin_inff();
-        lb[k] = 0.f;
-#pragma unroll
-        for (int u = 0; u < NU; ++u) ob[k][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  };
-  auto accumulate = [&](int j0) {
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      if (j0 + k < nparts) {
-        const float diff = mb[k] - M;  // integer-valued or -inf, <= 0
-        const float wt =
-            (mb[k] == -__builtin_inff()) ? 0.f : ((diff >= -126.f) ? __builtin_ldexpf(1.0f, (int)diff) : 0.f);
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          acc[u][0] = __builtin_fmaf(wt, ob[k][u][0], acc[u][0]);
-          acc[u][1] = __builtin_fmaf(wt, ob[k][u][1], acc[u][1]);
-          acc[u][2] = __builtin_fmaf(wt, ob[k][u][2], acc[u][2]);
-          acc[u][3] = __builtin_fmaf(wt, ob[k][u][3], acc[u][3]);
-        }
-        L = __builtin_fmaf(wt, lb[k], L);
-      }
-    }
-  };
-  if (nparts <= kBatch) {
-    load_batch(0);
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k) M = fmaxf(M, mb[k]);  // repeats of the last part change nothing
-    accumulate(0);
-  } else {
-    for (int j0 = 0; j0 < nparts; j0 += kBatch) {
-#pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        const int j = j0 + k < nparts ? j0 + k : nparts - 1;
-        M = fmaxf(M, ml_at(j)[0]);
-      }
-    }
-    for (int j0 = 0; j0 < nparts; j0 += kBatch) {
-      load_batch(j0);
-      accumulate(j0);
-    }
-  }
-  const float inv = (L == 0.f) ? 0.f : kv_scale * __builtin_amdgcn_rcpf(L);
-#pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    out[u][0] = pack2_bf16_canon<kRTNE>(acc[u][0] * inv, acc[u][1] * inv);
-    out[u][1] = pack2_bf16_canon<kRTNE>(acc[u][2] * inv, acc[u][3] * inv);
-  }
+// Merge of one query row over its request's parts: M = max_p m_p, w_p = 2^(m_p - M)
+// (exact, m_p integer-valued), out = sum w_p O_p * kv_scale / sum w_p l_p.
+__device__ __forceinline__ float part_weight(float m_p, float M) {
+  const float diff = m_p - M;  // integer-valued or -inf, <= 0
+  return (m_p == -__builtin_inff()) ? 0.f : ((diff >= -126.f) ? __builtin_ldexpf(1.0f, (int)diff) : 0.f);
 }
-
+__device__ __forceinline__ u32x2 merge_finish(f32x4 acc, float L, float kv_scale) {
+  const float inv = (L == 0.f) ? 0.f : kv_scale * __builtin_amdgcn_rcpf(L);
+  return u32x2{pack2_bf16_canon<kRTNE>(acc[0] * inv, acc[1] * inv), pack2_bf16_canon<kRTNE>(acc[2] * inv, acc[3] * inv)};
+}
+// Parts j0, j0 + step, ... (up to kMergeBatch of them below nparts) added to
+// (acc, L) under the max M: their (m, l) pairs and O slices are loaded together,
+// one round of memory latency.
+constexpr int kMergeBatch = 8;
 template <class OAt, class MlAt>
-__device__ __forceinline__ u32x2 merge_slice(int nparts, float kv_scale, OAt o_at, MlAt ml_at) {
-  u32x2 o[1];
-  merge_slices<1>(nparts, kv_scale, [&](int j, int) { return o_at(j); }, ml_at, o);
-  return o[0];
+__device__ __forceinline__ void merge_batch(int j0, int step, int nparts, OAt o_at, MlAt ml_at, bool own_max, float& M,
+                                            f32x4& acc, float& L) {
+  float mb[kMergeBatch], lb[kMergeBatch];
+  f32x4 ob[kMergeBatch];
+#pragma unroll
+  for (int k = 0; k < kMergeBatch; ++k) {
+    const int j = j0 + k * step;
+    mb[k] = -__builtin_inff();
+    lb[k] = 0.f;
+    ob[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (j < nparts) {
+      const float2 m_l = *reinterpret_cast<const float2*>(ml_at(j));
+      mb[k] = m_l.x;
+      lb[k] = m_l.y;
+      ob[k] = *reinterpret_cast<const f32x4*>(o_at(j));
+    }
+  }
+  if (own_max) {
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) M = fmaxf(M, mb[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < kMergeBatch; ++k) {
+    if (j0 + k * step < nparts) {
+      const float wt = part_weight(mb[k], M);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(wt, ob[k][e], acc[e]);
+      L = __builtin_fmaf(wt, lb[k], L);
+    }
+  }
 }
 
 __device__ __forceinline__ int merge_out_row(const Params& p, int b) {
@@ -122,28 +83,67 @@ __device__ __forceinline__ int merge_out_row(const Params& p, int b) {
   return qb;
 }
 
-// Merge of row-major records: one thread = 4 output dims of one (b, query row).
-__global__ __launch_bounds__(256) void mla_merge_kernel(Params p) {
-  const long long cell = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long per_b = (long long)p.qrows * (kLat / 4);
-  if (cell >= per_b * p.B) return;
-  const int b = (int)(cell / per_b);
-  const int rem = (int)(cell % per_b);
-  const int qrow = rem / (kLat / 4);
-  const int d = (rem % (kLat / 4)) * 4;
-  const int qb = merge_out_row(p, b);
+// Merge of the split requests' records, 128 threads (4 output dims each) times
+// GROUPS per query row; group g adds parts g, g + GROUPS, ... and the groups'
+// sums meet in LDS. A thread's parts cost a round of memory latency per batch of
+// 8: four groups for many parts, as long as the rows are few (with many, latency
+// is covered and four times the threads only cost). Whole calls, one -> four
+// groups: 16 rows in 33 parts 15.1 -> 12.5 us, 128 rows in 33 parts 21.4 -> 20.8;
+// 1024 rows in 17 parts 26.9 -> 31.8, 2048 rows in 9 parts 41.1 -> 45.5, 1024 rows
+// in 5 parts 38.3 -> 41.6.
+constexpr int kMergeWideParts = 8;
+constexpr int kMergeWideRows = 256;
+template <int GROUPS>
+__global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS) void mla_merge_kernel(Params p) {
+  constexpr int kRowsPerCta = GROUPS == 1 ? 2 : 1;
+  const int tid = threadIdx.x;
+  const int cell = tid & 127;
+  const int grp = GROUPS == 1 ? 0 : tid >> 7;
+  const long long row = (long long)blockIdx.x * kRowsPerCta + (GROUPS == 1 ? tid >> 7 : 0);
+  if (row >= (long long)p.B * p.qrows) return;  // GROUPS > 1: the grid is exact
+  const int b = (int)(row / p.qrows);
+  const int qrow = (int)(row % p.qrows);
+  const int d = cell * 4;
   const float* ml = ws_ml(p);
   const int* tbl = ws_tbl(p);
   const int nparts = tbl[2 * b];
   const int rec0 = tbl[2 * b + 1];
   if (nparts <= 1) return;  // the decode kernel wrote this request's output
-  const u32x2 o = merge_slice(
-      nparts, p.kv_scale, [&](int j) { return ws_rec_o(p, (size_t)rec0 + j) + (size_t)qrow * kLat + d; },
-      [&](int j) { return ml + (((size_t)rec0 + j) * p.qrows + qrow) * 2; });
+  auto o_at = [&](int j) { return ws_rec_o(p, (size_t)rec0 + j) + (size_t)qrow * kLat + d; };
+  auto ml_at = [&](int j) { return ml + (((size_t)rec0 + j) * p.qrows + qrow) * 2; };
+  float M = -__builtin_inff(), L = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (GROUPS == 1 && nparts <= kMergeBatch) {
+    merge_batch(0, 1, nparts, o_at, ml_at, true, M, acc, L);
+  } else {
+    // The row's max by the wave: lane l looks at parts l, l + 64, ...
+    for (int j = tid & 63; j < nparts; j += 64) M = fmaxf(M, ml_at(j)[0]);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
+    for (int j0 = grp; j0 < nparts; j0 += kMergeBatch * GROUPS)
+      merge_batch(j0, GROUPS, nparts, o_at, ml_at, false, M, acc, L);
+  }
+  if constexpr (GROUPS > 1) {
+    __shared__ f32x4 part_o[GROUPS - 1][128];
+    __shared__ float part_l[GROUPS - 1];
+    if (grp > 0) {
+      part_o[grp - 1][cell] = acc;
+      if (cell == 0) part_l[grp - 1] = L;
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int k = 0; k < GROUPS - 1; ++k) {
+      const f32x4 o = part_o[k][cell];
+      acc += o;
+      L += part_l[k];
+    }
+  }
   // Non-temporal: written once, read by no later kernel of the call (H=16:
   // 45.8 -> 44.4 us per call; the same in the decode kernels measured neutral
   // or slower).
-  __builtin_nontemporal_store(o, reinterpret_cast<u32x2*>(p.o_lat + ((long long)qb * p.qrows + qrow) * kLat + d));
+  __builtin_nontemporal_store(merge_finish(acc, L, p.kv_scale),
+                              reinterpret_cast<u32x2*>(p.o_lat + ((long long)merge_out_row(p, b) * p.qrows + qrow) * kLat + d));
 }
 
 // Test hook: decode fp8 bytes with the same hardware convert the kernel uses.
@@ -169,7 +169,8 @@ namespace {
 using namespace mm::mla;
 
 constexpr int kNumCUs = 256;
-constexpr int kMaxParts = 64;
+constexpr int kMaxParts = 256;
+constexpr int kScratchParts = 64;          // parts that the allocation-free entry's size limit counts
 constexpr size_t kScratchRecords = 32768;  // record rows of the allocation-free entry's array
 
 // Requests of at most 16 query rows run mla_coop_kernel, larger ones
@@ -209,15 +210,28 @@ int unit_cap_for(int H, int q_len) {
   return c < 1 ? 1 : c;
 }
 
+// Tokens of the shortest part worth a CTA. One request of 4097 tokens: 16 heads
+// 12.9 us with 64, 12.5 with 128, 12.9 with 192, 13.5 with 256, 17.0 with 512; 128
+// heads 27.7, 20.8, 19.7, 19.7, 23.9 (64-row CTAs: more set-up and larger records).
+int min_chunk_for(int H, int q_len) { return use_coop(H, q_len) ? 128 : 256; }
+
 // Split planner: parts whose records let the balanced split fill the unit cap
 // (see workers_for), within the record workspace and the allocation-free
-// entry's array.
+// entry's array, or one where the tiles saved on the longest path (the batch's
+// mean length taken as 0.6 of the longest) are worth less than the merge launch:
+// 100 requests of 300 tokens, 16 heads: 17.7 us split, 12.9 whole.
+constexpr int kMergeCostTiles = 5;
 int plan_parts(int B, int H, int max_seq_len, int q_len) {
   if (B < 1) B = 1;
   if (q_len < 1) q_len = 1;
   const int units = unit_cap_for(H, q_len);
+  const int min_chunk = min_chunk_for(H, q_len);
+  const long long tiles = (long long)max_seq_len / kTileTok + 1;
+  const long long whole = tiles * ((B + units - 1) / units);
+  const long long shared = tiles * B * 3 / (5LL * units);
+  if (whole - (shared > min_chunk / kTileTok ? shared : min_chunk / kTileTok) < kMergeCostTiles) return 1;
   int p = 1 + (units + B - 2) / B;
-  const int by_len = 1 + max_seq_len / 512;  // chunks are at least 512 tokens
+  const int by_len = 1 + max_seq_len / min_chunk;
   if (p > by_len) p = by_len;
   const int cap = max_parts_for(B, H, q_len);
   if (p > cap) p = cap;
@@ -284,6 +298,7 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   p.ngroups = ngroups_for(H, q_len);
   p.unit_cap = unit_cap_for(H, q_len);
   p.workers = workers_for(B, H, p.parts, q_len);
+  p.min_chunk = min_chunk_for(H, q_len);
   p.paged = paged ? 1 : 0;
   p.qrows = H * q_len;
   p.rec_rows = rec_rows_for(H, q_len);
@@ -301,8 +316,11 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   else
     launch_rows64_kernel(p, grid, st);
   if (p.parts > 1) {
-    const long long cells = (long long)B * p.qrows * (kLat / 4);
-    hipLaunchKernelGGL(mla_merge_kernel, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, st, p);
+    const long long rows_all = (long long)B * p.qrows;
+    if (p.parts > kMergeWideParts && rows_all <= kMergeWideRows)
+      hipLaunchKernelGGL(mla_merge_kernel<4>, dim3((unsigned)rows_all), dim3(512), 0, st, p);
+    else
+      hipLaunchKernelGGL(mla_merge_kernel<1>, dim3((unsigned)((rows_all + 1) / 2)), dim3(256), 0, st, p);
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
@@ -386,10 +404,13 @@ int launch_mla_decode_a16w8_paged_dev_noalloc(const void* q_lat, const void* q_p
   const int arg_rc = check_launch_args(q_lat, q_pe, kv_pool, o_lat, seq_lens, kv_indices, kv_indptr, B, H, 0, q_len,
                                        lat_dim, rope_dim, true);
   if (arg_rc != 0) return arg_rc;
-  const int eff = clamp_parts(parts, B, H, q_len, true);
+  int eff = clamp_parts(parts, B, H, q_len, true);
   void* ws = nullptr;
   if (eff > 1) {
-    if ((size_t)B * eff * rec_rows_for(H, q_len) > kScratchRecords) return -9;
+    // The limit is on up to 64 parts; more of them share what fits.
+    const size_t rows_b = (size_t)B * rec_rows_for(H, q_len);
+    if (rows_b * (eff < kScratchParts ? eff : kScratchParts) > kScratchRecords) return -9;
+    if (rows_b * eff > kScratchRecords) eff = (int)(kScratchRecords / rows_b);
     const int rc = scratch_ptr(&ws);
     if (rc != 0) return rc;
   }

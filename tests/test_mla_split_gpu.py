@@ -131,3 +131,35 @@ def test_block_table_clamps_pages_and_lengths(H, parts):
         outs.append(o)
     assert not torch.isnan(outs[0].float()).any()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_noalloc_shares_its_array_beyond_64_parts():
+    """300 parts of 256 rows: the size limit of the allocation-free entry counts
+    64 of them (accepted); the call then uses the 128 that its array holds."""
+    from moonmath_attention import _lib
+
+    H, q_len, S = 128, 2, 20000
+    pool, idx, indptr = paged_pool([S], 99)
+    q_lat, q_pe = rand_q(1, q_len, H, 99)
+    t = [_d(x) for x in (q_lat, q_pe, pool)]
+    n = torch.tensor([S], dtype=torch.int32, device=DEV)
+    idx, indptr = _d(idx), _d(indptr)
+    lib, p, st = _lib.lib, _lib.ptr, _lib.stream_ptr(DEV)
+    outs = []
+    for noalloc in (True, False):
+        o = torch.full((1, q_len, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+        parts = 300 if noalloc else 128
+        head = (p(t[0]), p(t[1]), p(t[2]), p(o), p(n), None, p(idx), p(indptr), 1, H, parts, 512, 64, SCALE_576,
+                KV_SCALE, 1.0)
+        if noalloc:
+            rc = lib.launch_mla_decode_a16w8_paged_dev_noalloc(*head, st, 0, q_len)
+        else:
+            ws = torch.empty(lib.mla_decode_a16w8_multiq_workspace_for(1, H, parts, q_len), dtype=torch.uint8,
+                             device=DEV)
+            rc = lib.launch_mla_decode_a16w8_paged_dev(*head, p(ws), st, 0, q_len)
+        torch.cuda.synchronize()
+        assert rc == 0
+        outs.append(o)
+    assert not torch.isnan(outs[0].float()).any()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
