@@ -72,11 +72,18 @@ constexpr int kLdsBytes = kRing * (kKBytes + kVBytes);  // K ring + V_t ring
 // and l never hold a p above 2^20 (no fp32 overflow of O for |v| < 2^90).
 constexpr float kGrowLimit = 1048576.0f;     // 2^20
 
+// Half CTAs: 4 waves, 128 q rows, two CTAs per CU (one wave of each per SIMD),
+// 2-slot rings.
+constexpr int kHalfWaves = 4;
+constexpr int kHalfThreads = 64 * kHalfWaves;
+constexpr int kHalfRows = kHalfWaves * kQRowsPerTile;  // 128
+constexpr int kHalfRing = 2;
+constexpr int kLdsHalfBytes = kHalfRing * (kKBytes + kVBytes);
+
 // Split-KV limits: partial records are laid out for CTAs of kMaxRows q rows
 // and up to kMaxParts parts.
 constexpr int kMaxRows = kRowsPerCta;
 constexpr int kMaxParts = 1024;
-constexpr size_t kPartOFloats = (size_t)kMaxRows * kD;
 constexpr size_t kWorkspaceBytes = (size_t)kMaxParts * kMaxRows * (kD + 2) * sizeof(float);
 
 // LiteAttention: a CTA's processed block list (int16 ids, bit 15 marks the
@@ -119,6 +126,8 @@ struct Params {
   int nqb, nkb;      // q-blocks per head, kv blocks per head
   int prefix_wgs;    // CTAs that run the whole KV stream
   int split_ways;    // G (parts per tail q-block)
+  int rec_rows;      // rows of a split record: O [rec_parts][rec_rows][128], then (m, l) [rec_parts][rec_rows][2]
+  int rec_parts;
   float scale_log2e; // log2(e) / sqrt(128), rounded to fp32 on the host
   // LiteAttention only.
   const int16_t* read_list;   // [B*H][nqb][nkb + 2]
@@ -228,9 +237,12 @@ __device__ __forceinline__ void lite_emit(const Params& p, long long row, int n,
 // two transposing reads (ds_read_b64_tr_b16) each instead of one ds_read_b128.
 // Those move half the bytes per clock, but no V_t pass precedes the launch (see
 // prefers_direct for both sides measured).
-template <int MODE, bool LITE, bool SHORT = false, bool VROW = false>
+template <int MODE, bool LITE, bool SHORT = false, bool VROW = false, int NW = kWaves>
 __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb_begin, int kb_end, int part,
                                          char* lds, ShortCtx* sc = nullptr) {
+  static_assert(NW == kWaves || (NW == kHalfWaves && !LITE && !SHORT), "half CTAs: dense tiles");
+  constexpr int NI = 16 / NW;                            // K (and V) DMA instructions per wave and block
+  constexpr int RING = NW == kWaves ? kRing : kHalfRing;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -262,19 +274,19 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   // V_t slot: fragments [t(2)][s(2)][dt(4)], 1 KB each in lane order.
   // Short KV: K slots 0..1, V_t slots 0..1, the output stage, the Q stage.
   char* kring = lds;
-  char* vring = lds + (SHORT ? kShortMaxBlocks : kRing) * kKBytes;
+  char* vring = lds + (SHORT ? kShortMaxBlocks : RING) * kKBytes;
   auto kslot_off = [](int k, int c) { return (k >> 4) * 4096 + c * 256 + (k & 15) * 16; };
   // This lane's MFMA fragment cell for row tile t, k-step ds: kfrag_lane +
   // 8192 t + 512 ds (rows t*32 + r, chunk 2 ds + g), constants the LDS reads
   // carry as immediate offsets.
   const int kfrag_lane = kslot_off(r, g);
-  // Lane source row / chunk of this wave's 2 K-DMA instructions (instruction
-  // j = 2 wave + i fills slot bytes 1024 j .. 1024 j + 1023).
-  auto kdma_row = [&](int i) { return 16 * ((wave * 2 + i) >> 2) + (lane & 15); };
-  auto kdma_chunk = [&](int i) { return 4 * ((wave * 2 + i) & 3) + (lane >> 4); };
-  uint32_t koff[2];
+  // Lane source row / chunk of this wave's NI K-DMA instructions (instruction
+  // j = NI wave + i fills slot bytes 1024 j .. 1024 j + 1023).
+  auto kdma_row = [&](int i) { return 16 * ((wave * NI + i) >> 2) + (lane & 15); };
+  auto kdma_chunk = [&](int i) { return 4 * ((wave * NI + i) & 3) + (lane >> 4); };
+  uint32_t koff[NI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) koff[i] = (uint32_t)(kdma_row(i) * row_stride * 2) + (uint32_t)(kdma_chunk(i) * 16);
+  for (int i = 0; i < NI; ++i) koff[i] = (uint32_t)(kdma_row(i) * row_stride * 2) + (uint32_t)(kdma_chunk(i) * 16);
   const long long kblk_bytes = (long long)kKvBlock * row_stride * 2;
   // Instruction i of the last partial block: rows past Skv are clamped (they are
   // masked in softmax).
@@ -282,43 +294,43 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
     int kv = kb * kKvBlock + kdma_row(i);
     kv = kv < p.Skv ? kv : p.Skv - 1;
     dma16_opaque(kh + (long long)kv * row_stride * 2 + kdma_chunk(i) * 16,
-                 kring + slot * kKBytes + (wave * 2 + i) * kFragBytes);
+                 kring + slot * kKBytes + (wave * NI + i) * kFragBytes);
   };
   auto issue_k = [&](int kb, int slot) {
     char* st = kring + slot * kKBytes;
     if ((kb + 1) * kKvBlock <= p.Skv) {
       const char* base = kh + kb * kblk_bytes;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma16_sbase(base, koff[i], st + (wave * 2 + i) * kFragBytes);
+      for (int i = 0; i < NI; ++i) dma16_sbase(base, koff[i], st + (wave * NI + i) * kFragBytes);
     } else {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) issue_k_clamped(kb, slot, i);
+      for (int i = 0; i < NI; ++i) issue_k_clamped(kb, slot, i);
     }
   };
-  // V_t: 1 KB fragments as they are. VROW: instruction j = 2 wave + i moves rows
+  // V_t: 1 KB fragments as they are. VROW: instruction j = NI wave + i moves rows
   // 4j .. 4j+3 (lane l: row 4j + l/16, 16-byte slot l % 16), row rr's chunk c at
   // slot c ^ 4 (rr % 4): the four rows of a transposing read hit distinct banks.
-  auto vdma_row = [&](int i) { return 4 * (wave * 2 + i) + (lane >> 4); };
-  uint32_t voff[2];
+  auto vdma_row = [&](int i) { return 4 * (wave * NI + i) + (lane >> 4); };
+  uint32_t voff[NI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NI; ++i)
     voff[i] = VROW ? (uint32_t)(vdma_row(i) * row_stride * 2) + (uint32_t)(16 * ((lane & 15) ^ (4 * (vdma_row(i) & 3))))
-                   : (uint32_t)((wave * 2 + i) * kFragBytes + lane * 16);
+                   : (uint32_t)((wave * NI + i) * kFragBytes + lane * 16);
   const long long vblk_bytes = VROW ? kblk_bytes : (long long)kVBytes;
   auto issue_v = [&](int kb, int slot) {
     char* st = vring + slot * kVBytes;
     const char* base = vth + kb * vblk_bytes;
     if (!VROW || (kb + 1) * kKvBlock <= p.Skv) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma16_sbase(base, voff[i], st + (wave * 2 + i) * kFragBytes);
+      for (int i = 0; i < NI; ++i) dma16_sbase(base, voff[i], st + (wave * NI + i) * kFragBytes);
     } else {
       // Last partial block: rows past Skv are zero (p = 0 there, and 0 x inf is
       // not), written by the lanes that would have fetched them. The block waits
       // count instructions, so an instruction without any valid row is replaced
       // by a repeat of this wave's K one.
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        char* dst = st + (wave * 2 + i) * kFragBytes;
+      for (int i = 0; i < NI; ++i) {
+        char* dst = st + (wave * NI + i) * kFragBytes;
         const bool valid = kb * kKvBlock + vdma_row(i) < p.Skv;
         if (__builtin_amdgcn_ballot_w64(valid) == 0) issue_k_clamped(kb, slot, i);
         if (valid) {
@@ -336,7 +348,7 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
 
   // ---- Q fragments (B operand of S^T = K Q^T), kept in registers --------------
   bf16x8 qf[8];
-  const int q_row0 = qb * kRowsPerCta + wave * kQRowsPerTile;
+  const int q_row0 = qb * (NW * kQRowsPerTile) + wave * kQRowsPerTile;
   // A wave whose 32 query rows all lie past Sq (in the last q-block of a
   // ragged Sq; dense, unsplit tiles) issues its share of every block's DMAs
   // and meets every block barrier in the same order as its CTA's other waves,
@@ -344,26 +356,42 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   if constexpr (!LITE && !SHORT) {
     if (part < 0 && q_row0 >= p.Sq && kb_end > kb_begin) {
       const int nb = kb_end - kb_begin;
-      for (int j = 0; j < 3 && j < nb; ++j) {
-        issue_k(kb_begin + j, j);
-        issue_v(kb_begin + j, j);
-      }
-      if (nb > 2) {
-        wait_vmem_barrier<8>();
-      } else if (nb > 1) {
-        wait_vmem_barrier<4>();
-      } else {
-        wait_vmem_barrier<0>();
-      }
-      for (int i = 0; i < nb; ++i) {
-        if (i + 2 < nb) {
-          asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        } else {
-          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if constexpr (NW == kWaves) {
+        for (int j = 0; j < 3 && j < nb; ++j) {
+          issue_k(kb_begin + j, j);
+          issue_v(kb_begin + j, j);
         }
-        if (i + 3 < nb) {
-          issue_k(kb_begin + i + 3, (i + 3) % kRing);
-          issue_v(kb_begin + i + 3, (i + 3) % kRing);
+        if (nb > 2) {
+          wait_vmem_barrier<8>();
+        } else if (nb > 1) {
+          wait_vmem_barrier<4>();
+        } else {
+          wait_vmem_barrier<0>();
+        }
+        for (int i = 0; i < nb; ++i) {
+          if (i + 2 < nb) {
+            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          } else {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          }
+          if (i + 3 < nb) {
+            issue_k(kb_begin + i + 3, (i + 3) % kRing);
+            issue_v(kb_begin + i + 3, (i + 3) % kRing);
+          }
+        }
+      } else {
+        issue_k(kb_begin, 0);
+        issue_v(kb_begin, 0);
+        if (nb > 1) issue_k(kb_begin + 1, 1);
+        if (nb > 1) {
+          wait_vmem_barrier<2 * NI>();
+        } else {
+          wait_vmem_barrier<NI>();
+        }
+        for (int i = 0; i < nb; ++i) {
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          if (i + 2 < nb) issue_k(kb_begin + i + 2, i & 1);
+          if (i + 1 < nb) issue_v(kb_begin + i + 1, (i + 1) & 1);
         }
       }
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -563,6 +591,16 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
         }
       }
       sc->resident = bh;
+    } else if constexpr (NW != kWaves) {
+      // Two slots each: K of block 1 and V of block 0 behind K of block 0.
+      issue_k(blk_of(0), 0);
+      issue_v(blk_of(0), 0);
+      if (nblk > 1) {
+        issue_k(blk_of(1), 1);
+        wait_vmem_barrier<2 * NI>();
+      } else {
+        wait_vmem_barrier<NI>();
+      }
     } else {
       issue_kv(blk_of(0), 0);
       if (nblk > 1) issue_kv(blk_of(1), 1);
@@ -597,7 +635,7 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       if constexpr (SHORT) {
         // Every block is resident and no slot is refilled: no barrier, and no
         // wait for the Q prefetch in flight.
-      } else if (i + 2 < nblk) {
+      } else if (NW == kWaves && i + 2 < nblk) {
         asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       } else {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -609,23 +647,30 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       // Block kb+3: a full block's 4 DMAs go out one per odd QK step below (all
       // 8 waves issuing theirs back to back after the barrier stall their QK);
       // a partial last block is gathered here.
-      const bool dma3 = i + 3 < nblk;
-      const int kb3 = !dma3 ? kb : LITE ? __builtin_amdgcn_readfirstlane(kb3_raw & 0x7FFF) : kb_begin + i + 3;
-      const bool dma3_full = dma3 && (kb3 + 1) * kKvBlock <= p.Skv;
-      if (dma3 && !dma3_full) issue_kv(kb3, (i + 3) % kRing);
-      const int pd3 = __builtin_amdgcn_readfirstlane((int)dma3_full);
+      // Half CTAs have two slots each: block i+2 of K takes the slot that QK(i)
+      // has left, block i+1 of V that of PV(i-1); both land by the next barrier.
+      constexpr int kLeadK = NW == kWaves ? 3 : 2, kLeadV = NW == kWaves ? 3 : 1;
+      const bool dma_k = i + kLeadK < nblk, dma_v = i + kLeadV < nblk;
+      const int kb3 = !dma_k ? kb : LITE ? __builtin_amdgcn_readfirstlane(kb3_raw & 0x7FFF) : kb_begin + i + kLeadK;
+      const int vb3 = NW == kWaves ? kb3 : !dma_v ? kb : kb_begin + i + kLeadV;
+      const bool dma_k_full = dma_k && (kb3 + 1) * kKvBlock <= p.Skv;
+      const bool dma_v_full = NW == kWaves ? dma_k_full : dma_v && (vb3 + 1) * kKvBlock <= p.Skv;
+      if (dma_k && !dma_k_full) issue_k(kb3, (i + kLeadK) % RING);
+      if (dma_v && !dma_v_full) issue_v(vb3, (i + kLeadV) % RING);
+      const int pdk = __builtin_amdgcn_readfirstlane((int)dma_k_full);
+      const int pdv = __builtin_amdgcn_readfirstlane((int)dma_v_full);
       const char* kbase3 = kh + (long long)kb3 * kblk_bytes;
-      const char* vbase3 = vth + (long long)kb3 * vblk_bytes;
-      const char* kst3 = kring + ((i + 3) % kRing) * kKBytes;
-      const char* vst3 = vring + ((i + 3) % kRing) * kVBytes;
-      auto dma3_step = [&](int d) {  // d = 0, 1: K instructions; 2, 3: V instructions
+      const char* vbase3 = vth + (long long)vb3 * vblk_bytes;
+      const char* kst3 = kring + ((i + kLeadK) % RING) * kKBytes;
+      const char* vst3 = vring + ((i + kLeadV) % RING) * kVBytes;
+      auto dma3_step = [&](int d) {  // d < NI: K instructions; then V instructions
         // Global address = SGPR base + 32-bit lane offset (no 64-bit VALU add).
-        const char* base = d < 2 ? kbase3 : vbase3;
-        const uint32_t off = d < 2 ? koff[d] : voff[d - 2];
-        const char* dst = d < 2 ? kst3 + (wave * 2 + d) * kFragBytes : vst3 + (wave * 2 + d - 2) * kFragBytes;
+        const char* base = d < NI ? kbase3 : vbase3;
+        const uint32_t off = d < NI ? koff[d] : voff[d - NI];
+        const char* dst = d < NI ? kst3 + (wave * NI + d) * kFragBytes : vst3 + (wave * NI + d - NI) * kFragBytes;
         const uint32_t m0v = (uint32_t)(uintptr_t)(MM_LDS const char*)dst;
         asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 1f\n\tglobal_load_lds_dwordx4 %0, %1\n1:" ::"v"(off),
-                     "s"(base), "{m0}"(m0v), "s"(pd3)
+                     "s"(base), "{m0}"(m0v), "s"(d < NI ? pdk : pdv)
                      : "memory", "scc");
       };
       mask(scur, kb);
@@ -634,8 +679,8 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
       // the rest; PV(i) of row tile 1 follows, its second k-step after the next
       // barrier. Per-accumulator orders (S, O and each lpart sum) are those of
       // an unsliced softmax.
-      const char* kst = kring + ((i + 1) % kRing) * kKBytes;  // last block: stale slot, unused
-      const char* vst = vring + (i % kRing) * kVBytes;
+      const char* kst = kring + ((i + 1) % RING) * kKBytes;  // last block: stale slot, unused
+      const char* vst = vring + (i % RING) * kVBytes;
       const float neg_m0 = -row_m;
       float lpart[4] = {0.f, 0.f, 0.f, 0.f};
       uint32_t w[2][2][4];
@@ -755,7 +800,11 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
           vmx = fmaxf(fmaxf(vmx, scur[t][e0]), scur[t][e0 + 1]);
           vmx = fmaxf(fmaxf(vmx, scur[t][e0 + 2]), scur[t][e0 + 3]);
         }
-        if (ds & 1) dma3_step(ds >> 1);
+        if constexpr (NW == kWaves) {
+          if (ds & 1) dma3_step(ds >> 1);
+        } else {
+          dma3_step(ds);
+        }
         if constexpr (!LAST) {
           if (!half_next) snext[1] = mfma32(kf1, qf[ds], snext[1]);
         }
@@ -875,10 +924,9 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   // ---- epilogue -----------------------------------------------------------------
   row_l = xor32_sum(row_l);
   if (part >= 0) {
-    // Split part: unnormalised fp32 partials. Record layout per part:
-    // O [kMaxRows][128] fp32 then (m, l) [kMaxRows][2] fp32.
-    float* po = p.ws + (size_t)part * kPartOFloats;
-    float* pml = p.ws + (size_t)kMaxParts * kPartOFloats + (size_t)part * kMaxRows * 2;
+    // Split part: unnormalised fp32 partials (see Params).
+    float* po = p.ws + (size_t)part * p.rec_rows * kD;
+    float* pml = p.ws + (size_t)p.rec_parts * p.rec_rows * kD + (size_t)part * p.rec_rows * 2;
     const int row = wave * kQRowsPerTile + r;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -911,7 +959,8 @@ __device__ __forceinline__ void run_tile(const Params& p, int bh, int qb, int kb
   if constexpr (SHORT) {
     ost = lds + kShortOStageOff + wave * (kRoundRows * 256);
   } else {
-    const int slot = ((wave & 2) ? nblk + 2 : nblk + 1) & (kRing - 1);
+    // Half CTAs: the K slots, which the last step does not read.
+    const int slot = NW == kWaves ? ((wave & 2) ? nblk + 2 : nblk + 1) & (kRing - 1) : wave >> 1;
     ost = ((wave & 4) ? vring : kring) + slot * kKBytes + (wave & 1) * (kQRowsPerTile * 256);
   }
   u32x2 ow[4][4];
@@ -962,6 +1011,24 @@ __global__ __launch_bounds__(kThreads, 1) void attn_fwd_kernel(Params p) {
     const int kb0 = (int)((long long)p.nkb * j / p.split_ways);
     const int kb1 = (int)((long long)p.nkb * (j + 1) / p.split_ways);
     run_tile<MODE, false, false, VROW>(p, w / p.nqb, w % p.nqb, kb0, kb1, part, lds);
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kHalfThreads, 2) void attn_half_kernel(Params p) {
+  __shared__ __attribute__((aligned(1024))) char lds[kLdsHalfBytes];
+  if (p.split_ways == 1) {
+    const int w = xcd_remap(blockIdx.x, p.prefix_wgs);
+    run_tile<MODE, false, false, true, kHalfWaves>(p, w / p.nqb, w % p.nqb, 0, p.nkb, -1, lds);
+  } else {
+    // A head's tiles of one KV range run on one XCD (they read the same K and V).
+    const int id = xcd_remap(blockIdx.x, p.rec_parts);
+    const int per_head = p.split_ways * p.nqb;
+    const int bh = id / per_head, j = id % per_head / p.nqb, qb = id % p.nqb;
+    const int part = (bh * p.nqb + qb) * p.split_ways + j;
+    const int kb0 = (int)((long long)p.nkb * j / p.split_ways);
+    const int kb1 = (int)((long long)p.nkb * (j + 1) / p.split_ways);
+    run_tile<MODE, false, false, true, kHalfWaves>(p, bh, qb, kb0, kb1, part, lds);
   }
 }
 
@@ -1147,20 +1214,42 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(Params p, int
   if (qr >= p.Sq) return;
   const int G = p.split_ways;
   const int part0 = t * G;
-  const float* pml = p.ws + (size_t)kMaxParts * kPartOFloats;
+  const float* pml = p.ws + (size_t)p.rec_parts * p.rec_rows * kD;
+  // kBatch parts' loads go out together: a round of memory latency per batch,
+  // not per part.
+  constexpr int kBatch = 8;
+  auto ml_at = [&](int j) { return pml + ((size_t)(part0 + j) * p.rec_rows + row) * 2; };
   float M = kNegFltMax;
-  for (int j = 0; j < G; ++j) M = fmaxf(M, pml[(size_t)(part0 + j) * kMaxRows * 2 + row * 2]);
+  for (int j0 = 0; j0 < G; j0 += kBatch) {
+    float m[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) m[k] = j0 + k < G ? ml_at(j0 + k)[0] : kNegFltMax;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) M = fmaxf(M, m[k]);
+  }
   float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f, L = 0.f;
-  for (int j = 0; j < G; ++j) {
-    const float m_p = pml[(size_t)(part0 + j) * kMaxRows * 2 + row * 2];
-    const float l_p = pml[(size_t)(part0 + j) * kMaxRows * 2 + row * 2 + 1];
-    const f32x4 o = *reinterpret_cast<const f32x4*>(p.ws + (size_t)(part0 + j) * kPartOFloats + (size_t)row * kD + d);
-    const float wt = pow2_weight(m_p, M);
-    o0 = __builtin_fmaf(wt, o[0], o0);
-    o1 = __builtin_fmaf(wt, o[1], o1);
-    o2 = __builtin_fmaf(wt, o[2], o2);
-    o3 = __builtin_fmaf(wt, o[3], o3);
-    L = __builtin_fmaf(wt, l_p, L);
+  for (int j0 = 0; j0 < G; j0 += kBatch) {
+    float m[kBatch], l[kBatch];
+    f32x4 o[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      if (j0 + k < G) {
+        m[k] = ml_at(j0 + k)[0];
+        l[k] = ml_at(j0 + k)[1];
+        o[k] = *reinterpret_cast<const f32x4*>(p.ws + ((size_t)(part0 + j0 + k) * p.rec_rows + row) * kD + d);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      if (j0 + k < G) {
+        const float wt = pow2_weight(m[k], M);
+        o0 = __builtin_fmaf(wt, o[k][0], o0);
+        o1 = __builtin_fmaf(wt, o[k][1], o1);
+        o2 = __builtin_fmaf(wt, o[k][2], o2);
+        o3 = __builtin_fmaf(wt, o[k][3], o3);
+        L = __builtin_fmaf(wt, l[k], L);
+      }
+    }
   }
   const float inv = (L == 0.f) ? 0.f : __builtin_amdgcn_rcpf(L);
   const int b = bh / p.H, h = bh % p.H;
@@ -1310,6 +1399,57 @@ TailPlan plan_tail(int nqb, int nbh, int nkb, int slots, bool enable, int force_
   return TailPlan{wgs - tail, tail, G, tail * G};
 }
 
+// Whether a forward on V itself runs half CTAs, and into how many KV parts each
+// of its tiles is split. In KV blocks of a 256-row CTA's time:
+//  * At most one half CTA per CU: a wave alone on its SIMD takes 0.6 of the pair's
+//    time per block and twice the CUs work; split where the blocks saved outweigh
+//    the merge launch and the records. Measured, 256-row CTAs with their own split
+//    -> half CTAs: (1,2,256) 12.1 -> 9.3 us, (1,8,600) 20.9 -> 16.6, (1,24,1024)
+//    30.5 -> 23.2, (1,16,2000) 48.6 -> 40.9; with half CTAs split (1,8,128) x 2000
+//    20.0 -> 18.3 (38.1 unsplit), (1,2,256) x 8192 29.1 -> 26.6, (1,2,2000) 24.6 ->
+//    21.5; the other way (1,8,2000) 34.0 -> 36.5, (2,24,256) x 8192 67 -> 119.
+//  * More: two half CTAs of a CU overlap their ends and leave a finer last round,
+//    but gather K and V twice: whole pairs of them take 1.06 of a 256-row CTA's
+//    time, 0.96 up to 4 blocks. (2,24,2048) 113 -> 106 us, (2,12,3000) x 300 28.8
+//    -> 24.5, (2,24,8192) x 200 90.6 -> 86.0; (1,24,1531) 39.7 -> 42.0, (2,24,4096)
+//    361 -> 378.
+struct HalfPlan {
+  bool half;
+  int split_ways;
+};
+constexpr int kHalfSplitCost = 3;       // blocks: the merge launch
+constexpr int kFullSplitExtra = 2;      // what plan_tail's span leaves out of a split of whole CTAs here
+constexpr int kHalfPartsPerBlock = 48;  // records per block of time
+HalfPlan plan_half(int seq_len, long long nbh, int nkb, bool split) {
+  const long long tiles = (seq_len + kHalfRows - 1) / kHalfRows * nbh;
+  const int nqb = (seq_len + kRowsPerCta - 1) / kRowsPerCta;
+  if (nqb * nbh > 0x7FFFFFFFLL || tiles > 0x7FFFFFFFLL) return HalfPlan{false, 1};
+  const TailPlan tp = plan_tail(nqb, (int)nbh, nkb, kSlots, split, 0);
+  const double block = nkb + kCtaCostBlocks;
+  double full = block * ((tp.prefix_wgs + kSlots - 1) / kSlots);
+  if (tp.parts > 0) {
+    const long long rounds = (tp.parts + kSlots - 1) / kSlots;
+    full += rounds * ((nkb + tp.split_ways - 1) / tp.split_ways + kCtaCostBlocks) + kMergeCostBlocks +
+            (tp.parts + kPartsPerRecordBlock - 1) / kPartsPerRecordBlock + kFullSplitExtra;
+  }
+  if (tiles <= kNumCUs) {
+    int G = 1;
+    double best = kCtaCostBlocks + 0.6 * nkb;
+    for (int gw = 2; split && gw <= kNumCUs / tiles && nkb / gw >= 2; ++gw) {
+      const double span = kCtaCostBlocks + 0.6 * ((nkb + gw - 1) / gw) + kHalfSplitCost +
+                          (double)tiles * gw / kHalfPartsPerBlock;
+      if (span < best) {
+        best = span;
+        G = gw;
+      }
+    }
+    return HalfPlan{best < full, G};
+  }
+  const long long per_cu = (tiles + kNumCUs - 1) / kNumCUs;
+  const double half = block * ((nkb <= 4 ? 0.96 : 1.06) * (per_cu / 2) + 0.6 * (per_cu % 2));
+  return HalfPlan{half < full, 1};
+}
+
 // VROW: v_or_vt is V itself (moonmath_attention_forward_direct), else V_t.
 template <int MODE, bool VROW>
 int launch_fwd(const void* q, const void* k, const void* v_or_vt, void* out, int batch, int heads, int seq_len,
@@ -1347,9 +1487,28 @@ int launch_fwd(const void* q, const void* k, const void* v_or_vt, void* out, int
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
   }
+  if constexpr (VROW) {
+    const HalfPlan hp = force_ways > 1 ? HalfPlan{false, 1} : plan_half(seq_len, nbh, p.nkb, workspace != nullptr);
+    if (hp.half) {
+      p.nqb = (seq_len + kHalfRows - 1) / kHalfRows;
+      const int tiles = p.nqb * (int)nbh;
+      p.split_ways = hp.split_ways;
+      p.prefix_wgs = hp.split_ways > 1 ? 0 : tiles;
+      p.rec_rows = kHalfRows;
+      p.rec_parts = tiles * hp.split_ways;
+      hipLaunchKernelGGL((attn_half_kernel<MODE>), dim3(tiles * hp.split_ways), dim3(kHalfThreads), 0, st, p);
+      if (hp.split_ways > 1)
+        hipLaunchKernelGGL((attn_merge_kernel<MODE>), dim3(tiles * (kHalfRows * kD / 4 / kMergeThreads)),
+                           dim3(kMergeThreads), 0, st, p, kHalfRows);
+      const hipError_t e = hipGetLastError();
+      return e == hipSuccess ? 0 : (int)e;
+    }
+  }
   const TailPlan tp = plan_tail(p.nqb, (int)nbh, p.nkb, kSlots, workspace != nullptr, force_ways);
   p.prefix_wgs = tp.prefix_wgs;
   p.split_ways = tp.split_ways;
+  p.rec_rows = kMaxRows;
+  p.rec_parts = kMaxParts;
   const int grid = tp.prefix_wgs + tp.parts;
   hipLaunchKernelGGL((attn_fwd_kernel<MODE, VROW>), dim3(grid), dim3(kThreads), 0, st, p);
   if (tp.parts > 0) {
@@ -1518,6 +1677,20 @@ int moonmath_attention_forward_lite_direct(const void* q, const void* k, const v
   if (!launch) return 10;
   return launch(q, k, v, out, batch, heads, seq_len, seq_len_kv, head_dim, read_list, write_list, must_do_list,
                 threshold, phase, layout, workspace, stream);
+}
+
+size_t moonmath_attention_direct_workspace(int batch, int heads, int seq_len, int seq_len_kv) {
+  if (batch <= 0 || heads <= 0 || seq_len <= 0 || seq_len_kv <= 0) return 0;
+  const long long nbh = (long long)batch * heads;
+  const int nkb = (seq_len_kv + kKvBlock - 1) / kKvBlock;
+  const HalfPlan hp = plan_half(seq_len, nbh, nkb, true);
+  if (hp.half) {
+    const size_t parts = (size_t)((seq_len + kHalfRows - 1) / kHalfRows) * nbh * hp.split_ways;
+    return hp.split_ways > 1 ? parts * kHalfRows * (kD + 2) * sizeof(float) : 0;
+  }
+  const int nqb = (seq_len + kRowsPerCta - 1) / kRowsPerCta;
+  if (nqb * nbh > 0x7FFFFFFFLL) return 0;
+  return plan_tail(nqb, (int)nbh, nkb, kSlots, true, 0).parts > 0 ? kWorkspaceBytes : 0;
 }
 
 int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv) {

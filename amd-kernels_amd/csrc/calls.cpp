@@ -37,6 +37,7 @@ struct Abi {
   X(launch_v_transpose_rtne)                                                                               \
   X(moonmath_attention_forward_ex)                                                                         \
   X(moonmath_attention_forward_direct)                                                                     \
+  X(moonmath_attention_direct_workspace)                                                                   \
   X(moonmath_attention_forward_lite_direct)                                                                \
   X(moonmath_attention_prefers_direct)                                                                     \
   X(moonmath_attention_plan_tail)                                                                          \
@@ -200,16 +201,20 @@ PyObject* forward(PyObject*, PyObject* const* x, Py_ssize_t n) {
       if (!a.own_out) a.out = at::empty_like(a.q);
       void* stream = stream_of(a.q);
       Tensor vt, ws;
-      int plan[4];
-      check_rc(abi.moonmath_attention_plan_tail(a.B, a.H, a.Sq, a.Skv, 1, 0, plan), "moonmath_attention_plan_tail");
-      if (plan[3] > 0) ws = bytes(abi.tail_workspace_bytes_rtne(), a.q);
       const bool direct = abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
-      if (!direct) {
+      size_t ws_bytes = 0;
+      if (direct) {
+        ws_bytes = abi.moonmath_attention_direct_workspace(a.B, a.H, a.Sq, a.Skv);
+      } else {
+        int plan[4];
+        check_rc(abi.moonmath_attention_plan_tail(a.B, a.H, a.Sq, a.Skv, 1, 0, plan), "moonmath_attention_plan_tail");
+        if (plan[3] > 0) ws_bytes = abi.tail_workspace_bytes_rtne();
         vt = bytes(abi.moonmath_attention_vt_bytes(a.B, a.H, a.Skv), a.q);
         check_rc(abi.launch_v_transpose_rtne(a.v.data_ptr(), vt.data_ptr(), a.B * a.H * a.Skv, a.Skv, a.H, a.layout,
                                              stream),
                  "launch_v_transpose");
       }
+      if (ws_bytes) ws = bytes(ws_bytes, a.q);
       check_rc((direct ? abi.moonmath_attention_forward_direct : abi.moonmath_attention_forward_ex)(
                    a.q.data_ptr(), a.k.data_ptr(), direct ? a.v.data_ptr() : vt.data_ptr(), a.out.data_ptr(), a.B, a.H,
                    a.Sq, a.Skv, 128, a.layout, a.mode, ws.defined() ? ws.data_ptr() : nullptr, 0, stream),

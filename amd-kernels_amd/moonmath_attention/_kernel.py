@@ -129,13 +129,16 @@ def _forward_device(q, k, v, out, round_mode, layout):
         # MOONMATH_FORCE_SPLIT=G forces G parts on the last round (test hook).
         force = int(os.environ.get("MOONMATH_FORCE_SPLIT", "0") or 0)
         enable = os.environ.get("MOONMATH_NO_TAIL") is None
-        ws = None
+        direct = bool(lib.moonmath_attention_prefers_direct(B, H, Sq, Skv))
+        ws_bytes = 0
         if enable:
-            plan = _lib.plan_tail(B, H, Sq, Skv, True, force)
-            if plan[3] > 0:
-                ws = torch.empty(lib.tail_workspace_bytes_rtne(), dtype=torch.uint8, device=dev)
+            if direct and force <= 1:
+                ws_bytes = lib.moonmath_attention_direct_workspace(B, H, Sq, Skv)
+            elif _lib.plan_tail(B, H, Sq, Skv, True, force)[3] > 0:
+                ws_bytes = lib.tail_workspace_bytes_rtne()
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         src, fn = v, lib.moonmath_attention_forward_direct
-        if not lib.moonmath_attention_prefers_direct(B, H, Sq, Skv):
+        if not direct:
             src = torch.empty(lib.moonmath_attention_vt_bytes(B, H, Skv) // 2, dtype=torch.bfloat16, device=dev)
             rc = getattr(lib, f"launch_v_transpose_{round_mode}")(
                 _lib.ptr(v), _lib.ptr(src), B * H * Skv, Skv, H, lay, stream

@@ -34,6 +34,7 @@ SIGNATURES.update({
     "moonmath_attention_forward_direct": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _p]),
     "moonmath_attention_forward_lite_direct": (
         _i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _f, _i, _i, _i, _p, _p]),
+    "moonmath_attention_direct_workspace": (_sz, [_i, _i, _i, _i]),
     "moonmath_attention_prefers_direct": (_i, [_i, _i, _i, _i]),
     "moonmath_attention_plan_tail": (_i, [_i, _i, _i, _i, _i, _i, _ip]),
     "moonmath_attention_geometry": (_i, [_ip]),

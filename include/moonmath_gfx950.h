@@ -104,7 +104,10 @@ int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t,
 /* The same forward, and the same LiteAttention forward, on V itself
  * ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit for bit.
  * moonmath_attention_prefers_direct: 1 where that is the faster one (a V_t pass
- * costs more than the transposing reads). */
+ * costs more than the transposing reads). workspace of the dense one:
+ * moonmath_attention_direct_workspace bytes (0: none needed), or
+ * tail_workspace_bytes_<mode>() bytes with force_split_ways > 1, or NULL (no
+ * split). */
 int moonmath_attention_forward_direct(const void* q, const void* k, const void* v, void* out, int batch, int heads,
                                       int seq_len, int seq_len_kv, int head_dim, int layout, int round_mode,
                                       void* workspace, int force_split_ways, void* stream);
@@ -113,6 +116,7 @@ int moonmath_attention_forward_lite_direct(const void* q, const void* k, const v
                                            const void* read_list, void* write_list, const void* must_do_list,
                                            float threshold, int phase, int layout, int round_mode, void* workspace,
                                            void* stream);
+size_t moonmath_attention_direct_workspace(int batch, int heads, int seq_len, int seq_len_kv);
 int moonmath_attention_prefers_direct(int batch, int heads, int seq_len, int seq_len_kv);
 
 /* Tail split plan -> out4 = {prefix CTAs, tail, split ways G, parts}. Pure host.

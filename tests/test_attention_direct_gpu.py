@@ -78,6 +78,36 @@ def test_lite_direct_equals_vt(B, H, Sq, Skv, layout):
             assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and torch.equal(x, y)
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("B,H,Sq,Skv", [
+    (1, 1, 1, 1), (1, 2, 127, 64), (1, 2, 128, 65), (2, 3, 129, 128), (1, 3, 250, 700),   # one half CTA per CU
+    (2, 12, 3000, 300), (2, 24, 2048, 2048),                                             # two per CU
+    (1, 2, 100, 500), (1, 8, 128, 2000), (1, 1, 129, 4033), (1, 2, 1999, 2000)])         # split parts
+def test_half_ctas(B, H, Sq, Skv, layout):
+    """Calls that the launcher gives to half CTAs (with a workspace: split where
+    it pays) against the 256-row CTAs of the V_t forward. Unsplit they are the
+    same computation, bit for bit; split sums add in another order: 2 bf16 units
+    in the last place of values up to 4."""
+    g = torch.Generator(device=DEV).manual_seed(Sq + Skv)
+    shape = (lambda s: (B, s, H, 128)) if layout else (lambda s: (B, H, s, 128))
+    q, k, v = (torch.randn(shape(s), generator=g, device=DEV).bfloat16() for s in (Sq, Skv, Skv))
+    lib, p, st = _lib.lib, _lib.ptr, _lib.stream_ptr(DEV)
+    nbytes = lib.moonmath_attention_direct_workspace(B, H, Sq, Skv)
+    for mode in range(3):
+        want = _run("moonmath_attention_forward_ex", q, k, v, B, H, Sq, Skv, layout, mode, 0)
+        for ws in (None, torch.empty(max(1, nbytes), dtype=torch.uint8, device=DEV)):
+            if ws is not None and nbytes == 0:
+                continue
+            out = torch.full_like(q, float("nan"))
+            assert lib.moonmath_attention_forward_direct(p(q), p(k), p(v), p(out), B, H, Sq, Skv, 128, layout, mode,
+                                                         p(ws), 0, st) == 0
+            torch.cuda.synchronize()
+            if ws is None:
+                assert torch.equal(out.view(torch.int16), want.view(torch.int16)), mode
+            else:
+                assert (out.float() - want.float()).abs().max() <= 2 * 2.0 ** -6, mode
+
+
 def test_direct_argument_codes():
     nul = ctypes.c_void_p(0)
     f = _lib.lib.moonmath_attention_forward_direct
