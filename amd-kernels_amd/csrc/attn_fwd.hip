@@ -10,7 +10,7 @@
 //    S^T = K Q^T (A = K fragment, B = Q fragment), so each lane owns one query
 //    column and 16 kv rows per 32x32 tile; P^T then feeds O^T = V^T P^T as the
 //    B operand straight from registers (no shuffle).
-//  * K and V (up to 12288 query rows, see prefers_direct) or a pre-transposed
+//  * K and V (up to 8192 query rows, see prefers_direct) or a pre-transposed
 //    V_t (more) are staged through LDS with 16-byte global->LDS DMA
 //    (global_load_lds_dwordx4) in 4-slot rings, two blocks of lead. Every DMA is inline asm, waited for by explicit vmcnt waits: with
 //    one the compiler can see in flight, its wait counting turns every LDS
@@ -1478,9 +1478,11 @@ int launch_fwd(const void* q, const void* k, const void* v_or_vt, void* out, int
   if ((long long)p.nqb * nbh > 0x7FFFFFFFLL) return 9;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const long long items = (long long)p.nqb * nbh;
-  if (p.nkb <= kShortMaxBlocks && items > kSlots && force_ways <= 1 && short_kv_enabled()) {
-    // Short KV: one persistent CTA per CU (no tail split: nkb is far below the
-    // planner's minimum).
+  // Short KV: one persistent CTA per CU (no tail split: nkb is far below the
+  // planner's minimum), from three items a CTA on where half CTAs can take the
+  // rest: (2,24,4096) x 77 27.5 us against 30.6 with half CTAs, (2,24,8192) x 77
+  // 49.1 against 62.3; (1,24,4096) x 64, two items a CTA, 15.4 against 13.7.
+  if (p.nkb <= kShortMaxBlocks && items > (VROW ? 2 : 1) * kSlots && force_ways <= 1 && short_kv_enabled()) {
     const int per_cta = (int)((items + kSlots - 1) / kSlots);
     const int grid = (int)((items + per_cta - 1) / per_cta);
     hipLaunchKernelGGL((attn_short_kernel<MODE, VROW>), dim3(grid), dim3(kThreads), 0, st, p, per_cta);
@@ -1544,9 +1546,10 @@ int launch_mode(const void* q, const void* k, const void* v, void* out, int batc
 // reads ~1.5% of a CTA's main loop, so the line depends on the q rows that share
 // a V. Measured (V_t pass + kernel -> direct, us): (1,2,256) 14.4 -> 12.0,
 // (1,24,1531) 47.3 -> 39.5, (2,24,8192) x 77 55.3 -> 49.8, (2,24,4097) x 512 71.2
-// -> 66.8, (2,24,4096) 349 -> 337, (2,24,8192) 1412 -> 1399; (1,32,16384) 3628 ->
-// 3636, (2,24,16384) x 2048 748 -> 756, (2,8,32768) x 4096 929 -> 941.
-constexpr int kDirectMaxSq = 12288;
+// -> 66.8, (2,24,8192) x 512 132.3 -> 128.8, (2,24,4096) 349 -> 337, (2,24,8192)
+// 1340 -> 1338; (1,16,10519) 777 -> 780, (1,32,16384) 3628 -> 3636, (2,24,16384) x
+// 2048 748 -> 756, (2,8,32768) x 4096 929 -> 941.
+constexpr int kDirectMaxSq = 8192;
 bool prefers_direct(int seq_len) { return seq_len <= kDirectMaxSq; }
 
 // LiteAttention launcher (reference launch_attention_forward_lite,
