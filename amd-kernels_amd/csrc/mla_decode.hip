@@ -85,12 +85,13 @@ __device__ __forceinline__ int merge_out_row(const Params& p, int b) {
 
 // Merge of the split requests' records, 128 threads (4 output dims each) times
 // GROUPS per query row; group g adds parts g, g + GROUPS, ... and the groups'
-// sums meet in LDS. A thread's parts cost a round of memory latency per batch of
-// 8: four groups for many parts, as long as the rows are few (with many, latency
-// is covered and four times the threads only cost). Whole calls, one -> four
-// groups: 16 rows in 33 parts 15.1 -> 12.5 us, 128 rows in 33 parts 21.4 -> 20.8;
-// 1024 rows in 17 parts 26.9 -> 31.8, 2048 rows in 9 parts 41.1 -> 45.5, 1024 rows
-// in 5 parts 38.3 -> 41.6.
+// sums meet in LDS, each under the max its group has seen. A thread's parts cost
+// a round of memory latency per batch of 8: eight groups for many parts, as long
+// as the rows are few (with many, latency is covered and the threads only cost).
+// Whole calls, one -> four -> eight groups: 16 rows in 33 parts 15.1 -> 12.5 ->
+// 11.6 us, 128 rows in 17 parts 16.1 with four and eight; one -> four: 1024 rows
+// in 17 parts 26.9 -> 31.8, 2048 rows in 9 parts 41.1 -> 45.5, 1024 rows in 5
+// parts 38.3 -> 41.6.
 constexpr int kMergeWideParts = 8;
 constexpr int kMergeWideRows = 256;
 template <int GROUPS>
@@ -113,8 +114,8 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS) void mla_merge_ke
   auto ml_at = [&](int j) { return ml + (((size_t)rec0 + j) * p.qrows + qrow) * 2; };
   float M = -__builtin_inff(), L = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (GROUPS == 1 && nparts <= kMergeBatch) {
-    merge_batch(0, 1, nparts, o_at, ml_at, true, M, acc, L);
+  if (nparts <= kMergeBatch * GROUPS) {
+    merge_batch(grp, GROUPS, nparts, o_at, ml_at, true, M, acc, L);  // under the group's own max
   } else {
     // The row's max by the wave: lane l looks at parts l, l + 64, ...
     for (int j = tid & 63; j < nparts; j += 64) M = fmaxf(M, ml_at(j)[0]);
@@ -124,19 +125,26 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS) void mla_merge_ke
       merge_batch(j0, GROUPS, nparts, o_at, ml_at, false, M, acc, L);
   }
   if constexpr (GROUPS > 1) {
-    __shared__ f32x4 part_o[GROUPS - 1][128];
-    __shared__ float part_l[GROUPS - 1];
-    if (grp > 0) {
-      part_o[grp - 1][cell] = acc;
-      if (cell == 0) part_l[grp - 1] = L;
+    __shared__ f32x4 part_o[GROUPS][128];
+    __shared__ float part_m[GROUPS], part_l[GROUPS];
+    part_o[grp][cell] = acc;
+    if (cell == 0) {
+      part_m[grp] = M;
+      part_l[grp] = L;
     }
     __syncthreads();
     if (grp > 0) return;
 #pragma unroll
-    for (int k = 0; k < GROUPS - 1; ++k) {
+    for (int k = 1; k < GROUPS; ++k) M = fmaxf(M, part_m[k]);
+    L = 0.f;
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < GROUPS; ++k) {
+      const float wt = part_weight(part_m[k], M);
       const f32x4 o = part_o[k][cell];
-      acc += o;
-      L += part_l[k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(wt, o[e], acc[e]);
+      L = __builtin_fmaf(wt, part_l[k], L);
     }
   }
   // Non-temporal: written once, read by no later kernel of the call (H=16:
@@ -318,7 +326,7 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   if (p.parts > 1) {
     const long long rows_all = (long long)B * p.qrows;
     if (p.parts > kMergeWideParts && rows_all <= kMergeWideRows)
-      hipLaunchKernelGGL(mla_merge_kernel<4>, dim3((unsigned)rows_all), dim3(512), 0, st, p);
+      hipLaunchKernelGGL(mla_merge_kernel<8>, dim3((unsigned)rows_all), dim3(1024), 0, st, p);
     else
       hipLaunchKernelGGL(mla_merge_kernel<1>, dim3((unsigned)((rows_all + 1) / 2)), dim3(256), 0, st, p);
   }
