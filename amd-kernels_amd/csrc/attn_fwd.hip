@@ -1355,6 +1355,15 @@ constexpr int kMinBlocksPerPart = 4;
 constexpr int kMergeCostBlocks = 3;
 constexpr int kCtaCostBlocks = 4;
 constexpr int kPartsPerRecordBlock = 64;
+// A last round of more than half the slots can only be split over several rounds,
+// and what that replaces is a round that leaves CUs idle: the chip is held by its
+// power limit, so the busy ones run faster (a block 1.28 us with 144 CTAs, 1.41 with
+// 192, 1.56 with 224, 1.68 with 256), while the records of several rounds cost more
+// (40 per block of time). Measured on 8 heads, unsplit / split as planned without
+// this: 144 CTAs of 48 blocks 67.7 / 80.7 us, 160 68.1 / 85.5, 192 of 96 141 / 169,
+// 192 of 192 276 / 293, 200 after a full round, 192 blocks 619 / 649; still worth
+// it: 144 CTAs of 192 blocks 252 / 231, 160 255 / 245.
+constexpr int kPartsPerRecordBlockRounds = 40;
 
 struct TailPlan {
   int prefix_wgs, tail, split_ways, parts;
@@ -1384,12 +1393,20 @@ TailPlan plan_tail(int nqb, int nbh, int nkb, int slots, bool enable, int force_
   }
   if (tail == 0 || tail > slots * 19 / 20 || nkb < kMinKvBlocksToSplit) return none;
   int G = 1;
-  long long best = (long long)nkb + kCtaCostBlocks;
+  // In percent of a block. A round of n < slots CTAs that is split over more than
+  // one round: its blocks take 45 + 55 n / slots of a full round's.
+  const bool one_round = 2 * tail <= slots;
+  auto pct = [&](int n) { return one_round || n == 0 ? 100 : 45 + 55 * n / slots; };
+  long long best = (long long)nkb * pct(tail) + 100 * kCtaCostBlocks;
   for (int gw = 2; gw <= kMaxParts / tail && nkb / gw >= kMinBlocksPerPart; ++gw) {
-    const long long rounds = ((long long)tail * gw + slots - 1) / slots;
+    const int parts = tail * gw;
+    if (one_round && parts > slots) break;
+    const long long rounds = (parts + slots - 1) / slots;
     const long long per_part = (nkb + gw - 1) / gw;
-    const long long records = ((long long)tail * gw + kPartsPerRecordBlock - 1) / kPartsPerRecordBlock;
-    const long long span = rounds * (per_part + kCtaCostBlocks) + kMergeCostBlocks + records;
+    const int per_block = one_round ? kPartsPerRecordBlock : kPartsPerRecordBlockRounds;
+    const long long records = (parts + per_block - 1) / per_block;
+    const long long span = ((rounds - 1) * 100 + pct(parts % slots)) * per_part +
+                           100 * (rounds * kCtaCostBlocks + kMergeCostBlocks + records);
     if (span < best) {
       best = span;
       G = gw;

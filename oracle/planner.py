@@ -11,7 +11,10 @@ G <= max_parts/tail with nkb/G >= 4, against nkb + 3 unsplit.
 1 CTA of 256 rows): the same search and limits, from 16 kv blocks, with the
 cost of a CTA's prologue and epilogue (4 blocks) per round and of the parts'
 fp32 records (one block per 64 parts):
-unsplit nkb + 4; G parts rounds * (ceil(nkb/G) + 4) + 3 + ceil(tail*G/64).
+unsplit nkb + 4; G parts, in one round, ceil(nkb/G) + 4 + 3 + ceil(tail*G/64).
+A tail of more than half the slots can only be split over several rounds; there a
+round of n CTAs takes (45 + 55n/slots)% of a full round's time per block (a partly
+idle chip clocks higher) and the records one block per 40 parts.
 """
 
 REFERENCE_MIN_KV_BLOCKS = 48
@@ -20,6 +23,7 @@ MIN_BLOCKS_PER_PART = 4
 MERGE_COST = 3
 CTA_COST = 4
 PARTS_PER_RECORD_BLOCK = 64
+PARTS_PER_RECORD_BLOCK_ROUNDS = 40
 
 
 def _ceil(a, b):
@@ -56,11 +60,21 @@ def plan_tail(nqb, nbh, nkb, slots, max_parts, enable=True):
     tail = wgs % slots
     if tail == 0 or tail > slots * 19 // 20 or nkb < MIN_KV_BLOCKS:
         return none
-    best_g, best = 1, nkb + CTA_COST
+    one_round = 2 * tail <= slots
+
+    def pct(n):
+        return 100 if one_round or n == 0 else 45 + 55 * n // slots
+
+    best_g, best = 1, nkb * pct(tail) + 100 * CTA_COST
     g = 2
     while g <= max_parts // tail and nkb // g >= MIN_BLOCKS_PER_PART:
-        span = (_ceil(tail * g, slots) * (_ceil(nkb, g) + CTA_COST) + MERGE_COST
-                + _ceil(tail * g, PARTS_PER_RECORD_BLOCK))
+        parts = tail * g
+        if one_round and parts > slots:
+            break
+        rounds = _ceil(parts, slots)
+        per_block = PARTS_PER_RECORD_BLOCK if one_round else PARTS_PER_RECORD_BLOCK_ROUNDS
+        span = (((rounds - 1) * 100 + pct(parts % slots)) * _ceil(nkb, g)
+                + 100 * (rounds * CTA_COST + MERGE_COST + _ceil(parts, per_block)))
         if span < best:
             best, best_g = span, g
         g += 1
