@@ -102,7 +102,8 @@ int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t,
                                   void* workspace, int force_split_ways, void* stream);
 
 /* The same forward, and the same LiteAttention forward, on V itself
- * ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit for bit.
+ * ([B,H,Skv,128] or [B,Skv,H,128], no V_t), bit for bit where
+ * neither splits the keys.
  * moonmath_attention_prefers_direct: 1 where that is the faster one (a V_t pass
  * costs more than the transposing reads). workspace of the dense one:
  * moonmath_attention_direct_workspace bytes (0: none needed), or
@@ -169,7 +170,8 @@ int launch_mla_decode_a16w8_paged_dev(const void* q_lat, const void* q_pe, const
  * live in a 64.3 MiB device array of the library (held on each GPU the library
  * runs on until the process ends); the call performs no allocation. Limit:
  * B * parts * R <= 32768 split-record rows once parts is clamped as in the
- * workspace launcher (parts 1 needs none), R = H * q_len, rounded up to a
+ * workspace launcher and to 64 (parts 1 needs none; of more than 64 parts as many
+ * run as the array holds), R = H * q_len, rounded up to a
  * multiple of 32 when 96 <= H * q_len <= 128; else returns -9 with nothing
  * launched. Calls that overlap on one GPU share the array and race: serialise
  * them (one stream, or events). */
