@@ -1,6 +1,6 @@
 // Absorbed-MLA decode for small query blocks (H * q_len <= 16, e.g. DeepSeek-V3's
 // 128 heads split over 8 GPUs) on MI355X (gfx950). Same contract, split plan,
-// records and numerics as mla_decode_kernel (reference csrc/mla_decode_a16w8.hip
+// records and numerics as the 64-row kernel (reference csrc/mla_decode_a16w8.hip
 // :183-754, csrc/mla_decode_a16w8_multiq.hip:282-856). With at most 16 query
 // rows the decode is bound by HBM: besides streaming the KV, the time goes to
 // per-CTA set-up and, in a kernel whose waves split the tokens, to merging the
