@@ -187,11 +187,14 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
       tok = tok < kv_hi ? tok : kv_hi - 1;
       dma4_opaque(p.table ? p.table + slot0 + tok / kPage : p.kv_indices + slot0 + tok, idx + 256 * (q & 1));
     };
-    // Slot of token i of this wave's share of tile j.
+    // Slot of token i of this wave's share of tile j; past the part's end that of
+    // its last token (a page's rows beyond it may hold anything, and 0 x NaN in
+    // PV is not 0).
     auto idx_at = [&](int j) -> int {
       if constexpr (PAGED) {
         const int v = *reinterpret_cast<const int*>(idx + 64 * (j & 7) + 4 * i);
-        return p.table ? page_slot(p, v) + kCSubTok * wave + i : v;
+        const int last = kv_hi - 1 - (kv_lo + kCTileTok * j), tok = kCSubTok * wave + i;
+        return p.table ? page_slot(p, v) + (tok < last ? tok : last) : v;
       } else {
         return 0;
       }

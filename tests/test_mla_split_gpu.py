@@ -163,3 +163,39 @@ def test_noalloc_shares_its_array_beyond_64_parts():
         outs.append(o)
     assert not torch.isnan(outs[0].float()).any()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [1, 70])
+@pytest.mark.parametrize("H,q_len", [(16, 1), (4, 4), (32, 1), (64, 1), (16, 4), (128, 1)])
+def test_no_row_outside_the_requests_is_read(H, q_len, parts):
+    """Every cache row that no token owns holds NaN codes (a pool from
+    torch.empty, a recycled page): the rest of a request's last page, and pages
+    of no request. Block tables and flat slots give the same bits, with no NaN,
+    at lengths around each wave's 8 or 16 tokens of a last tile."""
+    lens = [1, 7, 8, 9, 15, 16, 17, 47, 48, 49, 56, 57, 63, 64, 65, 130, 177, 700, 1025]
+    B, most = len(lens), -(-max(lens) // 64)
+    num_blocks = sum(-(-n // 64) for n in lens) + 3
+    g = torch.Generator().manual_seed(101)
+    order = torch.randperm(num_blocks, generator=g).tolist()
+    bits = torch.full((num_blocks * 64, QK), 0x7F, dtype=torch.uint8)
+    rows = rand_kv_rows(sum(lens), 101).view(torch.uint8)
+    table = torch.full((B, most), order[-1], dtype=torch.int32)
+    slots = []
+    for b, n in enumerate(lens):
+        pages = [order.pop(0) for _ in range(-(-n // 64))]
+        table[b, :len(pages)] = torch.tensor(pages, dtype=torch.int32)
+        slots += [pages[t // 64] * 64 + t % 64 for t in range(n)]
+    bits[torch.tensor(slots)] = rows
+    pool = _d(bits.view(torch.float8_e4m3fn).view(num_blocks, 64, QK))
+    idx = _d(torch.tensor(slots, dtype=torch.int32))
+    indptr = _d(torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32))
+    n = _d(torch.tensor(lens, dtype=torch.int32))
+    q_lat, q_pe = (_d(t) for t in rand_q(B, q_len, H, 101))
+    flat, blocks = (torch.full((B, q_len, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ma.mla_decode_a16w8_paged_dev(q_lat, q_pe, pool.view(-1, 1, QK), flat, n, None, idx, indptr, parts, SCALE_576,
+                                  KV_SCALE)
+    ma.mla_decode_a16w8_paged_blocks(q_lat, q_pe, pool, blocks, n, _d(table), parts, SCALE_576, KV_SCALE)
+    torch.cuda.synchronize()
+    assert not torch.isnan(flat.float()).any()
+    assert torch.equal(blocks.view(torch.int16), flat.view(torch.int16))
