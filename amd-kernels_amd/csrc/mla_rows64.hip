@@ -527,7 +527,9 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
                 const float M = fmaxf(fmaxf(rm[0], rm[kRRows]), fmaxf(rm[2 * kRRows], rm[3 * kRRows]));
                 row_m = (M == -__builtin_inff()) ? M : __builtin_ceilf(M * c);
               }
-              const float neg_m = (row_m == -__builtin_inff()) ? 0.f : -row_m;
+              // No finite score in the first tile (nor a token, where the window ends
+              // before it): a later one gives p = inf, which asks for the exact max.
+              const float neg_m = (row_m == -__builtin_inff()) ? -kNegFltMax : -row_m;
               float pe[8];
               if constexpr (kPV) {
 #pragma unroll

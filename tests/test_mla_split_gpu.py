@@ -199,3 +199,33 @@ def test_no_row_outside_the_requests_is_read(H, q_len, parts):
     torch.cuda.synchronize()
     assert not torch.isnan(flat.float()).any()
     assert torch.equal(blocks.view(torch.int16), flat.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [1, 70])
+@pytest.mark.parametrize("H", [16, 32, 64, 128])
+def test_scores_of_minus_infinity_before_finite_ones(H, parts):
+    """Scores that overflow to -inf over a part's first tiles weigh nothing: the
+    result is that of the tokens after them. (Queries of 2^120 in one dim, where
+    those tokens hold -448, and 0 elsewhere in it.)"""
+    S, cut = 700, 150
+    kv = rand_kv_rows(S, 103).float()
+    kv[:, 5] = 0.0
+    kv[:cut, 5] = -448.0
+    q_lat, q_pe = (t[:, 0].contiguous() for t in rand_q(1, 1, H, 103))
+    q_lat[..., 5] = 2.0 ** 120
+    pool = _d(kv.to(torch.float8_e4m3fn).view(S, 1, QK))
+    outs = []
+    for lo in (0, cut):
+        o = torch.full((1, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+        idx = _d(torch.arange(lo, S, dtype=torch.int32))
+        n, indptr = (_d(torch.tensor(t, dtype=torch.int32)) for t in ([S - lo], [0, S - lo]))
+        ma.mla_decode_a16w8_paged_dev(_d(q_lat), _d(q_pe), pool, o, n, None, idx, indptr, parts, SCALE_576, KV_SCALE)
+        outs.append(o.float())
+    torch.cuda.synchronize()
+    # The two place tiles differently: fp32 sums in another order, then one bf16
+    # rounding each (2^-8 of a value, both sides), P's rounding unchanged up to
+    # the row max's power of two.
+    a, b = outs
+    assert torch.isfinite(a).all()
+    assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5).all()
