@@ -183,6 +183,14 @@ AttnArgs attn_args(PyObject* q, PyObject* k, PyObject* v, PyObject* out, PyObjec
   return a;
 }
 
+// Whether the call reads V itself: a kernel that gathers V while others of its
+// CTAs store `out` cannot have the two in one place, as a V_t pass before it can.
+bool direct_call(const AttnArgs& a) {
+  const auto at = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()); };
+  const bool apart = !a.own_out || at(a.out) + a.out.nbytes() <= at(a.v) || at(a.v) + a.v.nbytes() <= at(a.out);
+  return apart && abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
+}
+
 PyObject* attn_result(const AttnArgs& a, PyObject* out) {
   if (a.own_out) {
     Py_INCREF(out);
@@ -201,7 +209,7 @@ PyObject* forward(PyObject*, PyObject* const* x, Py_ssize_t n) {
       if (!a.own_out) a.out = at::empty_like(a.q);
       void* stream = stream_of(a.q);
       Tensor vt, ws;
-      const bool direct = abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
+      const bool direct = direct_call(a);
       size_t ws_bytes = 0;
       if (direct) {
         ws_bytes = abi.moonmath_attention_direct_workspace(a.B, a.H, a.Sq, a.Skv);
@@ -243,7 +251,7 @@ PyObject* forward_lite(PyObject*, PyObject* const* x, Py_ssize_t n) {
       if (!a.own_out) a.out = at::empty_like(a.q);
       void* stream = stream_of(a.q);
       const Tensor ws = bytes(abi.lite_workspace_bytes_rtne(a.B, a.H, a.Sq), a.q);
-      if (abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv)) {
+      if (direct_call(a)) {
         check_rc(abi.moonmath_attention_forward_lite_direct(
                      a.q.data_ptr(), a.k.data_ptr(), a.v.data_ptr(), a.out.data_ptr(), a.B, a.H, a.Sq, a.Skv, 128,
                      read.data_ptr(), write.data_ptr(), nullptr, threshold, phase, a.layout, a.mode, ws.data_ptr(),

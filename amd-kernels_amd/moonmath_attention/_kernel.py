@@ -31,7 +31,8 @@ def forward(
             ("bhsd") or (batch, seq_len, heads, head_dim) ("bshd"). Contiguous,
             head_dim = 128, any Sq / Skv >= 1. CPU tensors are moved to cuda:0
             and the result is returned on the CPU.
-        out: optional preallocated output (q's shape, bf16, contiguous, same device).
+        out: optional preallocated output (q's shape, bf16, contiguous, same device;
+            may be q or overlap v).
         round_mode: "rtna" (default), "rtne" or "rtz" -- the bf16 rounding of P
             and of the output.
         layout: "bhsd" (default) or "bshd".
@@ -116,6 +117,14 @@ def check_args(q, k, v, out, round_mode, layout):
     return B, H, Sq, Skv, int(bshd)
 
 
+def _direct(v, out, B, H, Sq, Skv):
+    """Whether the call reads V itself: a kernel that gathers V while others of its
+    CTAs store ``out`` cannot have the two in one place, as a V_t pass before it can."""
+    o0, v0 = out.data_ptr(), v.data_ptr()
+    apart = o0 + out.numel() * 2 <= v0 or v0 + v.numel() * 2 <= o0
+    return apart and bool(_lib.lib.moonmath_attention_prefers_direct(B, H, Sq, Skv))
+
+
 def _forward_device(q, k, v, out, round_mode, layout):
     B, H, Sq, Skv, lay = check_args(q, k, v, out, round_mode, layout)
     if out is None:
@@ -129,7 +138,7 @@ def _forward_device(q, k, v, out, round_mode, layout):
         # MOONMATH_FORCE_SPLIT=G forces G parts on the last round (test hook).
         force = int(os.environ.get("MOONMATH_FORCE_SPLIT", "0") or 0)
         enable = os.environ.get("MOONMATH_NO_TAIL") is None
-        direct = bool(lib.moonmath_attention_prefers_direct(B, H, Sq, Skv))
+        direct = _direct(v, out, B, H, Sq, Skv)
         ws_bytes = 0
         if enable:
             if direct and force <= 1:
@@ -231,7 +240,7 @@ def forward_lite(
             ws = torch.empty(getattr(lib, f"lite_workspace_bytes_{round_mode}")(B, H, Sq), dtype=torch.uint8,
                              device=dev)
         lists = (_lib.ptr(read_list), _lib.ptr(write_list), _lib.ptr(must_do_list), float(threshold), int(phase), lay)
-        if lib.moonmath_attention_prefers_direct(B, H, Sq, Skv):
+        if _direct(v, out, B, H, Sq, Skv):
             rc = lib.moonmath_attention_forward_lite_direct(
                 _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), B, H, Sq, Skv, 128, *lists, _MODES[round_mode],
                 _lib.ptr(ws), stream,

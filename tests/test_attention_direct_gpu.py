@@ -7,7 +7,9 @@ import ctypes
 import pytest
 import torch
 
+import moonmath_attention as ma
 from moonmath_attention import _lib
+from test_calls import _python_path
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -114,3 +116,64 @@ def test_direct_argument_codes():
     assert f(nul, nul, nul, nul, 0, 1, 1, 1, 128, 0, 0, nul, 0, nul) == 1
     assert f(nul, nul, nul, nul, 1, 1, 1, 1, 128, 0, 0, nul, 0, nul) == 8
     assert f(nul, nul, nul, nul, 1, 1, 1, 1, 128, 0, 9, nul, 0, nul) == 10
+
+
+def _ramp_lists(B, H, Sq, Skv):
+    """A full read list and an empty list to write."""
+    nqb, nkb = -(-Sq // 256), -(-Skv // 64)
+    pair = torch.zeros(2, B, H, nqb, nkb + 2, dtype=torch.int16, device=DEV)
+    pair[0, ..., :3] = torch.tensor([2, nkb - 1, -1], dtype=torch.int16)
+    return pair
+
+
+def _vt_result(monkeypatch, fn):
+    """`fn` by the Python path with a V_t pass."""
+    with monkeypatch.context() as m:
+        _python_path(m)
+        m.setattr(_lib.lib, "moonmath_attention_prefers_direct", lambda *a: 0)
+        out = fn()
+        torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("B,H,S,shift", [(1, 2, 256, 0), (1, 3, 1000, 0), (2, 8, 2048, 0), (2, 24, 1531, 0),
+                                         (1, 3, 1000, 128), (2, 4, 1100, -256), (1, 2, 300, 128 * 599)])
+def test_out_may_overlap_v(B, H, S, shift, layout, native, monkeypatch):
+    """``out`` on V's own memory, or `shift` elements from it: V is read before
+    any of it is overwritten, in both forwards."""
+    g = torch.Generator(device=DEV).manual_seed(S)
+    shape = (B, H, S, 128) if layout == "bhsd" else (B, S, H, 128)
+    q, k, v0 = (torch.randn(shape, generator=g, device=DEV).bfloat16() for _ in range(3))
+    n = v0.numel()
+    for lite in (False, True):
+        def call(v, out, pair):
+            if lite:
+                return ma.forward_lite(q, k, v, pair[0], pair[1], threshold=-3.0, phase=1, out=out, layout=layout)
+            return ma.forward(q, k, v, out=out, layout=layout)
+
+        want_pair, pair = _ramp_lists(B, H, S, S), _ramp_lists(B, H, S, S)
+        want = _vt_result(monkeypatch, lambda: call(v0, None, want_pair))
+        buf = torch.empty(n + abs(shift), dtype=torch.bfloat16, device=DEV)
+        v, out = (buf[max(0, -s):][:n].view(shape) for s in (shift, -shift))
+        v.copy_(v0)
+        with monkeypatch.context() as m:
+            if not native:
+                _python_path(m)
+            assert call(v, out, pair) is out
+            torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(pair, want_pair)
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+def test_out_may_be_q(layout):
+    """Every CTA reads its query rows before it stores them, in both forwards."""
+    for B, H, S in ((1, 2, 256), (2, 24, 1531), (1, 3, 4097)):
+        g = torch.Generator(device=DEV).manual_seed(S)
+        shape = (B, H, S, 128) if layout == "bhsd" else (B, S, H, 128)
+        q, k, v = (torch.randn(shape, generator=g, device=DEV).bfloat16() for _ in range(3))
+        want = ma.forward(q, k, v, layout=layout)
+        q2 = q.clone()
+        assert torch.equal(ma.forward(q2, k, v, out=q2, layout=layout).view(torch.int16), want.view(torch.int16))
