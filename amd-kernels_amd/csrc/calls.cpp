@@ -184,11 +184,12 @@ AttnArgs attn_args(PyObject* q, PyObject* k, PyObject* v, PyObject* out, PyObjec
 }
 
 // Whether the call reads V itself: a kernel that gathers V while others of its
-// CTAs store `out` cannot have the two in one place, as a V_t pass before it can.
+// CTAs store `out` cannot have the two in one place, as a V_t pass before it can,
+// and its 16-byte gathers want V's rows aligned, as plain loads do not.
 bool direct_call(const AttnArgs& a) {
   const auto at = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()); };
   const bool apart = !a.own_out || at(a.out) + a.out.nbytes() <= at(a.v) || at(a.v) + a.v.nbytes() <= at(a.out);
-  return apart && abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
+  return apart && at(a.v) % 16 == 0 && abi.moonmath_attention_prefers_direct(a.B, a.H, a.Sq, a.Skv);
 }
 
 PyObject* attn_result(const AttnArgs& a, PyObject* out) {

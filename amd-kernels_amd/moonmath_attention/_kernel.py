@@ -119,10 +119,11 @@ def check_args(q, k, v, out, round_mode, layout):
 
 def _direct(v, out, B, H, Sq, Skv):
     """Whether the call reads V itself: a kernel that gathers V while others of its
-    CTAs store ``out`` cannot have the two in one place, as a V_t pass before it can."""
+    CTAs store ``out`` cannot have the two in one place, as a V_t pass before it can,
+    and its 16-byte gathers want V's rows aligned, as plain loads do not."""
     o0, v0 = out.data_ptr(), v.data_ptr()
     apart = o0 + out.numel() * 2 <= v0 or v0 + v.numel() * 2 <= o0
-    return apart and bool(_lib.lib.moonmath_attention_prefers_direct(B, H, Sq, Skv))
+    return apart and v0 % 16 == 0 and bool(_lib.lib.moonmath_attention_prefers_direct(B, H, Sq, Skv))
 
 
 def _forward_device(q, k, v, out, round_mode, layout):

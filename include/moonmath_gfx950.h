@@ -106,7 +106,8 @@ int moonmath_attention_forward_ex(const void* q, const void* k, const void* v_t,
  * neither splits the keys.
  * moonmath_attention_prefers_direct: 1 where that is the faster one (a V_t pass
  * costs more than the transposing reads). out must not overlap v, which is read
- * while out is stored (it may where V_t is read). workspace of the dense one:
+ * while out is stored, and v is 16-byte aligned (neither holds where V_t is
+ * read). workspace of the dense one:
  * moonmath_attention_direct_workspace bytes (0: none needed), or
  * tail_workspace_bytes_<mode>() bytes with force_split_ways > 1, or NULL (no
  * split). */

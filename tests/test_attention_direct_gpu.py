@@ -177,3 +177,34 @@ def test_out_may_be_q(layout):
         want = ma.forward(q, k, v, layout=layout)
         q2 = q.clone()
         assert torch.equal(ma.forward(q2, k, v, out=q2, layout=layout).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_v_off_a_16_byte_boundary(offset, native, monkeypatch):
+    """V as a view that starts `offset` elements into its buffer: read by plain
+    loads (the V_t pass), not by 16-byte gathers; the bits are those of an
+    aligned copy."""
+    B, H, S = 2, 3, 700
+    g = torch.Generator(device=DEV).manual_seed(offset)
+    q, k, v0 = (torch.randn(B, H, S, 128, generator=g, device=DEV).bfloat16() for _ in range(3))
+    v = torch.empty(v0.numel() + offset, dtype=torch.bfloat16, device=DEV)[offset:].view(v0.shape)
+    v.copy_(v0)
+    for lite in (False, True):
+        def call(v, pair):
+            if lite:
+                return ma.forward_lite(q, k, v, pair[0], pair[1], threshold=-3.0, phase=1)
+            return ma.forward(q, k, v)
+
+        want_pair, pair = _ramp_lists(B, H, S, S), _ramp_lists(B, H, S, S)
+        want = _vt_result(monkeypatch, lambda: call(v0, want_pair))
+        passes = []
+        with monkeypatch.context() as m:
+            if not native:
+                _python_path(m)
+                real = _lib.lib.launch_v_transpose_rtna
+                m.setattr(_lib.lib, "launch_v_transpose_rtna", lambda *a: passes.append(1) or real(*a))
+            got = call(v, pair)
+            torch.cuda.synchronize()
+        assert native or passes
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(pair, want_pair)
