@@ -50,6 +50,7 @@ struct Params {
   int workers;            // > 0: balanced split over this many units (see plan_work), 0: equal parts
   int qrows;              // H * q_len
   int rec_rows;           // O rows per split record (>= qrows)
+  int q_plain;            // the query rows are off a 16-byte boundary: plain loads instead of gathers
   float score_c;          // scale * kv_scale * log2(e), fp32
   float kv_scale;
 };
@@ -442,6 +443,13 @@ __device__ __forceinline__ Seg read_seg(const int* misc) {
 __device__ __forceinline__ void dma4_opaque(const void* gsrc, const char* lds_dst) {
   const uint32_t m0v = (uint32_t)(uintptr_t)(MM_LDS const char*)lds_dst;
   asm volatile("global_load_lds_dword %0, off" ::"v"(gsrc), "{m0}"(m0v) : "memory");
+}
+
+// 16 bytes from any address to LDS (`lds_dst`: this lane's), by plain loads.
+__device__ __forceinline__ void copy16_plain(const void* gsrc, char* lds_dst) {
+  u32x4 v;
+  __builtin_memcpy(&v, gsrc, 16);
+  *reinterpret_cast<u32x4*>(lds_dst) = v;
 }
 
 // Staging layout of one tile: token t's 576-byte row at t*576, its 16-byte

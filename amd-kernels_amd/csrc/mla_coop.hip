@@ -274,16 +274,24 @@ __global__ __launch_bounds__(kCThreads, 1) void mla_coop_kernel(Params p) {
     // slot 3 by whole-row DMAs behind tile 0, row rr's 16-byte chunk c at rr *
     // 1152 + 16 * (c ^ ((rr / 2) & 7)) (conflict-free fragment reads). Wave w
     // fetches rows 4w .. 4w+3; padding rows repeat the last row.
-    const char* qstage = lds + kCScratchOff;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
+    char* qstage = lds + kCScratchOff;
+    auto q_src = [&](int k) {
       const int pc = 64 * k + lane;
       const int rl = pc / 72, cs = pc - 72 * rl;
       const int rr = 4 * wave + rl;
       const int ch = cs ^ ((rr >> 1) & 7);
       const long long qoff = (long long)qb * p.qrows + (rr < p.qrows ? rr : p.qrows - 1);
-      const uint16_t* src = ch < 64 ? p.q_lat + qoff * kLat + 8 * ch : p.q_pe + qoff * kRope + 8 * (ch - 64);
-      if (k < 4 || lane < 32) dma16_opaque(src, qstage + 4608 * wave + 1024 * k);
+      return ch < 64 ? p.q_lat + qoff * kLat + 8 * ch : p.q_pe + qoff * kRope + 8 * (ch - 64);
+    };
+    if (p.q_plain) {
+#pragma unroll 1
+      for (int k = 0; k < 5; ++k)
+        if (k < 4 || lane < 32) copy16_plain(q_src(k), qstage + 4608 * wave + 1024 * k + 16 * lane);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    } else {
+#pragma unroll
+      for (int k = 0; k < 5; ++k)
+        if (k < 4 || lane < 32) dma16_opaque(q_src(k), qstage + 4608 * wave + 1024 * k);
     }
     // Tile 1 goes out behind them (tile 2 in body(0)) and stays in flight.
     if (ntiles > 1) {

@@ -312,6 +312,7 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   p.rec_rows = rec_rows_for(H, q_len);
   p.score_c = (float)((double)scale * (double)kv_scale * 1.4426950408889634);
   p.kv_scale = kv_scale;
+  p.q_plain = ((reinterpret_cast<uintptr_t>(q_lat) | reinterpret_cast<uintptr_t>(q_pe)) & 15) != 0;
   // Unit slots per XCD for the snake deal of units 0..U-1, U <= B * parts (the
   // kernel's split plan never exceeds that bound; CTAs past the real count exit).
   const long long umax = p.workers > 0 ? p.workers : (long long)B * p.parts;

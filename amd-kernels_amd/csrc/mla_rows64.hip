@@ -293,17 +293,22 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
     // rr's 16-byte chunk c at rr * 1152 + 16 * (c ^ ((rr / 2) & 7)): the fragment
     // reads are conflict-free. Wave w fetches rows 8w .. 8w+7.
     char* qstage = lds + kRTileBytes;
+    auto q_src = [&](int k) {
+      const int pc = 64 * k + lane;
+      const int rl = pc / 72, cs = pc - 72 * rl;
+      const int rr = 8 * wave + rl;
+      const int ch = cs ^ ((rr >> 1) & 7);
+      const int row = row0 + rr < p.qrows ? row0 + rr : p.qrows - 1;
+      const long long qoff = (long long)qb * p.qrows + row;
+      return ch < 64 ? p.q_lat + qoff * kLat + 8 * ch : p.q_pe + qoff * kRope + 8 * (ch - 64);
+    };
     if (wave < 4 * NRT) {
+      if (p.q_plain) {
+#pragma unroll 1
+        for (int k = 0; k < 9; ++k) copy16_plain(q_src(k), qstage + 9216 * wave + 1024 * k + 16 * lane);
+      } else {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        const int pc = 64 * k + lane;
-        const int rl = pc / 72, cs = pc - 72 * rl;
-        const int rr = 8 * wave + rl;
-        const int ch = cs ^ ((rr >> 1) & 7);
-        const int row = row0 + rr < p.qrows ? row0 + rr : p.qrows - 1;
-        const long long qoff = (long long)qb * p.qrows + row;
-        const uint16_t* src = ch < 64 ? p.q_lat + qoff * kLat + 8 * ch : p.q_pe + qoff * kRope + 8 * (ch - 64);
-        dma16_opaque(src, qstage + 9216 * wave + 1024 * k);
+        for (int k = 0; k < 9; ++k) dma16_opaque(q_src(k), qstage + 9216 * wave + 1024 * k);
       }
     }
     lds_reads_done_barrier_vm0();

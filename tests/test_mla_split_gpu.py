@@ -229,3 +229,36 @@ def test_scores_of_minus_infinity_before_finite_ones(H, parts):
     a, b = outs
     assert torch.isfinite(a).all()
     assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["q_lat", "q_pe", "both"])
+@pytest.mark.parametrize("H,q_len", [(5, 1), (16, 1), (33, 1), (128, 1), (16, 5)])
+def test_queries_off_a_16_byte_boundary(H, q_len, which):
+    """Views that start one element into their buffers: read by plain loads, the
+    bits are those of aligned copies."""
+    lens = [130, 1000, 64, 2500]
+    B = len(lens)
+    pool, idx, indptr = paged_pool(lens, 107)
+    q = [_d(t) for t in rand_q(B, q_len, H, 107)]
+
+    def off(t):
+        v = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape)
+        return v.copy_(t)
+
+    moved = [off(t) if which in (name, "both") else t for name, t in zip(("q_lat", "q_pe"), q, strict=True)]
+    n, pool, idx, indptr = _d(torch.tensor(lens, dtype=torch.int32)), _d(pool), _d(idx), _d(indptr)
+    slab = _d(rand_kv_rows(B * 300, 109).view(B, 300, QK))
+    outs = []
+    for ql, qp in (q, moved):
+        o = torch.full((3, B, q_len, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+        for i, parts in enumerate((1, 20)):
+            ma.mla_decode_a16w8_paged_dev(ql, qp, pool, o[i], n, None, idx, indptr, parts, SCALE_576, KV_SCALE)
+        if q_len == 1:
+            ma.mla_decode_a16w8(ql[:, 0], qp[:, 0], slab, o[2, :, 0], SCALE_576, KV_SCALE)
+        else:
+            ma.mla_decode_a16w8_multiq(ql, qp, slab, o[2], SCALE_576, KV_SCALE)
+        torch.cuda.synchronize()
+        outs.append(o)
+    assert not torch.isnan(outs[0].float()).any()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
