@@ -310,11 +310,17 @@ const Tensor& index_tensor(PyObject* o, const Tensor& q, int64_t least) {
 
 void* ptr_or_null(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
-// q_lat, q_pe, kv, o_lat, scale, kv_scale, multiq
+// The single-query ops take scale_p and use it nowhere, but refuse what is no number.
+void unused_scale_p(PyObject* o, bool multiq) {
+  if (!multiq) float_arg(o);
+}
+
+// q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p, multiq
 PyObject* mla_slab(PyObject*, PyObject* const* x, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    plain(n == 7);
-    const bool multiq = x[6] == Py_True;
+    plain(n == 8);
+    const bool multiq = x[7] == Py_True;
+    unused_scale_p(x[6], multiq);
     const MlaArgs a = mla_args(x[0], x[1], x[3], multiq);
     plain(multiq || a.q_len == 1);
     const Tensor& kv = unpack(x[2]);
@@ -344,11 +350,12 @@ PyObject* mla_slab(PyObject*, PyObject* const* x, Py_ssize_t n) {
   });
 }
 
-// q_lat, q_pe, kv_pool, o_lat, seq_lens, rows or None, kv_indices, kv_indptr, parts, scale, kv_scale, multiq
+// q_lat, q_pe, kv_pool, o_lat, seq_lens, rows or None, kv_indices, kv_indptr, parts, scale, kv_scale, scale_p, multiq
 PyObject* mla_paged(PyObject*, PyObject* const* x, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    plain(n == 12);
-    const bool multiq = x[11] == Py_True;
+    plain(n == 13);
+    const bool multiq = x[12] == Py_True;
+    unused_scale_p(x[11], multiq);
     const MlaArgs a = mla_args(x[0], x[1], x[3], multiq);
     const Tensor& pool = unpack(x[2]);
     check_tensor(pool, at::kFloat8_e4m3fn, a.q_lat.device());
@@ -383,10 +390,11 @@ PyObject* mla_paged(PyObject*, PyObject* const* x, Py_ssize_t n) {
   });
 }
 
-// q_lat, q_pe, kv_pool, o_lat, seq_lens, block_table, parts, scale, kv_scale, rows or None
+// q_lat, q_pe, kv_pool, o_lat, seq_lens, block_table, parts, scale, kv_scale, scale_p, rows or None
 PyObject* mla_blocks(PyObject*, PyObject* const* x, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    plain(n == 10);
+    plain(n == 11);
+    unused_scale_p(x[9], false);
     const MlaArgs a = mla_args(x[0], x[1], x[3], false);
     const Tensor& pool = unpack(x[2]);
     check_tensor(pool, at::kFloat8_e4m3fn, a.q_lat.device());
@@ -394,7 +402,7 @@ PyObject* mla_blocks(PyObject*, PyObject* const* x, Py_ssize_t n) {
     const Tensor& lens = index_tensor(x[4], a.q_lat, a.B);
     const Tensor& table = index_tensor(x[5], a.q_lat, 1);
     plain(table.dim() == 2 && table.size(0) == a.B && table.size(1) >= 1);
-    const Tensor rows = x[9] == Py_None ? Tensor() : index_tensor(x[9], a.q_lat, a.B);
+    const Tensor rows = x[10] == Py_None ? Tensor() : index_tensor(x[10], a.q_lat, a.B);
     const int parts = int_arg(x[6]);
     plain(parts <= (1 << 20));
     const float scale = float_arg(x[7]), kv_scale = float_arg(x[8]);

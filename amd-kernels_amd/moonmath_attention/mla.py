@@ -144,7 +144,7 @@ def mla_decode_a16w8(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0) -> No
     o_lat [B,H,512] bf16 (written in place). scale = softmax scale,
     kv_scale = per-tensor fp8 KV descale. (Reference mla.py:41-61.)
     """
-    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, False):
+    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p, False):
         return
     who = "mla_decode_a16w8"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
@@ -173,7 +173,7 @@ def mla_decode_a16w8_paged_dev(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_i
     the caller (plan_parts*). (Reference mla.py:64-95.)
     """
     if _lib.calls.mla_paged(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, parts, scale, kv_scale,
-                            False):
+                            scale_p, False):
         return
     who = "mla_decode_a16w8_paged_dev"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
@@ -204,7 +204,8 @@ def mla_decode_a16w8_paged_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_t
     driven and graph capturable with ``parts`` fixed: the decode reads the table
     on the GPU (page ids clamped to the pool, lengths to the table).
     """
-    if _lib.calls.mla_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_table, parts, scale, kv_scale, rows):
+    if _lib.calls.mla_blocks(q_lat, q_pe, kv_pool, o_lat, seq_lens, block_table, parts, scale, kv_scale,
+                             scale_p, rows):
         return
     who = "mla_decode_a16w8_paged_blocks"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=False)
@@ -263,7 +264,7 @@ def mla_decode_a16w8_multiq(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0
     float8_e4m3fn; o_lat like q_lat. Position t attends kv[:, : S - q_len + t + 1].
     (Reference mla.py:122-145.)
     """
-    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, True):
+    if _lib.calls.mla_slab(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p, True):
         return
     who = "mla_decode_a16w8_multiq"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=True)
@@ -282,7 +283,7 @@ def mla_decode_a16w8_multiq_paged_dev(q_lat, q_pe, kv_pool, o_lat, seq_lens, row
     """Multi-query decode over a paged pool, device-driven (graph capturable).
     (Reference mla.py:148-176.)"""
     if _lib.calls.mla_paged(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, parts, scale, kv_scale,
-                            True):
+                            scale_p, True):
         return
     who = "mla_decode_a16w8_multiq_paged_dev"
     B, H, q_len = _check_q(q_lat, q_pe, o_lat, who, multiq=True)

@@ -26,9 +26,9 @@ def test_leaves_everything_else_to_python():
                  (q, q, q, None, "xyz", "bhsd"), (q, q, q, None, 3, "bhsd"), (q, q)):
         assert c.forward(*args) is None
     assert c.forward_lite(q, q, q, q, q, -6.0, 1, None, "rtna", "bhsd") is None
-    assert c.mla_slab(q, q, q, q, 1.0, 1.0, False) is None
-    assert c.mla_paged(q, q, q, q, q, None, q, q, 1, 1.0, 1.0, True) is None
-    assert c.mla_blocks(q, q, q, q, q, q, 1, 1.0, 1.0, None) is None
+    assert c.mla_slab(q, q, q, q, 1.0, 1.0, 1.0, False) is None
+    assert c.mla_paged(q, q, q, q, q, None, q, q, 1, 1.0, 1.0, 1.0, True) is None
+    assert c.mla_blocks(q, q, q, q, q, q, 1, 1.0, 1.0, 1.0, None) is None
     assert c.kv_quantize(q, q, q, q, 1.0, False) is None
 
 
@@ -141,6 +141,30 @@ def test_refusals_stay_refused_on_gpu():
         ma.forward(q, k, v, round_mode="up")
     sub = ma.forward(q.as_subclass(_Sub), k, v)  # taken, by the Python path
     assert torch.equal(sub.as_subclass(torch.Tensor), ma.forward(q, k, v))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad,error", [("much", ValueError), (object(), TypeError), (None, TypeError)])
+def test_scale_p_must_be_a_number(bad, error):
+    """The single-query ops use scale_p nowhere and refuse what is no number; what
+    converts to one is taken."""
+    q_lat, q_pe = (t[:, 0].contiguous().to(DEV) for t in rand_q(1, 1, 16, 5))
+    rows = rand_kv_rows(128, 7).to(DEV)
+    n, idx, indptr, table = (torch.tensor(t, dtype=torch.int32, device=DEV)
+                             for t in ([128], list(range(128)), [0, 128], [[0, 1]]))
+    o = torch.zeros_like(q_lat)
+    for scale_p in (bad, 1, "2.5"):
+        for call in (lambda s: ma.mla_decode_a16w8(q_lat, q_pe, rows.view(1, 128, QK), o, SCALE_192, KV_SCALE, s),
+                     lambda s: ma.mla_decode_a16w8_paged_dev(q_lat, q_pe, rows, o, n, None, idx, indptr, 1, SCALE_192,
+                                                             KV_SCALE, s),
+                     lambda s: ma.mla_decode_a16w8_paged_blocks(q_lat, q_pe, rows.view(2, 64, QK), o, n, table, 1,
+                                                                SCALE_192, KV_SCALE, s)):
+            if scale_p is bad:
+                with pytest.raises(error):
+                    call(scale_p)
+            else:
+                call(scale_p)
+    torch.cuda.synchronize()
 
 
 @pytest.mark.gpu
