@@ -22,6 +22,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <climits>
 #include <cstdlib>
@@ -479,6 +480,8 @@ PyObject* bound_names(PyObject*, PyObject*) {
   return t;
 }
 
+PyObject* torch_version(PyObject*, PyObject*) { return PyUnicode_FromString(TORCH_VERSION); }
+
 #define MM_FAST(name) {#name, (PyCFunction)(void (*)())name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {MM_FAST(forward),
                          MM_FAST(forward_lite),
@@ -488,6 +491,7 @@ PyMethodDef methods[] = {MM_FAST(forward),
                          MM_FAST(kv_quantize),
                          {"bind", bind, METH_O, nullptr},
                          {"bound_names", bound_names, METH_NOARGS, nullptr},
+                         {"torch_version", torch_version, METH_NOARGS, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods};

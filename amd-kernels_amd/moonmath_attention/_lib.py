@@ -7,9 +7,12 @@ The library is loaded once; a missing or incomplete library raises ImportError
 at import time -- there is no fallback path.
 """
 import ctypes
+import importlib
 import os
+import re
+import warnings
 
-import torch  # noqa: F401  (loads the libtorch that _calls is linked to)
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("MOONMATH_LIB") or os.path.join(_HERE, "libmoonmath_gfx950.so")
@@ -90,15 +93,32 @@ class _Lib:
 
 lib = _Lib(LIB_PATH)
 
-try:
-    from . import _calls as calls
-except ImportError as e:
-    raise ImportError(
-        f"moonmath_attention: the _calls module is not usable ({e}). "
-        "Build it with `python amd-kernels_amd/build_lib.py`."
-    ) from e
-# The plain GPU calls go through native code to the same launchers (csrc/calls.cpp).
-calls.bind({name: ctypes.cast(getattr(lib.dll, name), _p).value for name in calls.bound_names()})
+class _PythonOnly:
+    """In the native path's place: leaves every call to the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def load_calls():
+    """The native path of plain GPU calls (csrc/calls.cpp), bound to ``lib``'s
+    launchers. It is compiled against one torch; with another the wrappers' Python
+    path makes the same launches."""
+    try:
+        calls = importlib.import_module("._calls", __package__)
+        built = calls.torch_version()
+        if built != re.match(r"[\d.]*\d", torch.__version__).group():
+            raise ImportError(f"built against torch {built}, running {torch.__version__}")
+    except ImportError as e:
+        warnings.warn(
+            f"moonmath_attention: the _calls module is not usable ({e}): calls take ~10 us more on the host. "
+            "Build it with `python amd-kernels_amd/build_lib.py`.", RuntimeWarning, stacklevel=2)
+        return _PythonOnly()
+    calls.bind({name: ctypes.cast(getattr(lib.dll, name), _p).value for name in calls.bound_names()})
+    return calls
+
+
+calls = load_calls()
 
 
 def stream_ptr(device):

@@ -1,6 +1,8 @@
 """The native call path (csrc/calls.cpp): it takes plain GPU calls and nothing
 else, and gives what the Python path gives."""
+import sys
 import threading
+import types
 
 import pytest
 import torch
@@ -34,6 +36,22 @@ def test_leaves_everything_else_to_python():
 
 def test_binds_every_launcher_it_uses():
     assert all(hasattr(_lib.lib, name) for name in _lib.calls.bound_names())
+
+
+@pytest.mark.parametrize("why", ["missing", "other torch"])
+def test_without_the_native_path(why, monkeypatch):
+    """No module, or one of another torch: a warning, and the Python path alone."""
+    if why == "missing":
+        monkeypatch.setitem(sys.modules, "moonmath_attention._calls", None)
+    else:
+        monkeypatch.setattr(torch, "__version__", "1.2.3+other")
+    with pytest.warns(RuntimeWarning, match="_calls module is not usable"):
+        calls = _lib.load_calls()
+    assert calls.forward(1, 2) is None and calls.kv_quantize() is None
+
+
+def test_native_path_is_loaded():
+    assert isinstance(_lib.calls, types.ModuleType)
 
 
 def _python_path(monkeypatch):
