@@ -114,7 +114,7 @@ __device__ __forceinline__ uint32_t u16_field(uint32_t w, int k) {
 constexpr int kMaxPagedB = 3072;  // 12 B per request: 36 KB of plan scratch
 
 // ceil(a / d) for 0 <= a, 1 <= d, a + d < 2^32.
-__device__ __forceinline__ int ceil_div_u(int a, int d) {
+__host__ __device__ __forceinline__ int ceil_div_u(int a, int d) {
   return (int)(((unsigned)a + (unsigned)d - 1u) / (unsigned)d);
 }
 __device__ __forceinline__ int nparts_of(int L, int C) { return L <= C ? 1 : ceil_div_u(L, C); }
@@ -356,10 +356,16 @@ struct Seg {
   int pos;             // place of the request's first tile (balanced split)
   int tw;              // places per unit (0: equal parts, one segment per unit)
 };
-__device__ __forceinline__ int work_tiles(int len) { return len > kTileTok ? (len - 1) / kTileTok + 1 : 1; }
+__host__ __device__ __forceinline__ int work_tiles(int len) { return len > kTileTok ? (len - 1) / kTileTok + 1 : 1; }
+
+// Places per unit when `total` of them share `workers` units.
+__host__ __device__ __forceinline__ int work_share(int total, int workers) {
+  const int tw = ceil_div_u(total, workers);
+  return tw > kMinWork ? tw : kMinWork;
+}
 
 // Unit u's segment of a request whose first tile is at `pos`.
-__device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, int slot0) {
+__host__ __device__ __forceinline__ Seg work_seg(int u, int tw, int b, int pos, int len, int slot0) {
   const int nt = work_tiles(len);
   const int u0 = pos / tw;
   const int lo = u * tw > pos ? u * tw - pos : 0;
@@ -384,13 +390,9 @@ __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
   }
   const Seg none{-1, 0, 1, 0, 0, 0, 0, 0, 0, 1};
   if (u >= p.workers) return none;
-  auto share = [&](int total) {
-    const int tw = ceil_div_u(total, p.workers);
-    return tw > kMinWork ? tw : kMinWork;
-  };
   if constexpr (!PAGED) {
     const int per = work_tiles(p.S_fixed) + kSegCost;
-    const int tw = share(p.B * per);
+    const int tw = work_share(p.B * per, p.workers);
     const int b = u * tw / per;
     return b < p.B ? work_seg(u, tw, b, b * per + kSegCost, p.S_fixed, 0) : none;
   }
@@ -400,7 +402,7 @@ __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
   auto places = [&](int c0, int l) { return c0 + lane < p.B ? work_tiles(l) + kSegCost : 0; };
   int total = 0;
   for (int c0 = 0; c0 < p.B; c0 += 64) total += wave_sum_i(places(c0, len_at(c0)));
-  const int tw = share(total);
+  const int tw = work_share(total, p.workers);
   int run = 0;
   for (int c0 = 0; c0 < p.B; c0 += 64) {
     const int l = len_at(c0);
@@ -419,10 +421,10 @@ __device__ Seg plan_work(const Params& p, int u, int lane, int* scratch) {
 }
 
 // Unit u's segment after `sg`, or b = -1. `len`, `slot0`: of request sg.b + 1.
-__device__ __forceinline__ Seg next_work(const Params& p, const Seg& sg, int u, int len, int slot0) {
+__host__ __device__ __forceinline__ Seg next_work(int B, const Seg& sg, int u, int len, int slot0) {
   Seg r = sg;
   r.b = -1;
-  if (sg.tw == 0 || sg.b + 1 >= p.B) return r;
+  if (sg.tw == 0 || sg.b + 1 >= B) return r;
   const int pos = sg.pos + work_tiles(sg.len) + kSegCost;
   return pos < (u + 1) * sg.tw ? work_seg(u, sg.tw, sg.b + 1, pos, len, slot0) : r;
 }

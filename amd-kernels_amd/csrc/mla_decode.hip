@@ -494,6 +494,29 @@ int moonmath_mla_effective_parts(int B, int H, int parts, int q_len, int have_wo
   return clamp_parts(parts, B, H, q_len, have_workspace != 0);
 }
 
+int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, int* segments, int max_segments) {
+  if (B < 1 || H < 1 || q_len < 1 || !lens || !segments) return -6;
+  const int workers = workers_for(B, H, clamp_parts(parts, B, H, q_len, true), q_len);
+  if (workers == 0) return 0;
+  int total = 0, count = 0;
+  for (int b = 0; b < B; ++b) total += work_tiles(lens[b]) + kSegCost;
+  const int tw = work_share(total, workers);
+  int b0 = 0, end = work_tiles(lens[0]) + kSegCost;  // the first request that ends past the unit's places
+  for (int u = 0; u < workers; ++u) {
+    while (end <= u * tw && ++b0 < B) end += work_tiles(lens[b0]) + kSegCost;
+    if (b0 == B) break;
+    Seg s = work_seg(u, tw, b0, end - work_tiles(lens[b0]), lens[b0], 0);
+    for (; s.b >= 0; ++count) {
+      if (count < max_segments) {
+        const int v[7] = {u, s.b, s.part, s.nparts, s.rec0 + s.part, s.kv_lo, s.kv_hi};
+        for (int i = 0; i < 7; ++i) segments[7 * (size_t)count + i] = v[i];
+      }
+      s = next_work(B, s, u, s.b + 1 < B ? lens[s.b + 1] : 0, 0);
+    }
+  }
+  return count;
+}
+
 int moonmath_fp8e4m3_to_bf16(const void* in, void* out, int n, void* stream) {
   if (!in || !out || n < 0) return -6;
   if (n == 0) return 0;

@@ -710,7 +710,7 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
       tbl[2 * b] = sg.nparts;
       tbl[2 * b + 1] = sg.rec0;
     }
-    sg = next_work(p, sg, u, next_len, next_slot0);
+    sg = next_work(p.B, sg, u, next_len, next_slot0);
     if (sg.b < 0) break;
     lds_reads_done_barrier();  // every wave is done with this part's LDS
   }

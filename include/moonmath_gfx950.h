@@ -227,6 +227,13 @@ int mla_decode_a16w8_max_ctas(void);
  * workspace (have_workspace != 0) or none. */
 int moonmath_mla_effective_parts(int B, int H, int parts, int q_len, int have_workspace);
 
+/* The balanced split that a launch with a workspace makes of a batch of these
+ * lengths (host array): 7 ints per segment, {unit, request, part, parts of the
+ * request, record, first token, end token}, units in order, the first
+ * max_segments of them. Returns their number; 0: equal parts per request within
+ * the parts budget (fewer records than a round of units needs); -6. Pure host. */
+int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, int* segments, int max_segments);
+
 /* fp8 KV producer: for each token i < n_tokens with 0 <= slots[i] < num_slots,
  * writes row slots[i] of kv_pool ([num_slots, 576] bytes) as
  * e4m3fn(fl32(x / kv_scale)) of c_kv[i, 0:512] then k_pe[i, 0:64] (bf16,

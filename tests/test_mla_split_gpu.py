@@ -2,56 +2,56 @@
 shares the batch's 64-token tiles, several requests to a CTA and several CTAs
 to a request) at its edges, against the CPU oracle, and its arithmetic on the
 CPU. Tolerance: the oracle's 1-ULP rule of test_mla_gpu."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import moonmath_attention as ma
+from moonmath_attention import _lib
 from mla_inputs import KV_SCALE, QK, SCALE_576, fp8_bits, paged_pool, ragged_lens, rand_kv_rows, rand_q
 from test_mla_gpu import DEV, _check, _d
 
 
-def _tiles(n):
-    return max(1, -(-n // 64))
+def _split(lens, H, q_len, parts):
+    """(unit, request, part, parts, record, first token, end token) of every segment,
+    as the launchers' plan gives them; [] for equal parts within the parts budget."""
+    arr = (ctypes.c_int * len(lens))(*lens)
+    n = _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, (ctypes.c_int * 7)(), 0)
+    assert n >= 0
+    out = (ctypes.c_int * (7 * n + 1))()
+    assert _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, out, n) == n
+    return [tuple(out[7 * i:7 * i + 7]) for i in range(n)]
 
 
-def _segments(lens, units, cost=4):
-    """csrc/mla_common.hpp plan_work: (unit, request, first tile, end tile, part, parts, record) of
-    every segment."""
-    total = sum(_tiles(n) + cost for n in lens)
-    tw = max(-(-total // units), 4)
-    out, pos = [], 0
-    for b, n in enumerate(lens):
-        pos += cost
-        nt = _tiles(n)
-        u0, u1 = pos // tw, (pos + nt - 1) // tw
-        for u in range(u0, u1 + 1):
-            out.append((u, b, max(u * tw - pos, 0), min((u + 1) * tw - pos, nt), u - u0, u1 - u0 + 1, u + b))
-        pos += nt
-    return out
-
-
-@pytest.mark.parametrize("units", [256, 128, 85, 64, 16])
-def test_balanced_split_covers_every_tile_once(units):
-    """Each request's tiles are cut into consecutive, non-empty parts on
-    consecutive units, every unit is below the round's size, and the records
-    (unit + request) are distinct, consecutive per request and fit the B * P
-    of the workspace whenever units <= B * (P - 1) + 1."""
+@pytest.mark.parametrize("H,q_len,units", [(16, 1, 256), (5, 3, 256), (64, 1, 256), (128, 1, 128), (96, 2, 85),
+                                           (128, 2, 64), (128, 8, 16)])
+def test_balanced_split_covers_every_tile_once(H, q_len, units):
+    """Every token of every request in one segment, in order; parts consecutive, on
+    whole tiles and not empty (but the one of an empty request); records distinct,
+    consecutive per request and within the B * parts of the workspace; units within
+    a round. At the fewest parts the launchers run it with: one fewer leaves the
+    records of a round short."""
     rng = np.random.default_rng(units)
     cases = [rng.integers(0, 9000, size=int(rng.integers(1, 400))).tolist() for _ in range(60)]
-    cases += [[0] * 300, [1] * 70, [100000] + [0] * 90, [64] * 256, [8192] * 64, [5]]
+    cases += [[0] * 300, [1] * 70, [100000] + [0] * 90, [64] * 256, [8192] * 64, [5], [-3, 70, 5000], [2048] * 128]
     for lens in cases:
-        segs = _segments(lens, units)
         B = len(lens)
-        P = 1 + -(-(units - 1) // B)  # the fewest parts the host lets the split run with
-        recs = [s[6] for s in segs]
-        assert recs == sorted(set(recs)) and recs[-1] < B * P, (lens, units)
-        at = [0] * B
-        for u, b, lo, hi, part, parts, rec in segs:
-            assert 0 <= u < units and lo == at[b] < hi
-            at[b] = hi
-            assert 0 <= part < parts
-        assert at == [_tiles(n) for n in lens]
+        parts = 1 + -(-(units - 1) // B)
+        if _lib.lib.moonmath_mla_effective_parts(B, H, parts, q_len, 1) != parts:
+            continue  # more records than a workspace holds
+        assert parts == 1 or _split(lens, H, q_len, parts - 1) == []
+        at, first, recs, last = [0] * B, {}, [], 0
+        for u, b, part, nparts, rec, lo, hi in _split(lens, H, q_len, parts):
+            assert last <= u < units and lo == at[b] and (hi > lo or lens[b] <= 0 and lo == hi == 0)
+            assert 0 <= part < nparts and (hi % 64 == 0 or hi == lens[b])
+            assert part == 0 or rec == first[b] + part
+            first.setdefault(b, rec)
+            recs.append(rec)
+            at[b], last = hi, u
+        assert at == [max(0, n) for n in lens] and sorted(first) == list(range(B))
+        assert recs == sorted(set(recs)) and recs[-1] < B * parts
 
 
 LENS = [0, 1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513, 700, 1500, 2100, 9000]
@@ -137,8 +137,6 @@ def test_block_table_clamps_pages_and_lengths(H, parts):
 def test_noalloc_shares_its_array_beyond_64_parts():
     """300 parts of 256 rows: the size limit of the allocation-free entry counts
     64 of them (accepted); the call then uses the 128 that its array holds."""
-    from moonmath_attention import _lib
-
     H, q_len, S = 128, 2, 20000
     pool, idx, indptr = paged_pool([S], 99)
     q_lat, q_pe = rand_q(1, q_len, H, 99)
