@@ -50,8 +50,7 @@ struct Abi {
   X(lite_workspace_bytes_rtne)                                                                             \
   X(mla_decode_a16w8_multiq_workspace_for)                                                                 \
   X(moonmath_mla_effective_parts)                                                                          \
-  X(mla_decode_a16w8_plan_parts)                                                                           \
-  X(mla_decode_a16w8_multiq_plan_parts_q)                                                                  \
+  X(moonmath_mla_slab_parts)                                                                               \
   X(launch_mla_decode_a16w8)                                                                               \
   X(launch_mla_decode_a16w8_multiq)                                                                        \
   X(launch_mla_decode_a16w8_paged_dev)                                                                     \
@@ -332,8 +331,7 @@ PyObject* mla_slab(PyObject*, PyObject* const* x, Py_ssize_t n) {
     {
       pybind11::gil_scoped_release no_gil;
       const c10::DeviceGuard guard(a.q_lat.device());
-      const int parts = multiq ? abi.mla_decode_a16w8_multiq_plan_parts_q(a.B, S, a.q_len, a.H)
-                               : abi.mla_decode_a16w8_plan_parts(a.B, a.H, S, 512);
+      const int parts = abi.moonmath_mla_slab_parts(a.B, a.H, S, a.q_len);
       const Tensor ws = mla_workspace(a, parts);
       void* stream = stream_of(a.q_lat);
       if (multiq)

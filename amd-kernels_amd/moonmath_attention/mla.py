@@ -156,7 +156,7 @@ def mla_decode_a16w8(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0) -> No
     S = kv.shape[1]
     dev = q_lat.device
     with torch.cuda.device(dev):
-        parts = _lib.lib.mla_decode_a16w8_plan_parts(B, H, S, _LAT)
+        parts = _lib.lib.moonmath_mla_slab_parts(B, H, S, 1)
         ws = _workspace(B, H, parts, 1, dev)
         _run("launch_mla_decode_a16w8", _lib.ptr(q_lat), _lib.ptr(q_pe), _lib.ptr(kv), None, _lib.ptr(o_lat),
              B, H, S, _LAT, _ROPE, float(scale), float(kv_scale), float(scale_p), _lib.ptr(ws), _lib.stream_ptr(dev))
@@ -272,7 +272,7 @@ def mla_decode_a16w8_multiq(q_lat, q_pe, kv, o_lat, scale, kv_scale, scale_p=1.0
     S = kv.shape[1]
     dev = q_lat.device
     with torch.cuda.device(dev):
-        parts = _lib.lib.mla_decode_a16w8_multiq_plan_parts_q(B, S, q_len, H)
+        parts = _lib.lib.moonmath_mla_slab_parts(B, H, S, q_len)
         ws = _workspace(B, H, parts, q_len, dev)
         _run("launch_mla_decode_a16w8_multiq", _lib.ptr(q_lat), _lib.ptr(q_pe), _lib.ptr(kv), _lib.ptr(o_lat),
              B, H, S, q_len, _LAT, _ROPE, float(scale), float(kv_scale), _lib.ptr(ws), _lib.stream_ptr(dev))

@@ -227,6 +227,10 @@ int mla_decode_a16w8_max_ctas(void);
  * workspace (have_workspace != 0) or none. */
 int moonmath_mla_effective_parts(int B, int H, int parts, int q_len, int have_workspace);
 
+/* The parts the contiguous launchers run (B, S, H, q_len) with, given a workspace:
+ * at most what the planners above give. */
+int moonmath_mla_slab_parts(int B, int H, int S, int q_len);
+
 /* The balanced split that a launch with a workspace makes of a batch of these
  * lengths (host array): 7 ints per segment, {unit, request, part, parts of the
  * request, record, first token, end token}, units in order, the first

@@ -54,6 +54,19 @@ def test_balanced_split_covers_every_tile_once(H, q_len, units):
         assert recs == sorted(set(recs)) and recs[-1] < B * parts
 
 
+def test_contiguous_parts():
+    """Never more than the planners reserve records for; whole requests where they
+    fill most of a round, parts where a round has room for two of each."""
+    lib = _lib.lib
+    rng = np.random.default_rng(5)
+    for _ in range(2000):
+        B, H, S, q_len = (int(rng.integers(1, m)) for m in (600, 129, 9000, 9))
+        assert 1 <= lib.moonmath_mla_slab_parts(B, H, S, q_len) <= lib.mla_decode_a16w8_multiq_plan_parts_q(B, S, q_len, H)
+    for B, H, S, whole in [(256, 16, 2048, True), (200, 16, 2048, True), (230, 32, 1000, True), (128, 128, 1500, True),
+                           (150, 16, 2000, False), (80, 128, 3000, False), (100, 16, 2048, False), (1, 16, 4097, False)]:
+        assert (lib.moonmath_mla_slab_parts(B, H, S, 1) == 1) == whole, (B, H, S)
+
+
 LENS = [0, 1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513, 700, 1500, 2100, 9000]
 
 
@@ -81,7 +94,9 @@ def test_balanced_split_matches_oracle(H, q_len, page):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,q_len,B,S", [(16, 1, 5, 3001), (64, 1, 130, 100), (128, 1, 3, 1025), (32, 4, 2, 4097)])
+@pytest.mark.parametrize("H,q_len,B,S", [
+    (16, 1, 5, 3001), (64, 1, 130, 100), (128, 1, 3, 1025), (32, 4, 2, 4097),
+    (16, 1, 256, 600), (16, 1, 200, 1000), (128, 2, 64, 700)])  # whole requests where paged ones are split
 def test_balanced_split_contiguous(H, q_len, B, S):
     kv = rand_kv_rows(B * S, 93).view(B, S, QK)
     q_lat, q_pe = rand_q(B, q_len, H, 93)
@@ -91,7 +106,8 @@ def test_balanced_split_contiguous(H, q_len, B, S):
     (ma.mla_decode_a16w8 if q_len == 1 else ma.mla_decode_a16w8_multiq)(_d(q_lat), _d(q_pe), _d(kv), o, SCALE_576,
                                                                         KV_SCALE)
     torch.cuda.synchronize()
-    _check(o, q_lat, q_pe, fp8_bits(kv), [S] * B, SCALE_576)
+    pick = [b for b in range(B) if B <= 5 or b in (0, 1, 63, 64, B // 2, B - 1)]
+    _check(o, q_lat, q_pe, fp8_bits(kv), [S] * B, SCALE_576, batches=pick)
 
 
 @pytest.mark.gpu
