@@ -210,12 +210,16 @@ int max_parts_for(int B, int H, int q_len) {
   return m < 1 ? 1 : (int)m;
 }
 
-// Units one round of CTAs over the CUs holds (one CTA per CU fits in LDS; a
-// unit's ngroups CTAs share the CUs). Per-CTA set-up dominates short CTAs, so a
-// second round costs more than longer parts.
+// Units one round of CTAs over the CUs holds (one CTA per CU fits in LDS). A unit's
+// ngroups CTAs share an XCD, so it is what one XCD's CUs hold, times the XCDs: with
+// 3 groups 85 units are 33 CTAs on some XCDs, and one CTA's second round doubles
+// the longest path: 32 requests of 1024..8192 tokens, 64 heads, 3 drafts 123 us with
+// 85 units, 78 with 80; 12 of 5580, 128 heads, 3 drafts 100 with 42, 66 with 40.
+// Per-CTA set-up dominates short CTAs, so a second round costs more than longer
+// parts.
 int unit_cap_for(int H, int q_len) {
-  const int c = kNumCUs / ngroups_for(H, q_len);
-  return c < 1 ? 1 : c;
+  const int per_xcd = kNumCUs / mm::kNumXcds / ngroups_for(H, q_len);
+  return mm::kNumXcds * (per_xcd < 1 ? 1 : per_xcd);
 }
 
 // Tokens of the shortest part worth a CTA. One request of 4097 tokens: 16 heads
