@@ -181,13 +181,26 @@ constexpr int kMaxParts = 256;
 constexpr int kScratchParts = 64;          // parts that the allocation-free entry's size limit counts
 constexpr size_t kScratchRecords = 32768;  // record rows of the allocation-free entry's array
 
-// Requests of at most 16 query rows run mla_coop_kernel, larger ones
-// mla_rows64_kernel in groups of 64 rows. At 32 rows and 256 requests of 2048
-// tokens the 64-row kernel is bound by HBM (54 us); the 16-row kernel would
-// read every token twice.
+// Query rows of a CTA. Requests of at most 16 rows run mla_coop_kernel, larger ones
+// mla_rows64_kernel in groups of 64 rows (at 32 rows and 256 requests of 2048
+// tokens it is bound by HBM, 54 us; the 16-row kernel would read every token
+// twice). Calls of 33..64 rows that one round of 32-row groups holds run those
+// instead, two to a token read, while the batch is small: half the round's units,
+// so half the records, and half of Q and O per CTA, against a second reading of
+// the tokens from L2. 64 -> 32 rows, us: one request of 550 tokens 16.1 -> 13.0; 10
+// of 9028 35.1 -> 29.1; 123 of 599 32.6 -> 21.4; 128 of 2048 (4096 tiles) 58.5 ->
+// 49.3; 60 of 6147 (5820) 77.7 -> 74.1; over the line 32 of 7041..16338 (5850) 74.2
+// -> 76.0, 65 of 7245 (7410) 90.6 -> 99.9, 216 of 1303 54.5 -> 63.6. `tokens`: of the
+// whole call or a bound on them, 0 if unknown.
 constexpr int kCoopMaxRows = 16;
+constexpr int kRows32MaxTiles = 5120;
 bool use_coop(int H, int q_len) { return H * q_len <= kCoopMaxRows; }
-int ngroups_for(int H, int q_len) { return use_coop(H, q_len) ? 1 : (H * q_len + kRows64 - 1) / kRows64; }
+int cta_rows_for(int B, int H, int q_len, long long tokens) {
+  if (use_coop(H, q_len)) return kCoopMaxRows;
+  const bool small = tokens > 0 && tokens <= (long long)kRows32MaxTiles * kTileTok;
+  return small && H * q_len > 32 && H * q_len <= kRows64 && B <= kNumCUs / 2 ? 32 : kRows64;
+}
+int ngroups_for(int H, int q_len, int cta_rows) { return (H * q_len + cta_rows - 1) / cta_rows; }
 
 // O rows of one split record in the workspace: whole 32-row tiles for 96..128
 // query rows (the size its callers have), otherwise the query rows.
@@ -217,8 +230,8 @@ int max_parts_for(int B, int H, int q_len) {
 // 85 units, 78 with 80; 12 of 5580, 128 heads, 3 drafts 100 with 42, 66 with 40.
 // Per-CTA set-up dominates short CTAs, so a second round costs more than longer
 // parts.
-int unit_cap_for(int H, int q_len) {
-  const int per_xcd = kNumCUs / mm::kNumXcds / ngroups_for(H, q_len);
+int unit_cap_for(int H, int q_len, int cta_rows) {
+  const int per_xcd = kNumCUs / mm::kNumXcds / ngroups_for(H, q_len, cta_rows);
   return mm::kNumXcds * (per_xcd < 1 ? 1 : per_xcd);
 }
 
@@ -236,7 +249,7 @@ constexpr int kMergeCostTiles = 5;
 int plan_parts(int B, int H, int max_seq_len, int q_len) {
   if (B < 1) B = 1;
   if (q_len < 1) q_len = 1;
-  const int units = unit_cap_for(H, q_len);
+  const int units = unit_cap_for(H, q_len, cta_rows_for(B, H, q_len, 0));
   const int min_chunk = min_chunk_for(H, q_len);
   const long long tiles = (long long)max_seq_len / kTileTok + 1;
   const long long whole = tiles * ((B + units - 1) / units);
@@ -255,8 +268,8 @@ int plan_parts(int B, int H, int max_seq_len, int q_len) {
 // Units of the balanced split: a full round, where its records fit (unit u's
 // segment of request b is record u + b, so W units need W + B - 1 of the B *
 // parts); otherwise 0, equal parts per request.
-int workers_for(int B, int H, int parts, int q_len) {
-  const int cap = unit_cap_for(H, q_len);
+int workers_for(int B, int H, int parts, int q_len, int cta_rows) {
+  const int cap = unit_cap_for(H, q_len, cta_rows);
   return parts > 1 && (long long)B * (parts - 1) + 1 >= cap ? cap : 0;
 }
 
@@ -274,7 +287,8 @@ constexpr double kIdleCoop = 0.56, kIdleRows64 = 0.86;
 constexpr double kSlabMergeTiles = 1.0;
 int slab_parts(int B, int H, int S, int q_len) {
   const int parts = plan_parts(B, H, S, q_len);
-  const int units = unit_cap_for(H, q_len);
+  const int cta_rows = cta_rows_for(B, H, q_len, (long long)B * S);
+  const int units = unit_cap_for(H, q_len, cta_rows);
   if (parts <= 1 || B > units || 2 * B <= units) return parts;
   const int tiles = work_tiles(S);
   const double idle = use_coop(H, q_len) ? kIdleCoop : kIdleRows64;
@@ -282,7 +296,7 @@ int slab_parts(int B, int H, int S, int q_len) {
   const int tw = work_share(B * (tiles + kSegCost), units);
   const double borders = (double)B * (tiles - 1) / tw;
   const double records = borders + (borders < B ? borders : B);
-  const int rows = H * q_len < kRows64 ? H * q_len : kRows64;
+  const int rows = H * q_len < cta_rows ? H * q_len : cta_rows;
   return whole <= tw + records * rows / (9.0 * units) + kSlabMergeTiles ? 1 : parts;
 }
 
@@ -293,6 +307,9 @@ int clamp_parts(int parts, int B, int H, int q_len, bool have_ws) {
   if (!have_ws) p = 1;
   return p;
 }
+
+// Tokens of `kv_bytes` fused rows, at least.
+long long tokens_of(size_t kv_bytes) { return (long long)(kv_bytes / kQK); }
 
 // Argument codes shared by every decode launcher (0 = arguments usable).
 int check_launch_args(const void* q_lat, const void* q_pe, const void* kv, const void* o_lat, const void* seq_lens,
@@ -311,7 +328,7 @@ int check_launch_args(const void* q_lat, const void* q_pe, const void* kv, const
 int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, const void* seq_lens,
            const void* rows, const void* kv_indices, const void* kv_indptr, int B, int H, int S_fixed, int parts,
            int q_len, int lat_dim, int rope_dim, float scale, float kv_scale, void* workspace, void* stream,
-           bool paged, const void* table = nullptr, int max_blocks = 0, int num_blocks = 0) {
+           bool paged, long long tokens, const void* table = nullptr, int max_blocks = 0, int num_blocks = 0) {
   const int arg_rc = check_launch_args(q_lat, q_pe, kv, o_lat, seq_lens, kv_indices, kv_indptr, B, H, S_fixed, q_len,
                                        lat_dim, rope_dim, paged);
   if (arg_rc != 0) return arg_rc;
@@ -333,9 +350,10 @@ int launch(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, con
   p.q_len = q_len;
   p.S_fixed = S_fixed;
   p.parts = clamp_parts(parts, B, H, q_len, workspace != nullptr);
-  p.ngroups = ngroups_for(H, q_len);
-  p.unit_cap = unit_cap_for(H, q_len);
-  p.workers = workers_for(B, H, p.parts, q_len);
+  const int cta_rows = cta_rows_for(B, H, q_len, tokens);
+  p.ngroups = ngroups_for(H, q_len, cta_rows);
+  p.unit_cap = unit_cap_for(H, q_len, cta_rows);
+  p.workers = workers_for(B, H, p.parts, q_len, cta_rows);
   p.min_chunk = min_chunk_for(H, q_len);
   p.paged = paged ? 1 : 0;
   p.qrows = H * q_len;
@@ -418,7 +436,7 @@ int launch_mla_decode_a16w8(const void* q_lat, const void* q_pe, const void* c_k
   (void)scale_p;
   const int parts = workspace ? slab_parts(B, H, S, 1) : 1;
   return launch(q_lat, q_pe, c_kv, o_lat, nullptr, nullptr, nullptr, nullptr, B, H, S, parts, 1, lat_dim, rope_dim,
-                scale, kv_scale, workspace, stream, false);
+                scale, kv_scale, workspace, stream, false, (long long)B * S);
 }
 
 int launch_mla_decode_a16w8_paged_dev(const void* q_lat, const void* q_pe, const void* kv_pool, void* o_lat,
@@ -427,9 +445,8 @@ int launch_mla_decode_a16w8_paged_dev(const void* q_lat, const void* q_pe, const
                                       float scale, float kv_scale, float scale_p, void* workspace, void* stream,
                                       size_t kv_bytes, int q_len) {
   (void)scale_p;
-  (void)kv_bytes;
   return launch(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, B, H, 0, parts, q_len, lat_dim,
-                rope_dim, scale, kv_scale, workspace, stream, true);
+                rope_dim, scale, kv_scale, workspace, stream, true, tokens_of(kv_bytes));
 }
 
 int launch_mla_decode_a16w8_paged_dev_noalloc(const void* q_lat, const void* q_pe, const void* kv_pool, void* o_lat,
@@ -438,7 +455,6 @@ int launch_mla_decode_a16w8_paged_dev_noalloc(const void* q_lat, const void* q_p
                                               int rope_dim, float scale, float kv_scale, float scale_p, void* stream,
                                               size_t kv_bytes, int q_len) {
   (void)scale_p;
-  (void)kv_bytes;
   // The workspace launcher's argument codes first, then the scratch limit.
   const int arg_rc = check_launch_args(q_lat, q_pe, kv_pool, o_lat, seq_lens, kv_indices, kv_indptr, B, H, 0, q_len,
                                        lat_dim, rope_dim, true);
@@ -454,7 +470,7 @@ int launch_mla_decode_a16w8_paged_dev_noalloc(const void* q_lat, const void* q_p
     if (rc != 0) return rc;
   }
   return launch(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, B, H, 0, eff, q_len, lat_dim,
-                rope_dim, scale, kv_scale, ws, stream, true);
+                rope_dim, scale, kv_scale, ws, stream, true, tokens_of(kv_bytes));
 }
 
 size_t mla_decode_a16w8_blocks_index_bytes(int B, int max_blocks) {
@@ -476,7 +492,8 @@ int launch_mla_decode_a16w8_paged_blocks_dev(const void* q_lat, const void* q_pe
   // The kernels read the table themselves (a page is a tile): no per-token slots
   // are written, and the index workspace, sized for them, stays untouched.
   return launch(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, block_table, block_table, B, H, 0, parts, q_len, lat_dim,
-                rope_dim, scale, kv_scale, workspace, stream, true, block_table, max_blocks, num_blocks);
+                rope_dim, scale, kv_scale, workspace, stream, true, (long long)B * max_blocks * kPage, block_table,
+                max_blocks, num_blocks);
 }
 
 int launch_mla_decode_a16w8_multiq(const void* q_lat, const void* q_pe, const void* kv, void* o_lat, int B, int H,
@@ -484,7 +501,7 @@ int launch_mla_decode_a16w8_multiq(const void* q_lat, const void* q_pe, const vo
                                    void* workspace, void* stream) {
   const int parts = workspace ? slab_parts(B, H, S, q_len) : 1;
   return launch(q_lat, q_pe, kv, o_lat, nullptr, nullptr, nullptr, nullptr, B, H, S, parts, q_len, lat_dim,
-                rope_dim, scale, kv_scale, workspace, stream, false);
+                rope_dim, scale, kv_scale, workspace, stream, false, (long long)B * S);
 }
 
 int launch_mla_decode_a16w8_multiq_paged_dev(const void* q_lat, const void* q_pe, const void* kv_pool, void* o_lat,
@@ -492,9 +509,8 @@ int launch_mla_decode_a16w8_multiq_paged_dev(const void* q_lat, const void* q_pe
                                              const void* kv_indptr, int B, int H, int parts, int q_len,
                                              int lat_dim, int rope_dim, float scale, float kv_scale,
                                              void* workspace, void* stream, size_t kv_bytes) {
-  (void)kv_bytes;
   return launch(q_lat, q_pe, kv_pool, o_lat, seq_lens, rows, kv_indices, kv_indptr, B, H, 0, parts, q_len, lat_dim,
-                rope_dim, scale, kv_scale, workspace, stream, true);
+                rope_dim, scale, kv_scale, workspace, stream, true, tokens_of(kv_bytes));
 }
 
 int mla_decode_a16w8_plan_parts(int B, int H, int max_seq_len, int lat_dim) {
@@ -529,9 +545,11 @@ int moonmath_mla_slab_parts(int B, int H, int S, int q_len) {
   return slab_parts(B, H, S, q_len < 1 ? 1 : q_len);
 }
 
-int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, int* segments, int max_segments) {
+int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, long long tokens, int* segments,
+                       int max_segments) {
   if (B < 1 || H < 1 || q_len < 1 || !lens || !segments) return -6;
-  const int workers = workers_for(B, H, clamp_parts(parts, B, H, q_len, true), q_len);
+  const int workers =
+      workers_for(B, H, clamp_parts(parts, B, H, q_len, true), q_len, cta_rows_for(B, H, q_len, tokens));
   if (workers == 0) return 0;
   int total = 0, count = 0;
   for (int b = 0; b < B; ++b) total += work_tiles(lens[b]) + kSegCost;

@@ -79,7 +79,7 @@ static_assert(12 * kMaxPagedB <= kRTileBytes, "plan scratch fits ring slot 2");
 static_assert(kRRows * kLat * 4 <= kRIdxOff, "the staged output rows leave the rest alone");
 static_assert(kRLdsBytes <= 160 * 1024, "LDS budget");
 
-// NRT: row tiles that hold query rows (1: at most 32 rows in the call). NT:
+// NRT: row tiles of a CTA (1: at most 32 rows in the call, or groups of 32). NT:
 // non-temporal gathers, for calls whose tokens one CTA reads once (one row
 // group).
 template <bool PAGED, int NRT, bool NT>
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kRThreads, 1) void mla_rows64_kernel(Params p) {
     const int kv_hi = __builtin_amdgcn_readfirstlane(sg.kv_hi);
 
     // ---- the query row of this lane's MFMA column --------------------------------------
-    const int row0 = grp * kRRows;
+    const int row0 = grp * 32 * NRT;
     const int qrow = row0 + 32 * rt + n;
     const int qr = qrow < p.qrows ? qrow : p.qrows - 1;  // padding columns repeat the last row
     const int lim = S - (p.q_len - 1 - qr / p.H);          // tokens >= lim are masked for this row
@@ -720,6 +720,8 @@ template <bool PAGED>
 static void launch_rows64(const Params& p, dim3 grid, hipStream_t st) {
   if (p.qrows <= 32)
     hipLaunchKernelGGL((mla_rows64_kernel<PAGED, 1, true>), grid, dim3(kRThreads), 0, st, p);
+  else if (p.qrows <= kRows64 && p.ngroups == 2)
+    hipLaunchKernelGGL((mla_rows64_kernel<PAGED, 1, false>), grid, dim3(kRThreads), 0, st, p);
   else if (p.ngroups == 1)
     hipLaunchKernelGGL((mla_rows64_kernel<PAGED, 2, true>), grid, dim3(kRThreads), 0, st, p);
   else

@@ -157,7 +157,9 @@ int launch_mla_decode_a16w8(const void* q_lat, const void* q_pe, const void* c_k
 
 /* Paged pool [slots,576]; request b owns kv_indices[kv_indptr[b] ..
  * kv_indptr[b] + seq_lens[b]); rows[B] (nullable) maps request -> q/out row;
- * parts fixed by the caller. kv_bytes is accepted for ABI parity.
+ * parts fixed by the caller. kv_bytes: bytes of the requests' rows (576 per index)
+ * or a bound on them, 0 if unknown; it decides how calls of 33..64 query rows are
+ * laid out (by speed alone).
  * Replaces csrc/mla_decode_a16w8.hip:813-844. */
 int launch_mla_decode_a16w8_paged_dev(const void* q_lat, const void* q_pe, const void* kv_pool, void* o_lat,
                                       const void* seq_lens, const void* rows, const void* kv_indices,
@@ -232,11 +234,12 @@ int moonmath_mla_effective_parts(int B, int H, int parts, int q_len, int have_wo
 int moonmath_mla_slab_parts(int B, int H, int S, int q_len);
 
 /* The balanced split that a launch with a workspace makes of a batch of these
- * lengths (host array): 7 ints per segment, {unit, request, part, parts of the
+ * lengths (host array), `tokens` = its kv_bytes / 576: 7 ints per segment, {unit, request, part, parts of the
  * request, record, first token, end token}, units in order, the first
  * max_segments of them. Returns their number; 0: equal parts per request within
  * the parts budget (fewer records than a round of units needs); -6. Pure host. */
-int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, int* segments, int max_segments);
+int moonmath_mla_split(int B, const int* lens, int H, int q_len, int parts, long long tokens, int* segments,
+                       int max_segments);
 
 /* fp8 KV producer: for each token i < n_tokens with 0 <= slots[i] < num_slots,
  * writes row slots[i] of kv_pool ([num_slots, 576] bytes) as

@@ -14,20 +14,21 @@ from mla_inputs import KV_SCALE, QK, SCALE_576, fp8_bits, paged_pool, ragged_len
 from test_mla_gpu import DEV, _check, _d
 
 
-def _split(lens, H, q_len, parts):
+def _split(lens, H, q_len, parts, tokens=0):
     """(unit, request, part, parts, record, first token, end token) of every segment,
     as the launchers' plan gives them; [] for equal parts within the parts budget."""
     arr = (ctypes.c_int * len(lens))(*lens)
-    n = _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, (ctypes.c_int * 7)(), 0)
+    n = _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, tokens, (ctypes.c_int * 7)(), 0)
     assert n >= 0
     out = (ctypes.c_int * (7 * n + 1))()
-    assert _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, out, n) == n
+    assert _lib.lib.moonmath_mla_split(len(lens), arr, H, q_len, parts, tokens, out, n) == n
     return [tuple(out[7 * i:7 * i + 7]) for i in range(n)]
 
 
-@pytest.mark.parametrize("H,q_len,units", [(16, 1, 256), (5, 3, 256), (64, 1, 256), (128, 1, 128), (96, 2, 80),
-                                           (128, 2, 64), (128, 8, 16)])
-def test_balanced_split_covers_every_tile_once(H, q_len, units):
+@pytest.mark.parametrize("H,q_len,tokens,units", [
+    (16, 1, 0, 256), (5, 3, 9000, 256), (64, 1, 0, 256), (64, 1, 1, 128), (11, 3, 327680, 128), (64, 1, 327681, 256),
+    (128, 1, 1, 128), (96, 2, 0, 80), (128, 2, 0, 64), (128, 8, 0, 16)])
+def test_balanced_split_covers_every_tile_once(H, q_len, tokens, units):
     """Every token of every request in one segment, in order; parts consecutive, on
     whole tiles and not empty (but the one of an empty request); records distinct,
     consecutive per request and within the B * parts of the workspace; units within
@@ -38,12 +39,14 @@ def test_balanced_split_covers_every_tile_once(H, q_len, units):
     cases += [[0] * 300, [1] * 70, [100000] + [0] * 90, [64] * 256, [8192] * 64, [5], [-3, 70, 5000], [2048] * 128]
     for lens in cases:
         B = len(lens)
+        if tokens and 32 < H * q_len <= 64 and B > 128:
+            continue  # row groups of 64
         parts = 1 + -(-(units - 1) // B)
         if _lib.lib.moonmath_mla_effective_parts(B, H, parts, q_len, 1) != parts:
             continue  # more records than a workspace holds
-        assert parts == 1 or _split(lens, H, q_len, parts - 1) == []
+        assert parts == 1 or _split(lens, H, q_len, parts - 1, tokens) == []
         at, first, recs, last = [0] * B, {}, [], 0
-        for u, b, part, nparts, rec, lo, hi in _split(lens, H, q_len, parts):
+        for u, b, part, nparts, rec, lo, hi in _split(lens, H, q_len, parts, tokens):
             assert last <= u < units and lo == at[b] and (hi > lo or lens[b] <= 0 and lo == hi == 0)
             assert 0 <= part < nparts and (hi % 64 == 0 or hi == lens[b])
             assert part == 0 or rec == first[b] + part
@@ -108,6 +111,32 @@ def test_balanced_split_contiguous(H, q_len, B, S):
     torch.cuda.synchronize()
     pick = [b for b in range(B) if B <= 5 or b in (0, 1, 63, 64, B // 2, B - 1)]
     _check(o, q_lat, q_pe, fp8_bits(kv), [S] * B, SCALE_576, batches=pick)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,q_len", [(33, 1), (16, 3), (64, 1), (16, 4)])
+def test_row_groups_of_32_and_64(H, q_len):
+    """Calls of 33..64 rows as one 64-row group (kv_bytes 0: unknown) and as two of
+    32: the same sums for whole requests, bit for bit, and both within the oracle's
+    rule when split."""
+    lens = [1, 64, 200, 1000, 3000]
+    B = len(lens)
+    pool, idx, indptr = paged_pool(lens, 113)
+    q_lat, q_pe = rand_q(B, q_len, H, 113)
+    t = [_d(x) for x in (q_lat, q_pe, pool, torch.tensor(lens, dtype=torch.int32), idx, indptr)]
+    lib, p = _lib.lib, _lib.ptr
+    for parts in (1, 60):
+        ws = torch.empty(lib.mla_decode_a16w8_multiq_workspace_for(B, H, parts, q_len), dtype=torch.uint8, device=DEV)
+        outs = []
+        for kv_bytes in (0, idx.numel() * QK):
+            o = torch.full((B, q_len, H, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+            assert lib.launch_mla_decode_a16w8_paged_dev(p(t[0]), p(t[1]), p(t[2]), p(o), p(t[3]), None, p(t[4]), p(t[5]), B,
+                                                         H, parts, 512, 64, SCALE_576, KV_SCALE, 1.0, p(ws),
+                                                         _lib.stream_ptr(DEV), kv_bytes, q_len) == 0
+            torch.cuda.synchronize()
+            _check(o, q_lat, q_pe, fp8_bits(pool), lens, SCALE_576, kv_indices=idx.numpy(), kv_indptr=indptr.numpy())
+            outs.append(o)
+        assert parts > 1 or torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
 @pytest.mark.gpu
