@@ -83,6 +83,56 @@ def _qkv(layout, Sq=300, Skv=200, B=2, H=3):
 
 
 @pytest.mark.gpu
+def test_plain_gpu_calls_are_taken(monkeypatch):
+    """Each native function does a plain call itself, and its result is that of the
+    Python path."""
+    c = _lib.calls
+    q, k, v = _qkv("bhsd")
+    B, H, Sq, Skv = q.shape[0], q.shape[1], q.shape[2], k.shape[2]
+    lists = [torch.zeros(2, B, H, -(-Sq // 256), -(-Skv // 64) + 2, dtype=torch.int16, device=DEV) for _ in range(2)]
+    for pair in lists:
+        pair[0, ..., :3] = torch.tensor([2, -(-Skv // 64) - 1, -1], dtype=torch.int16)
+    lens = [700, 64, 1300]
+    pool, idx, indptr = (t.to(DEV) for t in paged_pool(lens, 5))
+    q4, p4 = (t.to(DEV) for t in rand_q(3, 3, 16, 5))
+    q3, p3 = q4[:, 0].contiguous(), p4[:, 0].contiguous()
+    n = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    slab = rand_kv_rows(3 * 500, 7).view(3, 500, QK).to(DEV)
+    table = torch.arange(15, dtype=torch.int32, device=DEV).view(3, 5)
+    blocks = pool.view(-1, 64, QK)
+    ckv, kpe = (torch.randn(50, w, device=DEV).bfloat16() for w in (512, 64))
+    slots = torch.arange(50, dtype=torch.int32, device=DEV)
+    s, ks = SCALE_192, KV_SCALE
+
+    got = [c.forward(q, k, v, None, "rtna", "bhsd"),
+           c.forward_lite(q, k, v, lists[0][0], lists[0][1], -3.0, 1, None, "rtna", "bhsd"), lists[0]]
+    outs = [torch.zeros_like(q3), torch.zeros_like(q4), torch.zeros_like(q3), torch.zeros_like(q4), torch.zeros_like(q3)]
+    cache = [torch.zeros(60, QK, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn) for _ in range(2)]
+    taken = [c.mla_slab(q3, p3, slab, outs[0], s, ks, 1.0, False), c.mla_slab(q4, p4, slab, outs[1], s, ks, 1.0, True),
+             c.mla_paged(q3, p3, pool, outs[2], n, None, idx, indptr, 4, s, ks, 1.0, False),
+             c.mla_paged(q4, p4, pool, outs[3], n, None, idx, indptr, 4, s, ks, 1.0, True),
+             c.mla_blocks(q3, p3, blocks, outs[4], n, table, 4, s, ks, 1.0, None),
+             c.kv_quantize(ckv, kpe, cache[0], slots, 0.03125, False)]
+    assert all(t is not None for t in got) and all(t is True for t in taken)
+    got += outs + [cache[0]]
+    with monkeypatch.context() as m:
+        _python_path(m)
+        want = [ma.forward(q, k, v),
+                ma.forward_lite(q, k, v, lists[1][0], lists[1][1], threshold=-3.0, phase=1), lists[1]]
+        o = [torch.zeros_like(t) for t in outs]
+        ma.mla_decode_a16w8(q3, p3, slab, o[0], s, ks)
+        ma.mla_decode_a16w8_multiq(q4, p4, slab, o[1], s, ks)
+        ma.mla_decode_a16w8_paged_dev(q3, p3, pool, o[2], n, None, idx, indptr, 4, s, ks)
+        ma.mla_decode_a16w8_multiq_paged_dev(q4, p4, pool, o[3], n, None, idx, indptr, 4, s, ks)
+        ma.mla_decode_a16w8_paged_blocks(q3, p3, blocks, o[4], n, table, 4, s, ks)
+        ma.mla_kv_quantize(ckv, kpe, cache[1], slots, 0.03125)
+        want += o + [cache[1]]
+    torch.cuda.synchronize()
+    for a, b in zip(got, want, strict=True):
+        assert torch.equal(a.view(torch.int8), b.view(torch.int8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["bhsd", "bshd"])
 @pytest.mark.parametrize("mode", ["rtna", "rtne", "rtz"])
 def test_attention_equals_the_python_path(layout, mode, monkeypatch):
