@@ -12,10 +12,10 @@
 //    B operand straight from registers (no shuffle).
 //  * K and V (up to 8192 query rows, see prefers_direct) or a pre-transposed
 //    V_t (more) are staged through LDS with 16-byte global->LDS DMA
-//    (global_load_lds_dwordx4) in 4-slot rings, two blocks of lead. Every DMA is inline asm, waited for by explicit vmcnt waits: with
-//    one the compiler can see in flight, its wait counting turns every LDS
-//    fragment wait into lgkmcnt(0) instead of the partial count the
-//    in-order reads allow. K slots are chunk-major in 16-row groups and V_t
+//    (global_load_lds_dwordx4) in 4-slot rings, two blocks of lead. Every DMA
+//    is inline asm, waited for by explicit vmcnt waits: with one the compiler
+//    can see in flight, its wait counting turns every LDS fragment wait into
+//    lgkmcnt(0) instead of the partial count the in-order reads allow. K slots are chunk-major in 16-row groups and V_t
 //    slots hold whole MFMA fragments in lane order, so every operand read is
 //    a conflict-free ds_read_b128; V slots hold rows, read by transposing reads.
 //  * Online softmax in base 2 with the running max kept on the integer grid:
@@ -1332,10 +1332,7 @@ namespace {
 using namespace mm::attn;
 
 constexpr int kNumCUs = 256;
-// Kernel variant used by the launchers: QT q-tiles of 32 rows per wave and
-// MINB CTAs resident per CU.
-constexpr int kMinBlocks = 1;  // CTAs resident per CU
-constexpr int kSlots = kNumCUs * kMinBlocks;
+constexpr int kSlots = kNumCUs;  // 256-row CTAs of a round: one per CU
 
 // Tail KV-split cost model, in KV blocks of the last round (after reference
 // csrc/attention_kernel.hip:1349-1393, whose span is rounds x blocks per part
@@ -1558,14 +1555,16 @@ int launch_mode(const void* q, const void* k, const void* v, void* out, int batc
   }
 }
 
-// Whether a forward is faster on V itself than with a V_t pass before it. The
-// pass costs a launch and 4 bytes of traffic per element of V, the transposing
-// reads ~1.5% of a CTA's main loop, so the line depends on the q rows that share
-// a V. Measured (V_t pass + kernel -> direct, us): (1,2,256) 14.4 -> 12.0,
-// (1,24,1531) 47.3 -> 39.5, (2,24,8192) x 77 55.3 -> 49.8, (2,24,4097) x 512 71.2
-// -> 66.8, (2,24,8192) x 512 132.3 -> 128.8, (2,24,4096) 349 -> 337, (2,24,8192)
-// 1340 -> 1338; (1,16,10519) 777 -> 780, (1,32,16384) 3628 -> 3636, (2,24,16384) x
-// 2048 748 -> 756, (2,8,32768) x 4096 929 -> 941.
+// Whether a forward, dense or lite, is faster on V itself than with a V_t pass
+// before it. The pass costs a launch and 4 bytes of traffic per element of V, the
+// transposing reads ~1.5% of a CTA's main loop, so the line depends on the q rows
+// that share a V. Measured (V_t pass + kernel -> direct, us): (1,2,256) 14.4 ->
+// 12.0, (1,24,1531) 47.3 -> 39.5, (2,24,8192) x 77 55.3 -> 49.8, (2,24,4097) x 512
+// 71.2 -> 66.8, (2,24,8192) x 512 132.3 -> 128.8, (2,24,4096) 349 -> 337,
+// (2,24,8192) 1340 -> 1338; (1,16,10519) 777 -> 780, (1,32,16384) 3628 -> 3636,
+// (2,24,16384) x 2048 748 -> 756, (2,8,32768) x 4096 929 -> 941. Between 8192 and
+// 10519 rows the two are within 0.4%; the line is the last size measured without
+// a loss.
 constexpr int kDirectMaxSq = 8192;
 bool prefers_direct(int seq_len) { return seq_len <= kDirectMaxSq; }
 
