@@ -1,5 +1,5 @@
 // Shared pieces of the gfx950 absorbed-MLA decode kernels (mla_coop.hip: up
-// to 16 query rows per CTA; mla_rows64.hip: 64): the fused fp8 row format,
+// to 16 query rows per CTA; mla_rows64.hip: 64 or 32): the fused fp8 row format,
 // launch parameters, exact fp8 -> bf16 widening, and the device-side split
 // plans the kernels deal their units from.
 #pragma once

@@ -11,8 +11,8 @@
 // position t attends tokens [0, S - (q_len - 1 - t)) (end-aligned causal window,
 // reference mla_decode_a16w8.hip:213-217). Two decode kernels share the row
 // format, the work split, the split records and the numerics (mla_common.hpp):
-// mla_coop.hip for up to 16 query rows, mla_rows64.hip for more (64 rows per
-// CTA). This file holds what surrounds them: the merge of split requests, the
+// mla_coop.hip for up to 16 query rows, mla_rows64.hip for more (64 or 32 rows
+// per CTA). This file holds what surrounds them: the merge of split requests, the
 // planners and the C ABI.
 
 #include <hip/hip_runtime.h>

@@ -3,7 +3,8 @@
 // (reference csrc/mla_decode_a16w8.hip:183-754, csrc/mla_decode_a16w8_multiq.hip
 // :282-856), cut for two waves per SIMD:
 //
-//  * One CTA = 64 query rows (two row tiles of 32) of one request part, 8
+//  * One CTA = 64 query rows (two row tiles of 32; one in calls of 17..32 rows
+//    and in small ones of 33..64, see cta_rows_for) of one request part, 8
 //    waves. The part's fp8 rows are gathered in 64-token tiles into a shared
 //    3-slot LDS ring, wave w gathering tokens 8w .. 8w+7 of every tile.
 //  * S^T = K Q^T on v_mfma_f32_32x32x16_bf16: wave (rt, tt, kh) scores row tile
